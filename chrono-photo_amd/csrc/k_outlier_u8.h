@@ -45,30 +45,16 @@ constexpr uint32_t psel(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3) {
 // needed lie in a's dword (one pixel of 1 or 2 channels).
 template <int NQ, int NW>
 __device__ __forceinline__ void load_realigned(const uint8_t* a, uint32_t (&w)[NW]) {
+    static_assert(NQ <= 4, "at most 16 bytes per load");
     const uintptr_t ad = (uintptr_t)a;
     const uint32_t sft = (uint32_t)ad & 3u;
-    const uintptr_t al = ad & ~(uintptr_t)3;
+    // the address space by name: a pointer made from a number is a flat one, and flat loads
+    // count against the LDS counter too, so the first use would wait for the last load
+    typedef unsigned int vec __attribute__((ext_vector_type(NQ), aligned(4)));
+    const vec v = *(const __attribute__((address_space(1))) vec*)(ad & ~(uintptr_t)3);
     uint32_t q[NQ];
-    if constexpr (NQ == 1) {
-        q[0] = *reinterpret_cast<const uint32_t*>(al);
-    } else if constexpr (NQ == 2) {
-        const uint2 v = *reinterpret_cast<const uint2*>(al);
-        q[0] = v.x;
-        q[1] = v.y;
-    } else if constexpr (NQ == 3) {
-        typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
-        const u32x3 v = *reinterpret_cast<const u32x3*>(al);
-        q[0] = v.x;
-        q[1] = v.y;
-        q[2] = v.z;
-    } else {
-        static_assert(NQ == 4, "at most 16 bytes per load");
-        const uint4 v = *reinterpret_cast<const uint4*>(al);
-        q[0] = v.x;
-        q[1] = v.y;
-        q[2] = v.z;
-        q[3] = v.w;
-    }
+#pragma unroll
+    for (int h = 0; h < NQ; ++h) q[h] = v[h];
     if constexpr (NQ == NW + 1) {
 #pragma unroll
         for (int h = 0; h < NW; ++h) w[h] = __builtin_amdgcn_alignbyte(q[h + 1], q[h], sft);
@@ -138,19 +124,20 @@ __device__ __forceinline__ void load_block_u8(const uint8_t* __restrict__ base, 
     }
 }
 
-// min{x > v} over the group's packed bytes (exists by the caller's count); the bytes are
-// widened to 16-bit halves, where values at or below v wrap to the top.
+// min{x > v} over the group's packed bytes (exists by the caller's count): each byte as the high
+// byte of a 16-bit half (what lies below it there cannot change the order of high bytes) less
+// v + 1, so that bytes at or below v wrap to the top.
 template <int G, int ND>
 __device__ __forceinline__ uint32_t min_greater_u8(const uint32_t (&y)[ND], uint32_t v) {
-    const us2 V = {(unsigned short)(v + 1), (unsigned short)(v + 1)};
+    const unsigned short w = (unsigned short)((v + 1) << 8);
+    const us2 V = {w, w};
     us2 m = {0xFFFF, 0xFFFF};
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
-        const uint32_t lo = y[i] & 0x00FF00FFu, hi = (y[i] >> 8) & 0x00FF00FFu;
-        m = __builtin_elementwise_min(m, as_us2(lo) - V);
-        m = __builtin_elementwise_min(m, as_us2(hi) - V);
+        m = __builtin_elementwise_min(m, as_us2(y[i]) - V);
+        m = __builtin_elementwise_min(m, as_us2(y[i] << 8) - V);
     }
-    const uint32_t mm = min((uint32_t)m.x, (uint32_t)m.y);
+    const uint32_t mm = min((uint32_t)m.x, (uint32_t)m.y) >> 8;
     return grp_min_u32<G>(mm) + v + 1;
 }
 
@@ -338,7 +325,7 @@ template <int C, int G, int F, int X, int FS, bool ABS, bool SORT = false>
 __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, uint32_t y,
                                                 TileShared<C, G, F, X>& sh, const uint64_t* soff, uint32_t lane,
                                                 float* odist = nullptr) {
-    static_assert(F % 8 == 0 && F <= 96 && G <= 32 && FS % 4 == 0 && (X == 1 || X == 4), "tile shape");
+    static_assert(F % 8 == 0 && F <= 64 && G <= 32 && FS % 4 == 0 && (X == 1 || X == 4), "tile shape");
     static_assert(!SORT || (G == 1 && X == 1 && FS == 0), "sorting-network ranks: one lane per pixel");
     using TS = TileShared<C, G, F, X>;
     constexpr int P = TS::P;
@@ -404,6 +391,9 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
             }
         }
         const float tsq = k.th.min * k.th.min;
+        float wide_sq = 0.0f;
+#pragma unroll
+        for (int c = 0; c < C; ++c) wide_sq += 4.5f * k.w[c] * k.w[c];
         const bool want_max = k.outlier == 2 || k.stats != nullptr;
         const bool want_sums = k.background == 2 || k.outlier == 3;
         const bool full_tile = N == (uint32_t)(G * F);
@@ -420,6 +410,31 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
 #pragma unroll
             for (int c = 0; c < 4; ++c) sum_all[e][c] = sum_out[e][c] = 0;
         }
+        const uint32_t real = N > t0 ? min(N - t0, (uint32_t)F) : 0u;  // real frames of this lane's block
+        uint32_t vmask[MW];                                            // their bits in the mask words
+#pragma unroll
+        for (int w = 0; w < MW; ++w) {
+            const int32_t nw = (int32_t)real - 32 * w;
+            vmask[w] = nw >= 32 ? 0xFFFFFFFFu : (nw <= 0 ? 0u : (1u << nw) - 1u);
+        }
+        // With non-negative weights the pads of a tile that the stack does not fill become the
+        // median rounded down: no sample lies nearer to the median than that, so a pad's
+        // distance is at most every real frame's, and as ties go to the lower frame a pad is
+        // never the largest of a lane with a real frame.  The passes below then need no test of
+        // the frame count (it doubled the work per frame of every stack whose count is not
+        // exactly G * F: the 1200-frame 1080p RGB8 stack took 4.78 ms with it).
+        uint32_t pad_v[XC];
+#pragma unroll
+        for (int q = 0; q < XC; ++q) pad_v[q] = pos ? (m0[q] + m1[q]) >> 1 : 255u;
+        if (!full_tile) {
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                const int32_t rem = (int32_t)real - 4 * i;  // real frames in this dword
+                const uint32_t mk = rem >= 4 ? 0u : (rem <= 0 ? 0xFFFFFFFFu : (0xFFFFFFFFu << (8 * rem)));
+#pragma unroll
+                for (int q = 0; q < XC; ++q) yv[q][i] = (yv[q][i] & ~mk) | (mk & splat4(pad_v[q]));
+            }
+        }
 
         // Frames run from last to first so that the mask shifts in bit j for frame j; the
         // largest distance keeps the lowest frame among ties (>=).  lmax starts at the
@@ -428,20 +443,102 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
         constexpr bool ODIST = keeps_odist<G, F, X, FS, SORT>();
         const bool store_d = ODIST && k.outlier == 3;
         uint32_t nst = 0;
-        auto classify = [&](auto e_t, auto unit_t, auto pos_t, auto max_t, auto sums_t, auto check_t) {
+        // no branch: frames that are not stored go to the spare slot kOdistSlots
+        auto put_dist = [&](bool put, float d) {
+            odist[(put ? min(nst, (uint32_t)kOdistSlots) : (uint32_t)kOdistSlots) * (uint32_t)P + lane] = d;
+            nst += put ? 1u : 0u;
+        };
+        // Absolute thresholds with unit weights, in whole numbers: with M = m0 + m1 (twice the
+        // median) the reference's f32 distance is exactly sum x*x - sum x*M + sum M*M / 4 (every
+        // term and partial sum is a multiple of 1/4 below 2^18), so per frame two dot products
+        // of its channels' bytes with m0 and m1 and one with itself replace the 14 f32
+        // operations; `dev` below is the distance less the threshold and its sign is the outlier
+        // bit.  Bound by VALU issue: 1200 x 1080p RGB8, abs/0.05/0.2, extreme ran 8951 VALU
+        // instructions per wave and 4.76-4.79 ms with the checked f32 pass, 5424 and 3.82 ms with
+        // this one (loads alone 2.87 ms).
+        auto classify_dot = [&](auto e_t, auto max_t, auto od_t) {
             constexpr int E = decltype(e_t)::value;
-            constexpr bool UNIT = decltype(unit_t)::value, POS = decltype(pos_t)::value;
+            constexpr bool MAXT = decltype(max_t)::value, OD = decltype(od_t)::value;
+            uint32_t v0 = 0, v1 = 0;
+            int32_t s4 = 0;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const int q = E * C + c;
+                v0 |= m0[q] << (8 * c);
+                v1 |= m1[q] << (8 * c);
+                s4 += (int32_t)((m0[q] + m1[q]) * (m0[q] + m1[q]));
+            }
+            // an outlier is 4 d >= 4 tsq, i.e. dot products' sum >= et
+            const int32_t t4 = (int32_t)ceilf(fminf(4.0f * tsq, 8388608.0f));
+            const int32_t et = (t4 - s4 + 3) >> 2;
+            int32_t best = (int32_t)0x80000000;
+#pragma unroll
+            for (int i = ND - 1; i >= 0; --i) {
+                uint32_t px[4];  // the channels of frames 4i .. 4i + 3, one dword each
+                if constexpr (C >= 3) {
+                    const uint32_t lo = __builtin_amdgcn_perm(yv[E * C + 1][i], yv[E * C][i], psel(0, 4, 1, 5));
+                    const uint32_t hi = __builtin_amdgcn_perm(yv[E * C + 1][i], yv[E * C][i], psel(2, 6, 3, 7));
+                    if constexpr (C == 3) {
+                        const uint32_t b = yv[E * C + 2][i];
+                        px[0] = __builtin_amdgcn_perm(b, lo, psel(0, 1, 4, 12));
+                        px[1] = __builtin_amdgcn_perm(b, lo, psel(2, 3, 5, 12));
+                        px[2] = __builtin_amdgcn_perm(b, hi, psel(0, 1, 6, 12));
+                        px[3] = __builtin_amdgcn_perm(b, hi, psel(2, 3, 7, 12));
+                    } else {
+                        const uint32_t lo2 = __builtin_amdgcn_perm(yv[E * C + C - 1][i], yv[E * C + 2][i], psel(0, 4, 1, 5));
+                        const uint32_t hi2 = __builtin_amdgcn_perm(yv[E * C + C - 1][i], yv[E * C + 2][i], psel(2, 6, 3, 7));
+                        px[0] = __builtin_amdgcn_perm(lo2, lo, psel(0, 1, 4, 5));
+                        px[1] = __builtin_amdgcn_perm(lo2, lo, psel(2, 3, 6, 7));
+                        px[2] = __builtin_amdgcn_perm(hi2, hi, psel(0, 1, 4, 5));
+                        px[3] = __builtin_amdgcn_perm(hi2, hi, psel(2, 3, 6, 7));
+                    }
+                } else {
+                    StaticFor<0, 4>::run([&](auto f_t) {
+                        constexpr int f = decltype(f_t)::value;
+                        if constexpr (C == 2)
+                            px[f] = __builtin_amdgcn_perm(yv[E * C + C - 1][i], yv[E * C][i], psel(f, 4 + f, 12, 12));
+                        else
+                            px[f] = (yv[E * C][i] >> (8 * f)) & 0xFFu;
+                    });
+                }
+#pragma unroll
+                for (int f = 3; f >= 0; --f) {
+                    const int j = 4 * i + f;
+                    const uint32_t xx = __builtin_amdgcn_udot4(px[f], px[f], (uint32_t)-et, false);
+                    const uint32_t xm =
+                        __builtin_amdgcn_udot4(px[f], v1, __builtin_amdgcn_udot4(px[f], v0, 0u, false), false);
+                    const uint32_t dev = xx - xm;  // as a signed number: >= 0 for an outlier
+                    m[E][j >> 5] = __builtin_amdgcn_alignbit(m[E][j >> 5], dev, 31);
+                    if constexpr (MAXT) best = max(best, (int32_t)((dev << 6) | (uint32_t)(63 - j)));
+                    if constexpr (OD) {
+                        const int32_t d4 = 4 * ((int32_t)dev + et) + s4;
+                        put_dist((int32_t)dev >= 0 && (uint32_t)j < real, 0.25f * (float)d4);
+                    }
+                }
+            }
+#pragma unroll
+            for (int w = 0; w < MW; ++w) m[E][w] = ~m[E][w];  // the sign bits mark the others
+            if constexpr (MAXT) {
+                if (best >= 0) {
+                    lmax[E] = 0.25f * (float)(4 * ((best >> 6) + et) + s4);
+                    lmaxi[E] = t0 + 63u - ((uint32_t)best & 63u);
+                }
+            }
+        };
+        // The reference's f32 operations per frame.  CHECK: pads are 255 (negative weights).
+        auto classify = [&](auto e_t, auto pos_t, auto max_t, auto sums_t, auto check_t) {
+            constexpr int E = decltype(e_t)::value;
+            constexpr bool POS = decltype(pos_t)::value;
             constexpr bool MAXT = decltype(max_t)::value, SUMS = decltype(sums_t)::value;
             constexpr bool CHECK = decltype(check_t)::value;
 #pragma unroll
             for (int j = F - 1; j >= 0; --j) {
-                uint32_t xs[4];
                 float d = 0.0f;
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
-                    xs[c] = (yv[E * C + c][j >> 2] >> (8 * (j & 3))) & 0xFFu;
-                    const float diff = med[E][c] - (float)xs[c];
-                    const float a = UNIT ? diff : wi[E][c] * diff;
+                    const uint32_t xs = (yv[E * C + c][j >> 2] >> (8 * (j & 3))) & 0xFFu;
+                    const float diff = med[E][c] - (float)xs;
+                    const float a = wi[E][c] * diff;
                     float term = a * a;
                     if constexpr (!POS) term = sg[c] * term;
                     d = c == 0 ? term : d + term;  // 0 + term0 == term0 up to the sign of zero
@@ -449,35 +546,14 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
                 const bool o = d >= tsq;  // pads are masked out after the loop
                 m[E][j >> 5] = (m[E][j >> 5] << 1) | (o ? 1u : 0u);
                 bool in = true;
-                if constexpr (CHECK) in = t0 + (uint32_t)j < N;
+                if constexpr (CHECK) in = (uint32_t)j < real;
                 if constexpr (MAXT) {
                     if (in && d >= lmax[E]) {
                         lmax[E] = d;
                         lmaxi[E] = t0 + (uint32_t)j;
                     }
                 }
-                if constexpr (SUMS && CHECK) {
-#pragma unroll
-                    for (int c = 0; c < C; ++c) sum_out[E][c] += (o && in) ? xs[c] : 0u;
-                }
-                if constexpr (ODIST && SUMS) {
-                    // no branch: frames that are not stored go to the spare slot kOdistSlots
-                    const bool put = store_d && o && in;
-                    odist[(put ? min(nst, (uint32_t)kOdistSlots) : (uint32_t)kOdistSlots) * (uint32_t)P + lane] = d;
-                    nst += put ? 1u : 0u;
-                }
-            }
-            if constexpr (SUMS && !CHECK) {
-                // every frame is real: the outliers' sums from the mask, four frames per
-                // v_dot4_u32_u8 (the mask's four bits spread to one 0/1 byte per frame)
-#pragma unroll
-                for (int i = 0; i < ND; ++i) {
-                    const uint32_t nib = (m[E][i >> 3] >> (4 * (i & 7))) & 0xFu;
-                    const uint32_t sel = (nib * 0x00204081u) & 0x01010101u;
-#pragma unroll
-                    for (int c = 0; c < C; ++c)
-                        sum_out[E][c] = __builtin_amdgcn_udot4(yv[E * C + c][i], sel, sum_out[E][c], false);
-                }
+                if constexpr (ODIST && SUMS) put_dist(store_d && o && (uint32_t)j < real, d);
             }
         };
         using T_ = std::true_type;
@@ -487,10 +563,13 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
             // Bound check (lanes with few frames): with non-negative weights every frame's f32
             // distance is at most the same f32 expression on the per-channel maximum deviation
             // from the median (correct rounding is monotone), so below the threshold no frame
-            // of this lane is an outlier and the per-frame pass is skipped.
+            // of this lane is an outlier and the per-frame pass is skipped.  The whole-number
+            // pass costs less than the check.
+            // Relative thresholds below about two IQRs per channel leave it out: some lane of a
+            // wave exceeds the bound nearly always (noise reaches 2.8 IQRs among its samples).
             bool may_outlier = true;
             if constexpr (F <= 32) {
-                if (pos && full_tile) {
+                if (pos && !unit && (ABS || tsq >= wide_sq)) {
                     float bound = 0.0f;
 #pragma unroll
                     for (int c = 0; c < C; ++c) {
@@ -505,32 +584,52 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
                         const float lo = (float)min((uint32_t)mn.x, (uint32_t)mn.y);
                         const float hi = (float)max((uint32_t)mx.x, (uint32_t)mx.y);
                         const float dev = fmaxf(med[E][c] - lo, hi - med[E][c]);
-                        const float a = unit ? dev : wi[E][c] * dev;
+                        const float a = wi[E][c] * dev;
                         bound = c == 0 ? a * a : bound + a * a;
                     }
                     may_outlier = bound >= tsq;
                 }
             }
             if (may_outlier) {
-                if (!full_tile) classify(e_t, F_{}, F_{}, T_{}, T_{}, T_{});
-                else if (want_max) {
-                    if (want_sums) classify(e_t, F_{}, F_{}, T_{}, T_{}, F_{});
-                    else if (unit) classify(e_t, T_{}, T_{}, T_{}, F_{}, F_{});
-                    else if (pos) classify(e_t, F_{}, T_{}, T_{}, F_{}, F_{});
-                    else classify(e_t, F_{}, F_{}, T_{}, F_{}, F_{});
-                } else {
-                    if (want_sums) {
-                        if (pos) classify(e_t, F_{}, T_{}, F_{}, T_{}, F_{});
-                        else classify(e_t, F_{}, F_{}, F_{}, T_{}, F_{});
-                    } else if (unit) classify(e_t, T_{}, T_{}, F_{}, F_{}, F_{});
-                    else if (pos) classify(e_t, F_{}, T_{}, F_{}, F_{}, F_{});
-                    else classify(e_t, F_{}, F_{}, F_{}, F_{}, F_{});
+                if constexpr (ABS) {
+                    if (unit && ODIST && store_d) {
+                        if (want_max) classify_dot(e_t, T_{}, std::bool_constant<ODIST>{});
+                        else classify_dot(e_t, F_{}, std::bool_constant<ODIST>{});
+                    } else if (unit) {
+                        if (want_max) classify_dot(e_t, T_{}, F_{});
+                        else classify_dot(e_t, F_{}, F_{});
+                    }
+                }
+                if (!unit) {
+                    if (!pos) classify(e_t, F_{}, T_{}, T_{}, T_{});
+                    else if (want_max) {
+                        if (ODIST && want_sums) classify(e_t, T_{}, T_{}, T_{}, F_{});
+                        else classify(e_t, T_{}, T_{}, F_{}, F_{});
+                    } else {
+                        if (ODIST && want_sums) classify(e_t, T_{}, F_{}, T_{}, F_{});
+                        else classify(e_t, T_{}, F_{}, F_{}, F_{});
+                    }
+                }
+            }
+#pragma unroll
+            for (int w = 0; w < MW; ++w) m[E][w] &= vmask[w];
+            if (real == 0u) lmaxi[E] = NONE;
+            if (want_sums) {
+                // the outliers' sums from the mask, four frames per v_dot4_u32_u8 (the mask's
+                // four bits spread to one 0/1 byte per frame)
+#pragma unroll
+                for (int i = 0; i < ND; ++i) {
+                    const uint32_t nib = (m[E][i >> 3] >> (4 * (i & 7))) & 0xFu;
+                    const uint32_t sel = (nib * 0x00204081u) & 0x01010101u;
+#pragma unroll
+                    for (int c = 0; c < C; ++c)
+                        sum_out[E][c] = __builtin_amdgcn_udot4(yv[E * C + c][i], sel, sum_out[E][c], false);
                 }
             }
         });
         if (want_sums) {
-            // all-frame sums through v_sad_u8 against zero; pads (255) are taken back out
-            const uint32_t npad = t0 + F > N ? min(t0 + F - N, (uint32_t)F) : 0u;
+            // all-frame sums through v_sad_u8 against zero; pads are taken back out
+            const uint32_t npad = (uint32_t)F - real;
 #pragma unroll
             for (int e = 0; e < X; ++e)
 #pragma unroll
@@ -538,23 +637,18 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
                     uint32_t acc = 0;
 #pragma unroll
                     for (int i = 0; i < ND; ++i) acc = __builtin_amdgcn_sad_u8(yv[e * C + c][i], 0u, acc);
-                    sum_all[e][c] = (uint32_t)grp_sum<G>((int32_t)(acc - npad * 255u));
+                    sum_all[e][c] = (uint32_t)grp_sum<G>((int32_t)(acc - npad * pad_v[e * C + c]));
                     sum_out[e][c] = (uint32_t)grp_sum<G>((int32_t)sum_out[e][c]);
                 }
         }
 
         // ---- leave the lane's summaries and the pixels' statistics in LDS
         {
-            const int32_t nv = min((int32_t)N - (int32_t)t0, (int32_t)F);  // valid frames in this block
 #pragma unroll
             for (int e = 0; e < X; ++e) {
                 const uint32_t sl = TS::slot(g, pl * X + e);
 #pragma unroll
-                for (int w = 0; w < MW; ++w) {
-                    const int32_t nw = nv - 32 * w;
-                    const uint32_t vm = nw >= 32 ? 0xFFFFFFFFu : (nw <= 0 ? 0u : (1u << nw) - 1u);
-                    sh.mask[w][sl] = m[e][w] & vm;
-                }
+                for (int w = 0; w < MW; ++w) sh.mask[w][sl] = m[e][w];
                 if (want_max) {
                     sh.lmax[sl] = lmax[e];
                     sh.lmaxi[sl] = lmaxi[e];
