@@ -293,7 +293,7 @@ CP_API int cp_ctx_destroy(cp_ctx* ctx) {
         st->count = st->capacity = 0;
         st->ctx = nullptr;
     }
-    for (DeviceBuffer* b : {&ctx->out_px, &ctx->out_mask, &ctx->out_stats, &ctx->warn})
+    for (DeviceBuffer* b : {&ctx->out_px, &ctx->out_mask, &ctx->out_stats, &ctx->warn, &ctx->shake_ws})
         if (b->ptr) (void)hipFree(b->ptr);
     ctx->arena.release();
     (void)hipStreamDestroy(ctx->stream);

@@ -10,28 +10,36 @@
 // kernels sum exactly and the arg-min reads each total modulo 2^32, which is that wrapped
 // value.  u16 sums are exact 64-bit integers.
 //
-// Work split.  A workgroup owns one (frame, anchor, chunk of candidate rows, chunk of window
-// rows): it stages the frame-f search region those rows reach (window chunk + candidate
-// chunk - 1 rows, u16) and the frame-0 window rows (f32) in LDS.  Each candidate's sum is
-// expanded as
+// The sums on the matrix cores.  A difference does not change when a constant is taken from
+// both samples, so the samples are centred: 8-bit ones become v - 128, 16-bit ones
+// v - 128 * 257 = 256 h + l, with h and l signed bytes (the sample's two bytes less 128).
+// Each candidate's sum is
 //   sum (w - v)^2 = sum w^2 + sum v^2 - 2 sum w*v,
-// all three exact integers.  sum w^2 is one constant for every frame and candidate: the
-// frame-1 workgroups add it to a spare slot of the table, and the arg-min kernel adds it back.
-// sum v^2 comes from an LDS table of squared-sample box sums per region row and candidate
-// column (one sliding pass per row).  sum w*v is the inner loop: a lane owns a strip of K
-// horizontally adjacent candidates (ox0..ox0+K-1, oy) over a sub-chunk of the rows, and the
-// strip's region pixels slide through registers along dx, so one f64 FMA per term and each
-// LDS sample serves K terms.  Products and sums of integers below 2^16 stay exact in f64
-// while every partial sum is below 2^53, which the host guarantees by bounding the rows per
-// lane.  Each lane adds sum v^2 - 2 sum w*v (modulo 2^64) for its K candidates to the
-// per-frame table with 64-bit atomics: integer addition commutes, so the result does not
-// depend on order, and the table holds the exact sums once the constant is added.
+// and for one window row dy the last term is a product of matrices: with the samples q of a
+// region row as the contraction index, A[ox][q] = w[dy][q - ox * C] (zero outside the window
+// row; the same row at another byte offset for every ox) times B[q][oy] = v[oy + dy][q].
+// Signed-byte MFMA (16x16x64) accumulates it over q and dy in exact 32-bit sums: one product
+// per slab of 64 samples for 8-bit frames, and h*h, h*l + l*h and l*l for 16-bit ones.
+//
+// Work split.  A workgroup owns one (frame, anchor, block of up to 32 x 32 candidates, chunk
+// of window rows) and stages the chunk's window rows and the region rows they reach in LDS as
+// byte planes.  Its four waves take every fourth window row; each wave keeps all 2 x 2 tiles
+// of its candidate block, so that a slab costs 8 LDS reads for 16 MFMAs (waves that each took
+// one tile would read twice as much).  The window rows carry zeros on both sides; a lane reads
+// its 16 bytes at any byte offset from the dword at or below them and realigns them.
+// sum v^2 comes from per-row box sums by signed dot products, sum w^2 is one constant per
+// analysis (the frame-1 workgroups add it to a spare slot of the table; the arg-min kernel adds
+// it back).  The waves' sums meet in LDS (64-bit integer adds, any order) and one atomic per
+// candidate adds the workgroup's part to the frame's table.
+//
+// 256 x 4K RGB16, 5 anchors, r = 32, s = 12, per call: 0.78 ms with f64 products on the vector
+// units (bound by their issue), 0.245 ms with the matrix cores.  Staging, box sums and products
+// now take about a quarter each, one after another in a workgroup; three workgroups per CU
+// overlap them (16 window rows per workgroup: 12 or 13 measured alike, 22 leave two).
 #pragma once
 #include "device_common.h"
 
 namespace cp {
-
-constexpr int kShakeStrip = 5;  // candidate offsets per lane (K)
 
 struct ShakeK {
     const uint8_t* stack;
@@ -41,198 +49,337 @@ struct ShakeK {
     const int32_t* anchors;   // device, 2 per anchor
     uint32_t n_anchors;
     int32_t r, s;
-    int32_t chunk_rows;       // window rows per workgroup (blockIdx.z chunks them)
-    int32_t cand_rows;        // candidate rows oy per workgroup
-    int32_t cand_chunks;      // ceil((2s+1) / cand_rows); blockIdx.y = anchor * cand_chunks + chunk
-    int32_t nsub;             // row sub-chunks per workgroup (one per group of strip lanes)
-    int32_t spr;              // strips per offset row: ceil((2s+1) / K)
-    int32_t strips_pad;       // spr * cand_rows rounded up to whole waves
-    int32_t pitch_px;         // LDS region row pitch in pixels: spr * K + 2r
+    int32_t chunk_rows;       // window rows per workgroup
+    int32_t n_chunks;         // ceil((2r+1) / chunk_rows)
+    int32_t cand_rows;        // candidate rows oy per workgroup (at most 32)
+    int32_t cand_chunks;      // ceil((2s+1) / cand_rows)
+    int32_t cand_cols;        // candidate columns ox per workgroup (at most 32)
+    int32_t col_chunks;       // ceil((2s+1) / cand_cols)
+    uint32_t group0;          // first (chunk, candidate block, anchor) combination of this launch
     unsigned long long* sums; // [n][(2s+1)^2], then the sum of squared window samples
     int32_t* offsets;         // [n][2]
 };
 
-// LDS layout of one workgroup for `rows` window rows and `crow` candidate rows: region
-// samples (u16, rows + crow - 1 region rows of pitch_px pixels), window samples (f32,
-// rows x (2r+1) pixels), squared-sample box sums (f64, one per region row and candidate
-// column).
+// LDS layout of one workgroup for `rows` window rows and a block of orows x ocols candidates:
+// region byte planes (rows + orows - 1 rows of rpitch bytes each), window byte planes (rows
+// rows of wpitch bytes; the window row starts at byte wlead), box sums (i64, one per region row
+// and candidate column) and the block's totals (i64).
 struct ShakeLds {
-    uint32_t win_off, rq_off, bytes;
+    uint32_t rlen;    // samples of a region row that the block reaches
+    uint32_t slabs;   // slabs of 64 samples
+    uint32_t rpitch, wpitch, wlead;
+    uint32_t srows;
+    uint64_t win_off, rq_off, tot_off, bytes;
 };
-__host__ __device__ inline ShakeLds shake_lds(int32_t rows, int32_t crow, int32_t r, int32_t s, int32_t pitch_px,
-                                             int32_t channels) {
-    const uint64_t srows = (uint64_t)rows + crow - 1;
-    const uint64_t region = srows * pitch_px * channels * 2;
-    const uint64_t win_off = (region + 7) / 8 * 8;
-    const uint64_t rq_off = (win_off + (uint64_t)rows * (2 * r + 1) * channels * 4 + 7) / 8 * 8;
-    const uint64_t bytes = rq_off + srows * (2 * s + 1) * 8;
-    const uint64_t cap = 0xFFFFFFFFull;
-    return ShakeLds{(uint32_t)(win_off < cap ? win_off : cap), (uint32_t)(rq_off < cap ? rq_off : cap),
-                    (uint32_t)(bytes < cap ? bytes : cap)};
+__host__ __device__ inline ShakeLds shake_lds(int32_t rows, int32_t orows, int32_t ocols, int32_t r, int32_t channels,
+                                             int32_t planes) {
+    ShakeLds l;
+    const uint32_t otile = ocols > 16 ? 32u : 16u;  // columns covered by the tiles
+    l.srows = (uint32_t)(rows + orows - 1);
+    l.rlen = (uint32_t)((2 * r + 1 + ocols - 1) * channels);
+    l.slabs = (l.rlen + 63u) / 64u;
+    l.rpitch = l.slabs * 64u + 16u;  // rows 16 bytes apart modulo 64: their reads spread over the banks
+    l.wlead = (otile * (uint32_t)channels + 15u) / 16u * 16u;
+    l.wpitch = l.wlead + l.slabs * 64u + 16u;
+    l.win_off = (uint64_t)l.srows * l.rpitch * planes;
+    l.rq_off = l.win_off + (uint64_t)rows * l.wpitch * planes;
+    l.tot_off = l.rq_off + (uint64_t)l.srows * ocols * 8u;
+    l.bytes = l.tot_off + (uint64_t)orows * ocols * 8u;
+    return l;
 }
 
-// One dx step of a strip: load region pixel dx+K-1 into its register slot, then add the
-// K products w(dx) * v(dx + j) for every channel.  U = dx mod K names the slots statically.
-template <int C, int K, int U>
-__device__ __forceinline__ void shake_step(const uint16_t* rr, const float* wr, int32_t dx, double (&v)[K][C],
-                                           double (&acc)[K]) {
-#pragma unroll
-    for (int c = 0; c < C; ++c) v[(U + K - 1) % K][c] = (double)(uint32_t)rr[(dx + K - 1) * C + c];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const double w = (double)wr[dx * C + c];
-#pragma unroll
-        for (int j = 0; j < K; ++j) acc[j] = __fma_rn(w, v[(U + j) % K][c], acc[j]);
-    }
-}
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
-template <int C, int K, int U>
-__device__ __forceinline__ void shake_steps(const uint16_t* rr, const float* wr, int32_t dx, double (&v)[K][C],
-                                            double (&acc)[K]) {
-    if constexpr (U < K) {
-        shake_step<C, K, U>(rr, wr, dx + U, v, acc);
-        shake_steps<C, K, U + 1>(rr, wr, dx, v, acc);
-    }
-}
-
-// Remainder of a row (fewer than K steps, count uniform across the wave).
-template <int C, int K, int U>
-__device__ __forceinline__ void shake_tail(const uint16_t* rr, const float* wr, int32_t dx, int32_t left,
-                                           double (&v)[K][C], double (&acc)[K]) {
-    if constexpr (U < K - 1) {
-        if (U < left) {
-            shake_step<C, K, U>(rr, wr, dx + U, v, acc);
-            shake_tail<C, K, U + 1>(rr, wr, dx, left, v, acc);
+// Eight samples from element e of a row that holds `len` (samples past it read as the centre),
+// centred, as bytes: hi and lo planes for 16-bit samples, lo alone for 8-bit ones.
+template <int B>
+__device__ __forceinline__ void load_centred8(const uint8_t* row, uint32_t e, uint32_t len, uint2& hi, uint2& lo) {
+    typedef uint32_t words __attribute__((ext_vector_type(2 * B), aligned(B)));
+    typedef const __attribute__((address_space(1))) words gwords;
+    uint32_t w[2 * B];
+    const uint8_t* at = row + e * B;
+    if (e + 8u <= len) {
+        const words v = *(gwords*)(uintptr_t)at;
+#pragma unroll
+        for (int i = 0; i < 2 * B; ++i) w[i] = v[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2 * B; ++i) w[i] = 0x80808080u;
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i) {
+            if (e + i >= len) break;
+            const uint32_t bit = 8u * B * i, v = load_sample<B>(at, i);
+            w[bit / 32u] = (w[bit / 32u] & ~((B == 1 ? 0xFFu : 0xFFFFu) << (bit % 32u))) | (v << (bit % 32u));
         }
     }
+    if constexpr (B == 1) {
+        lo = uint2{w[0] ^ 0x80808080u, w[1] ^ 0x80808080u};
+        hi = uint2{0u, 0u};
+    } else {
+        lo = uint2{__builtin_amdgcn_perm(w[1], w[0], 0x06040200u) ^ 0x80808080u,
+                   __builtin_amdgcn_perm(w[2 * B - 1], w[2 * B - 2], 0x06040200u) ^ 0x80808080u};
+        hi = uint2{__builtin_amdgcn_perm(w[1], w[0], 0x07050301u) ^ 0x80808080u,
+                   __builtin_amdgcn_perm(w[2 * B - 1], w[2 * B - 2], 0x07050301u) ^ 0x80808080u};
+    }
+}
+
+// Stages `rows` rows of `len` samples (row y at base + y * stride bytes) as byte planes: plane p
+// of row y at dst + (p * rows + y) * pitch; samples past len are zero.  groups: eights of bytes
+// per row.  Sixteen lanes share a row, so that no lane divides and a row's loads are contiguous.
+template <int B>
+__device__ __forceinline__ void stage_rows(const uint8_t* base, uint64_t stride, uint32_t rows, uint32_t len,
+                                           uint32_t groups, uint8_t* dst, uint32_t pitch) {
+    constexpr int U = 4;  // groups in flight per lane
+    const uint32_t gx = threadIdx.x & 15u;
+    for (uint32_t y = threadIdx.x >> 4; y < rows; y += 16u) {
+        const uint8_t* row = base + y * stride;
+        uint8_t* out = dst + y * pitch;
+        for (uint32_t q0 = gx; q0 < groups; q0 += 16u * U) {
+            uint2 hi[U], lo[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (q0 + 16u * u < groups) load_centred8<B>(row, (q0 + 16u * u) * 8u, len, hi[u], lo[u]);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (q0 + 16u * u >= groups) break;
+                *reinterpret_cast<uint2*>(out + (q0 + 16u * u) * 8u) = lo[u];
+                if constexpr (B == 2) *reinterpret_cast<uint2*>(out + rows * pitch + (q0 + 16u * u) * 8u) = hi[u];
+            }
+        }
+    }
+}
+
+// Sum of squares of the packed centred samples of one dword (and its high plane's).
+template <int B>
+__device__ __forceinline__ void square_acc(uint32_t hi, uint32_t lo, int32_t& hh, int32_t& hl, int32_t& ll) {
+    ll = __builtin_amdgcn_sdot4((int)lo, (int)lo, ll, false);
+    if constexpr (B == 2) {
+        hl = __builtin_amdgcn_sdot4((int)hi, (int)lo, hl, false);
+        hh = __builtin_amdgcn_sdot4((int)hi, (int)hi, hh, false);
+    }
+}
+
+// 65536 hh + 512 hl + ll: the squares' sum of samples 256 h + l (hl once per sample).
+template <int B>
+__device__ __forceinline__ long long square_total(int32_t hh, int32_t hl, int32_t ll) {
+    if constexpr (B == 1) return ll;
+    else return ((long long)hh << 16) + ((long long)hl << 9) + ll;
+}
+
+// Sum over the eight adjacent lanes of a half-row (xor 1, xor 2, half-row mirror).
+__device__ __forceinline__ int32_t grp8_sum(int32_t v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true);
+    return v;
 }
 
 template <int B, int C>
 __global__ void __launch_bounds__(256) shake_ssd_kernel(ShakeK k) {
-    constexpr int K = kShakeStrip;
-    extern __shared__ double lds_f64[];
+    constexpr int PL = B;  // byte planes: low, then high
+    extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t f = blockIdx.x + 1;
-    const uint32_t a = blockIdx.y / (uint32_t)k.cand_chunks;
-    const int32_t oc = (int32_t)(blockIdx.y - a * (uint32_t)k.cand_chunks);
+    // (chunk of window rows, block of candidate columns, block of candidate rows, anchor)
+    uint32_t q = k.group0 + blockIdx.y;
+    const int32_t zc = (int32_t)(q % (uint32_t)k.n_chunks);
+    q /= (uint32_t)k.n_chunks;
+    const int32_t xc = (int32_t)(q % (uint32_t)k.col_chunks);
+    q /= (uint32_t)k.col_chunks;
+    const int32_t yc = (int32_t)(q % (uint32_t)k.cand_chunks);
+    const uint32_t a = q / (uint32_t)k.cand_chunks;
     const int32_t r = k.r, s = k.s;
     const int32_t size = 2 * r + 1, ssize = 2 * s + 1;
-    const int32_t c0 = (int32_t)blockIdx.z * k.chunk_rows;
-    const int32_t crows = min(size, c0 + k.chunk_rows) - c0;
-    const int32_t oy0 = oc * k.cand_rows;
-    const int32_t orows = min(ssize, oy0 + k.cand_rows) - oy0;
-    const int32_t srows = crows + orows - 1;  // region rows: the candidate rows over the chunk
-    const int32_t pitch = k.pitch_px * C;     // samples per LDS region row
-    const int32_t wl = size * C;              // samples per window row
-    const ShakeLds lay = shake_lds(crows, orows, r, s, k.pitch_px, C);
-    uint8_t* lds = reinterpret_cast<uint8_t*>(lds_f64);
-    uint16_t* region = reinterpret_cast<uint16_t*>(lds);
-    float* win = reinterpret_cast<float*>(lds + lay.win_off);
-    double* rq = reinterpret_cast<double*>(lds + lay.rq_off);
+    const int32_t c0 = zc * k.chunk_rows, crows = min(size, c0 + k.chunk_rows) - c0;
+    const int32_t oy0 = yc * k.cand_rows, orows = min(ssize, oy0 + k.cand_rows) - oy0;
+    const int32_t ox0 = xc * k.cand_cols, ocols = min(ssize, ox0 + k.cand_cols) - ox0;
+    const ShakeLds lay = shake_lds(crows, orows, ocols, r, C, PL);
+    uint8_t* region = lds;
+    uint8_t* win = lds + lay.win_off;
+    long long* rq = reinterpret_cast<long long*>(lds + lay.rq_off);
+    unsigned long long* tot = reinterpret_cast<unsigned long long*>(lds + lay.tot_off);
+    const uint32_t tid = threadIdx.x;
     const int32_t cx = k.anchors[2 * a], cy = k.anchors[2 * a + 1];
-    // Region pixel (x, y) is frame-f pixel (cx - s - r + x, cy - s - r + oy0 + c0 + y); the
-    // pixels past 2r + 2s only pad the last strip of a row and are never summed.
+    const uint32_t srows = lay.srows, wsamples = (uint32_t)(size * C);
+
+    // ---- stage: region rows oy0 + c0 .. of frame f, window rows c0 .. of frame 0 with zeros
+    // around them, the totals cleared
     {
-        // flat loops over (row, sample) with 8 loads in flight per lane
-        constexpr int U = 8;
-        const uint32_t nt = blockDim.x, tid = threadIdx.x;
-        const uint64_t rstride = (uint64_t)k.stack_w * C;
-        const uint32_t rlen = (uint32_t)((2 * r + 2 * s + 1) * C), rtotal = (uint32_t)(srows * pitch);
-        const uint64_t fbase = k.pos_off[f] + ((uint64_t)(cy - s - r + oy0 + c0) * k.stack_w + (cx - s - r)) * C;
-        for (uint32_t i0 = 0; i0 < rtotal; i0 += U * nt) {
-            uint32_t v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t i = i0 + u * nt + tid, y = i / (uint32_t)pitch, e = i - y * (uint32_t)pitch;
-                v[u] = i < rtotal && e < rlen ? load_sample<B>(k.stack, fbase + y * rstride + e) : 0u;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t i = i0 + u * nt + tid;
-                if (i < rtotal) region[i] = (uint16_t)v[u];
-            }
+        const uint64_t stride = (uint64_t)k.stack_w * C * B;
+        const uint8_t* rbase =
+            k.stack + (k.pos_off[f] + ((uint64_t)(cy - s - r + oy0 + c0) * k.stack_w + (cx - s - r + ox0)) * C) * B;
+        stage_rows<B>(rbase, stride, srows, lay.rlen, lay.slabs * 8u, region, lay.rpitch);
+        const uint8_t* wbase = k.stack + (k.pos_off[0] + ((uint64_t)(cy - r + c0) * k.stack_w + (cx - r)) * C) * B;
+        stage_rows<B>(wbase, stride, (uint32_t)crows, wsamples, (lay.wpitch - lay.wlead) / 8u, win + lay.wlead,
+                      lay.wpitch);
+        const uint32_t lead = lay.wlead / 4u, wrows = (uint32_t)crows * PL;
+        for (uint32_t i = tid; i < wrows * lead; i += 256u)
+            *reinterpret_cast<uint32_t*>(win + (i / lead) * lay.wpitch + (i % lead) * 4u) = 0u;
+        for (uint32_t i = tid; i < (uint32_t)(orows * ocols); i += 256u) tot[i] = 0ull;
+    }
+    __syncthreads();
+
+    // ---- sum w^2, once per (anchor, window chunk): the same for every frame and candidate
+    if (f == 1 && xc == 0 && yc == 0) {
+        const uint32_t words = (wsamples + 3u) / 4u;
+        unsigned long long w2 = 0;
+        for (uint32_t i = tid; i < (uint32_t)crows * words; i += 256u) {
+            const uint32_t y = i / words, e = lay.wlead + (i - y * words) * 4u;
+            const uint32_t lo = *reinterpret_cast<const uint32_t*>(win + y * lay.wpitch + e);
+            uint32_t hi = 0;
+            if constexpr (B == 2) hi = *reinterpret_cast<const uint32_t*>(win + ((uint32_t)crows + y) * lay.wpitch + e);
+            int32_t hh = 0, hl = 0, ll = 0;
+            square_acc<B>(hi, lo, hh, hl, ll);
+            w2 += (unsigned long long)square_total<B>(hh, hl, ll);
         }
-        const uint32_t wtotal = (uint32_t)(crows * wl);
-        const uint64_t wbase = k.pos_off[0] + ((uint64_t)(cy - r + c0) * k.stack_w + (cx - r)) * C;
-        double wsq = 0.0;
-        for (uint32_t i0 = 0; i0 < wtotal; i0 += U * nt) {
-            uint32_t v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t i = i0 + u * nt + tid, y = i / (uint32_t)wl, e = i - y * (uint32_t)wl;
-                v[u] = i < wtotal ? load_sample<B>(k.stack, wbase + y * rstride + e) : 0u;
+        if (w2 != 0) atomicAdd(k.sums + (uint64_t)k.n * ssize * ssize, w2);
+    }
+
+    // ---- rq[y][x] = squares' sum over the window width from candidate column x.  Per row, lane i
+    // of eight sums every eighth dword of the first window, the eight meet by DPP, and lane i
+    // then goes on from the sum of what enters and leaves on the way to its own columns.
+    {
+        constexpr uint32_t PITCH8 = 8u;
+        const uint32_t sub = tid & (PITCH8 - 1u);
+        const uint32_t per = ((uint32_t)ocols + PITCH8 - 1u) / PITCH8;  // columns per lane
+        const uint32_t words = wsamples / 4u;
+        for (uint32_t y0 = 0; y0 < srows; y0 += 256u / PITCH8) {
+            const uint32_t yr = y0 + tid / PITCH8, y = min(yr, srows - 1u);
+            const uint8_t* plo = region + y * lay.rpitch;
+            const uint8_t* phi = region + (srows + y) * lay.rpitch;
+            int32_t hh = 0, hl = 0, ll = 0;
+            auto one = [&](uint32_t at, int32_t sign) {
+                const int32_t l = (int8_t)plo[at];
+                ll += sign * l * l;
+                if constexpr (B == 2) {
+                    const int32_t h = (int8_t)phi[at];
+                    hl += sign * h * l;
+                    hh += sign * h * h;
+                }
+            };
+#pragma unroll 4
+            for (uint32_t b = sub; b < words; b += PITCH8) {
+                uint32_t hi = 0;
+                if constexpr (B == 2) hi = *reinterpret_cast<const uint32_t*>(phi + 4u * b);
+                square_acc<B>(hi, *reinterpret_cast<const uint32_t*>(plo + 4u * b), hh, hl, ll);
             }
+            if (sub < wsamples % 4u) one(words * 4u + sub, 1);
+            ll = grp8_sum(ll);
+            if constexpr (B == 2) {
+                hl = grp8_sum(hl);
+                hh = grp8_sum(hh);
+            }
+            // the step from column x to x + 1 takes pixel x out and pixel x + size in: lanes step
+            // over their own columns, then take the steps of the lanes before them
+            const long long first = square_total<B>(hh, hl, ll);
+            hh = hl = ll = 0;
+            const uint32_t xa = min(sub * per, (uint32_t)ocols), xb = min(xa + per, (uint32_t)ocols);
+            for (uint32_t x = xa; x < xb; ++x) {
+                if (yr < srows) rq[y * (uint32_t)ocols + x] = square_total<B>(hh, hl, ll);
+                if (x + 1u < (uint32_t)ocols) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t i = i0 + u * nt + tid;
-                if (i < wtotal) {
-                    const float w = (float)v[u];
-                    win[i] = w;
-                    wsq = __fma_rn((double)w, (double)w, wsq);
+                    for (uint32_t c = 0; c < (uint32_t)C; ++c) {
+                        one(x * C + c, -1);
+                        one(x * C + wsamples + c, 1);
+                    }
+                }
+            }
+            long long before = first, step = square_total<B>(hh, hl, ll);
+#pragma unroll
+            for (uint32_t j = 0; j < PITCH8 - 1u; ++j) {
+                const long long v = __shfl(step, (int)((tid & 56u) + j));
+                before += j < sub ? v : 0;
+            }
+            if (yr < srows)
+                for (uint32_t x = xa; x < xb; ++x) rq[y * (uint32_t)ocols + x] += before;
+        }
+    }
+
+    // ---- sum w * v by MFMA: tile rows are candidate columns ox, tile columns candidate rows oy
+    const uint32_t lane = tid & 63u, wave = tid >> 6, m16 = lane & 15u, kq = lane >> 4;
+    i32x4 acc[2][2][B == 2 ? 3 : 1];  // [ox tile][oy tile][l*l (, h*l + l*h, h*h)]
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int p = 0; p < (B == 2 ? 3 : 1); ++p) acc[i][j][p] = i32x4{0, 0, 0, 0};
+    const bool ox2 = ocols > 16, oy2 = orows > 16;
+    // byte of the window row that meets region sample 0 in this lane's candidate column
+    uint32_t wal[2], wsh[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t at = lay.wlead + kq * 16u - min(m16 + 16u * i, ox2 ? 31u : 15u) * C;
+        wal[i] = at & ~3u;
+        wsh[i] = at & 3u;
+    }
+    uint32_t brow[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) brow[j] = min(m16 + 16u * j, (uint32_t)orows - 1u) * lay.rpitch + kq * 16u;
+    for (uint32_t dy = wave; dy < (uint32_t)crows; dy += 4u) {
+        const uint8_t* wr = win + dy * lay.wpitch;
+        const uint8_t* rr = region + dy * lay.rpitch;
+        for (uint32_t sl = 0; sl < lay.slabs; ++sl) {
+            i32x4 av[2][PL], bv[2][PL];
+#pragma unroll
+            for (int p = 0; p < PL; ++p)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if (i == 1 && !ox2) break;
+                    const uint32_t* w = reinterpret_cast<const uint32_t*>(wr + (uint32_t)p * (uint32_t)crows * lay.wpitch +
+                                                                          wal[i] + sl * 64u);
+                    uint32_t d[5];
+#pragma unroll
+                    for (int h = 0; h < 5; ++h) d[h] = w[h];
+#pragma unroll
+                    for (int h = 0; h < 4; ++h) av[i][p][h] = (int)__builtin_amdgcn_alignbyte(d[h + 1], d[h], wsh[i]);
+                }
+#pragma unroll
+            for (int p = 0; p < PL; ++p)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if (j == 1 && !oy2) break;
+                    bv[j][p] = *reinterpret_cast<const i32x4*>(rr + (uint32_t)p * srows * lay.rpitch + brow[j] + sl * 64u);
+                }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if (i == 1 && !ox2) break;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if (j == 1 && !oy2) break;
+                    acc[i][j][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][0], bv[j][0], acc[i][j][0], 0, 0, 0);
+                    if constexpr (B == 2) {
+                        acc[i][j][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][0], bv[j][1], acc[i][j][1], 0, 0, 0);
+                        acc[i][j][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][1], bv[j][1], acc[i][j][2], 0, 0, 0);
+                        acc[i][j][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][1], bv[j][0], acc[i][j][1], 0, 0, 0);
+                    }
                 }
             }
         }
-        // sum of squared window samples, once per (anchor, window chunk): frame-independent
-        if (f == 1 && oc == 0 && wsq != 0.0)
-            atomicAdd(k.sums + (uint64_t)k.n * ssize * ssize, (unsigned long long)wsq);
     }
-    __syncthreads();
-    // rq[y][x] = sum over the window width of squared region samples starting at pixel x:
-    // one lane per (region row, strip of K columns), sliding along the row
-    for (int32_t t = threadIdx.x; t < srows * k.spr; t += blockDim.x) {
-        const int32_t y = t / k.spr, x0 = (t - y * k.spr) * K;
-        const uint16_t* row = region + y * pitch;
-        double sum = 0.0;
-        for (int32_t i = x0 * C; i < (x0 + size) * C; ++i) {
-            const double v = (double)(uint32_t)row[i];
-            sum = __fma_rn(v, v, sum);
-        }
-        rq[y * ssize + x0] = sum;
+    __syncthreads();  // the box sums are there
+
+    // ---- sum v^2 - 2 sum w * v of this wave's window rows
 #pragma unroll
-        for (int j = 1; j < K; ++j) {
-            if (x0 + j >= ssize) break;
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int c = 0; c < C; ++c) {
-                const double vin = (double)(uint32_t)row[(x0 + j - 1 + size) * C + c];
-                const double vout = (double)(uint32_t)row[(x0 + j - 1) * C + c];
-                sum = __fma_rn(vin, vin, sum);
-                sum = __fma_rn(-vout, vout, sum);
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t oy = m16 + 16u * j;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t ox = 16u * i + 4u * kq + e;
+                if (oy >= (uint32_t)orows || ox >= (uint32_t)ocols) continue;
+                long long wv = acc[i][j][0][e];
+                if constexpr (B == 2)
+                    wv += ((long long)acc[i][j][B == 2 ? 2 : 0][e] << 16) + ((long long)acc[i][j][B == 2 ? 1 : 0][e] << 8);
+                long long v = -2 * wv;
+                for (uint32_t dy = wave; dy < (uint32_t)crows; dy += 4u) v += rq[(oy + dy) * (uint32_t)ocols + ox];
+                atomicAdd(tot + oy * (uint32_t)ocols + ox, (unsigned long long)v);
             }
-            rq[y * ssize + x0 + j] = sum;
         }
-    }
     __syncthreads();
-    const int32_t nstrips = k.spr * orows;
-    const int32_t ntasks = k.strips_pad * k.nsub;
-    const uint64_t noff = (uint64_t)ssize * ssize;
-    for (int32_t t = threadIdx.x; t < ntasks; t += blockDim.x) {
-        // strips_pad is a multiple of 64, so a wave shares its sub-chunk (and window reads)
-        const int32_t sub = t / k.strips_pad, strip = t - sub * k.strips_pad;
-        if (strip >= nstrips) continue;
-        const int32_t oy = strip / k.spr, ox0 = (strip - oy * k.spr) * K;  // oy within the chunk
-        const int32_t lo = sub * crows / k.nsub, hi = (sub + 1) * crows / k.nsub;
-        double acc[K], sq[K];
-#pragma unroll
-        for (int j = 0; j < K; ++j) acc[j] = sq[j] = 0.0;
-        for (int32_t y = lo; y < hi; ++y) {
-            const uint16_t* rr = region + (oy + y) * pitch + ox0 * C;
-            const float* wr = win + y * wl;
-            double v[K][C];
-#pragma unroll
-            for (int u = 0; u < K - 1; ++u)
-#pragma unroll
-                for (int c = 0; c < C; ++c) v[u][c] = (double)(uint32_t)rr[u * C + c];
-            int32_t dx = 0;
-            for (; dx + K <= size; dx += K) shake_steps<C, K, 0>(rr, wr, dx, v, acc);
-            shake_tail<C, K, 0>(rr, wr, dx, size - dx, v, acc);
-#pragma unroll
-            for (int j = 0; j < K; ++j)
-                if (ox0 + j < ssize) sq[j] += rq[(oy + y) * ssize + ox0 + j];
-        }
-        unsigned long long* out = k.sums + (uint64_t)f * noff + (uint64_t)(oy0 + oy) * ssize + ox0;
-#pragma unroll
-        for (int j = 0; j < K; ++j)
-            if (ox0 + j < ssize)
-                atomicAdd(out + j, (unsigned long long)sq[j] - 2ull * (unsigned long long)acc[j]);
+    for (uint32_t i = tid; i < (uint32_t)(orows * ocols); i += 256u) {
+        const uint32_t oy = i / (uint32_t)ocols, ox = i - oy * (uint32_t)ocols;
+        atomicAdd(k.sums + (uint64_t)f * ssize * ssize + (uint64_t)(oy0 + oy) * ssize + ox0 + ox, tot[i]);
     }
 }
 

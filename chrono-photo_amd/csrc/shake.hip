@@ -13,6 +13,10 @@ namespace {
 // it (shake_scratch_init) and only that address is used on the host.
 constexpr uint64_t kShakeScratchBytes = 8ull << 20;
 constexpr int kMaxDevices = 64;
+// Sum tables and offsets up to this size live in a workspace that the context keeps.
+constexpr uint64_t kShakeKeepBytes = 4ull << 20;
+// Window rows per workgroup (a multiple of its four waves)
+constexpr int32_t kShakeRows = 16;
 static __device__ __align__(256) unsigned long long scratch[kShakeScratchBytes / 8];
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
@@ -104,9 +108,12 @@ static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, ui
     hipStream_t hs = ctx->stream;
     ShakeK k{};
     k.stack = st->dev;
-    k.pos_off = (const uint64_t*)ctx->arena.put(pos.data(), 8 * n, hs);
-    k.anchors = (const int32_t*)ctx->arena.put(anchors_xy, 8 * n_anchors, hs);
-    if (!k.pos_off || !k.anchors) return fail(CP_ERR_HIP, "parameter staging failed");
+    // the frame offsets and the anchors in one copy
+    pos.resize(n + n_anchors);
+    memcpy(pos.data() + n, anchors_xy, 8ull * n_anchors);
+    k.pos_off = (const uint64_t*)ctx->arena.put(pos.data(), 8ull * pos.size(), hs);
+    if (!k.pos_off) return fail(CP_ERR_HIP, "parameter staging failed");
+    k.anchors = (const int32_t*)(k.pos_off + n);
     k.stack_w = st->width;
     k.n = n;
     k.n_anchors = n_anchors;
@@ -114,14 +121,22 @@ static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, ui
     k.s = (int32_t)s;
     DeviceBuffer sums, offs;
     int rc = CP_OK;
+    bool kept = false;
     if (scratch_dev) {
         sums.ptr = scratch_dev;
         offs.ptr = dev_out ? (void*)offsets : (void*)((uint8_t*)scratch_dev + sums_al);
     } else {
         const uint64_t offs_bytes = dev_out ? 0 : 8ull * n;
         if ((rc = ctx->charge(sums_bytes + offs_bytes))) return rc;
-        if (hipMalloc(&sums.ptr, sums_bytes) != hipSuccess ||
-            (!dev_out && hipMalloc(&offs.ptr, offs_bytes) != hipSuccess)) {
+        // The context keeps one small workspace (an allocation and its release cost more than the
+        // search of a short stack); this call holds it until the stream has drained below.
+        kept = sums_al + offs_bytes <= kShakeKeepBytes &&
+               (ctx->shake_ws.ptr || hipMalloc(&ctx->shake_ws.ptr, kShakeKeepBytes) == hipSuccess);
+        if (kept) {
+            sums.ptr = ctx->shake_ws.ptr;
+            if (!dev_out) offs.ptr = (uint8_t*)ctx->shake_ws.ptr + sums_al;
+        } else if (hipMalloc(&sums.ptr, sums_bytes) != hipSuccess ||
+                   (!dev_out && hipMalloc(&offs.ptr, offs_bytes) != hipSuccess)) {
             if (sums.ptr) (void)hipFree(sums.ptr);
             ctx->uncharge(sums_bytes + offs_bytes);
             return fail(CP_ERR_HIP, "hipMalloc for shake sums failed");
@@ -135,61 +150,62 @@ static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, ui
     hipLaunchKernelGGL(zero_u64_kernel, dim3((uint32_t)std::min<uint64_t>(1024, (n_sums + 255) / 256)), dim3(256), 0,
                        hs, k.sums, n_sums);
     hipError_t e = hipGetLastError();
-    // Launch plan: strips of kShakeStrip offsets per lane, whole waves per row sub-chunk,
-    // about 8 window rows per sub-chunk and all candidate rows per workgroup; where that
-    // does not fit LDS, the larger of the two row counts shrinks.
-    constexpr int32_t K = kShakeStrip;
-    const int32_t size = (int32_t)(2 * r + 1), C = (int32_t)st->channels;
-    k.spr = (ssize + K - 1) / K;
-    k.pitch_px = k.spr * K + (int32_t)(2 * r);
-    int32_t block = 256;
-    auto set_lanes = [&](int32_t orows) {
-        k.strips_pad = (k.spr * orows + 63) / 64 * 64;
-        k.nsub = k.strips_pad <= 256 ? 256 / k.strips_pad : 1;
-        block = k.strips_pad <= 256 ? k.strips_pad * k.nsub : 256;
+    // Launch plan: candidate blocks of up to 32 x 32, about kRows window rows per workgroup in
+    // even chunks; where that does not fit LDS, the larger of the row counts shrinks, then the
+    // candidate columns.
+    const int32_t size = (int32_t)(2 * r + 1), C = (int32_t)st->channels, planes = (int32_t)st->bps;
+    auto even = [](int32_t total, int32_t most) {
+        const int32_t parts = (total + most - 1) / most;
+        return (total + parts - 1) / parts;
     };
-    // Exact f64 sums: each lane adds ceil(rows / nsub) * size * C products below maxsq.
-    const double maxsq = st->bps == 2 ? 65535.0 * 65535.0 : 255.0 * 255.0;
-    auto fits = [&](int32_t rows, int32_t orows) {
-        set_lanes(orows);
-        const double terms = (double)((rows + k.nsub - 1) / k.nsub) * size * C;
-        return shake_lds(rows, orows, (int32_t)r, (int32_t)s, k.pitch_px, C).bytes <= 64 * 1024 &&
-               terms * maxsq < 9007199254740992.0;
+    int32_t orows = even(ssize, 32), ocols = even(ssize, 32), rows = even(size, kShakeRows);
+    auto fits = [&]() {
+        // exact 32-bit sums: a wave adds at most ceil(rows / 4) * size * C products of two signed
+        // bytes (twice that many in the mixed plane)
+        return shake_lds(rows, orows, ocols, (int32_t)r, C, planes).bytes <= 64 * 1024 &&
+               (int64_t)((rows + 3) / 4) * size * C < 65536;
     };
-    int32_t orows = ssize;
-    set_lanes(orows);
-    const int32_t want = std::min<int32_t>(size, 8 * k.nsub);
-    const int32_t even_chunks = (size + want - 1) / want;
-    int32_t rows = (size + even_chunks - 1) / even_chunks;
-    while (!fits(rows, orows) && (rows > 1 || orows > 1)) {
-        if (orows > rows) --orows;
-        else --rows;
+    while (!fits() && (rows > 1 || orows > 1 || ocols > 1)) {
+        if (rows > 1 && rows >= orows) --rows;
+        else if (orows > 1) --orows;
+        else --ocols;
     }
-    const bool ok = fits(rows, orows);  // also leaves the lane split of the final orows in k
+    // The documented limit of the radii (chrono_hip.h): one region row as 16-bit samples up to a
+    // whole strip of five candidates, one window row as 32-bit values and one row of 64-bit box
+    // sums in 64 KiB.  Everything within it fits the layout above.
+    const uint64_t limit_row = ((uint64_t)((ssize + 4) / 5 * 5 + 2 * r) * C * 2 + 7) / 8 * 8;
+    const uint64_t limit_bytes = (limit_row + (uint64_t)size * C * 4 + 7) / 8 * 8 + (uint64_t)ssize * 8;
+    const bool ok = fits() && limit_bytes <= 64 * 1024;
     k.chunk_rows = rows;
+    k.n_chunks = (size + rows - 1) / rows;
     k.cand_rows = orows;
     k.cand_chunks = (ssize + orows - 1) / orows;
-    const uint32_t nchunk = (uint32_t)((size + rows - 1) / rows);
-    const size_t lds = shake_lds(rows, orows, (int32_t)r, (int32_t)s, k.pitch_px, C).bytes;
+    k.cand_cols = ocols;
+    k.col_chunks = (ssize + ocols - 1) / ocols;
+    const size_t lds = (size_t)shake_lds(rows, orows, ocols, (int32_t)r, C, planes).bytes;
     if (e == hipSuccess && !ok) {
         e = hipErrorInvalidValue;
         rc = fail(CP_ERR_INVALID_ARG,
                   "anchor search needs %zu bytes of LDS for one window row and one candidate row (64 KiB at most)",
-                  (size_t)shake_lds(1, 1, (int32_t)r, (int32_t)s, k.pitch_px, C).bytes);
-    } else if (e == hipSuccess && (uint64_t)n_anchors * k.cand_chunks > 65535) {
+                  (size_t)limit_bytes);
+    }
+    const uint64_t groups = (uint64_t)n_anchors * k.cand_chunks * k.col_chunks * k.n_chunks;
+    if (e == hipSuccess && (n_anchors > 65535 || groups > 0xFFFFFFFFull)) {
         e = hipErrorInvalidValue;
-        rc = fail(CP_ERR_INVALID_ARG, "%u anchors x %d candidate-row chunks exceed 65535 workgroup rows",
-                  n_anchors, k.cand_chunks);
+        rc = fail(CP_ERR_INVALID_ARG, "%u anchors need too many workgroups (65535 anchors at most)", n_anchors);
     }
     if (e == hipSuccess) {
-        dim3 grid(n - 1, n_anchors * (uint32_t)k.cand_chunks, nchunk), blk(block);
-        auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, blk, lds, hs, k); };
         const bool wide = st->bps == 2;
-        switch (st->channels) {
-        case 1: wide ? launch(shake_ssd_kernel<2, 1>) : launch(shake_ssd_kernel<1, 1>); break;
-        case 2: wide ? launch(shake_ssd_kernel<2, 2>) : launch(shake_ssd_kernel<1, 2>); break;
-        case 3: wide ? launch(shake_ssd_kernel<2, 3>) : launch(shake_ssd_kernel<1, 3>); break;
-        default: wide ? launch(shake_ssd_kernel<2, 4>) : launch(shake_ssd_kernel<1, 4>); break;
+        for (uint64_t g0 = 0; g0 < groups; g0 += 65535) {  // the grid's y extent
+            k.group0 = (uint32_t)g0;
+            dim3 grid(n - 1, (uint32_t)std::min<uint64_t>(65535, groups - g0)), blk(256);
+            auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, blk, lds, hs, k); };
+            switch (st->channels) {
+            case 1: wide ? launch(shake_ssd_kernel<2, 1>) : launch(shake_ssd_kernel<1, 1>); break;
+            case 2: wide ? launch(shake_ssd_kernel<2, 2>) : launch(shake_ssd_kernel<1, 2>); break;
+            case 3: wide ? launch(shake_ssd_kernel<2, 3>) : launch(shake_ssd_kernel<1, 3>); break;
+            default: wide ? launch(shake_ssd_kernel<2, 4>) : launch(shake_ssd_kernel<1, 4>); break;
+            }
         }
         if (wide) hipLaunchKernelGGL(shake_argmin_kernel<2>, dim3(n), dim3(256), 0, hs, k);
         else hipLaunchKernelGGL(shake_argmin_kernel<1>, dim3(n), dim3(256), 0, hs, k);
@@ -199,9 +215,11 @@ static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, ui
         if (e != hipSuccess && rc == CP_OK) rc = fail(CP_ERR_HIP, "shake kernels: %s", hipGetErrorString(e));
     }
     if (!scratch_dev) {
-        (void)hipStreamSynchronize(hs);
-        (void)hipFree(sums.ptr);
-        if (!dev_out) (void)hipFree(offs.ptr);
+        if (e != hipSuccess || dev_out || !kept) (void)hipStreamSynchronize(hs);
+        if (!kept) {
+            (void)hipFree(sums.ptr);
+            if (!dev_out) (void)hipFree(offs.ptr);
+        }
         ctx->uncharge(sums_bytes + (dev_out ? 0 : 8ull * n));
     }
     return rc;
