@@ -73,22 +73,32 @@ int launch_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uint64_t 
     return CP_OK;
 }
 
-template <int B, int PX>
+template <int B, int PX, bool PLAIN>
 static void launch_simple_b(const cp_stack* st, const SimpleK& k, hipStream_t s) {
     const uint32_t lanes = (k.out_w + PX - 1) / PX;
     dim3 block(256), grid((lanes + 255) / 256, k.out_h);
     switch (st->channels) {
-    case 1: hipLaunchKernelGGL((simple_kernel<B, 1, PX>), grid, block, 0, s, k); break;
-    case 2: hipLaunchKernelGGL((simple_kernel<B, 2, PX>), grid, block, 0, s, k); break;
-    case 3: hipLaunchKernelGGL((simple_kernel<B, 3, PX>), grid, block, 0, s, k); break;
-    default: hipLaunchKernelGGL((simple_kernel<B, 4, PX>), grid, block, 0, s, k); break;
+    case 1: hipLaunchKernelGGL((simple_kernel<B, 1, PX, PLAIN>), grid, block, 0, s, k); break;
+    case 2: hipLaunchKernelGGL((simple_kernel<B, 2, PX, PLAIN>), grid, block, 0, s, k); break;
+    case 3: hipLaunchKernelGGL((simple_kernel<B, 3, PX, PLAIN>), grid, block, 0, s, k); break;
+    default: hipLaunchKernelGGL((simple_kernel<B, 4, PX, PLAIN>), grid, block, 0, s, k); break;
     }
 }
 
-int launch_simple(cp_ctx* ctx, const cp_stack* st, const SimpleK& k, hipStream_t s) {
+int launch_simple(cp_ctx* ctx, const cp_stack* st, const SimpleK& k_in, hipStream_t s) {
     (void)ctx;
-    if (st->bps == 1) launch_simple_b<1, 4>(st, k, s);
-    else launch_simple_b<2, 2>(st, k, s);
+    SimpleK k = k_in;
+    // Whole frames are one row: no lane is lost at the row ends, and the waves of a full-HD image
+    // fit the device at once (8100 for 8192 slots; row by row 8640, whose last 448 ran alone).
+    if (k.out_w == k.stack_w && (uint64_t)k.out_w * k.out_h < 0x80000000ull) {
+        k.out_w *= k.out_h;
+        k.out_h = 1;
+    }
+    // whole-number steps (k_simple.h) where every weight is one and nothing fades
+    bool plain = k.fade.is_none != 0;
+    for (uint32_t c = 0; c < st->channels; ++c) plain = plain && k.w[c] == 1.0f;
+    if (st->bps == 1) plain ? launch_simple_b<1, 4, true>(st, k, s) : launch_simple_b<1, 4, false>(st, k, s);
+    else plain ? launch_simple_b<2, 2, true>(st, k, s) : launch_simple_b<2, 2, false>(st, k, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(CP_ERR_HIP, "simple kernel launch: %s", hipGetErrorString(e));
     return CP_OK;
