@@ -34,7 +34,9 @@ FLAGS = [
 
 LIBS = {
     "libchrono_hip.so": ["abi.hip", "kernels.hip", "kernels_fast_b1_c3.hip", "kernels_fast_b1_c4.hip",
-                         "kernels_fast_b2_c3.hip", "kernels_fast_b2_c4.hip", "kernels_u8_c1.hip",
+                         "kernels_fast_b2_c1_abs.hip", "kernels_fast_b2_c1_rel.hip", "kernels_fast_b2_c2_abs.hip",
+                         "kernels_fast_b2_c2_rel.hip", "kernels_fast_b2_c3_abs.hip", "kernels_fast_b2_c3_rel.hip",
+                         "kernels_fast_b2_c4_abs.hip", "kernels_fast_b2_c4_rel.hip", "kernels_u8_c1.hip",
                          "kernels_u8_c2.hip", "kernels_u8_c3.hip", "kernels_u8_c4.hip", "kernels_batch_u8_c1.hip",
                          "kernels_batch_u8_c2.hip", "kernels_batch_u8_c3.hip", "kernels_batch_u8_c4.hip",
                          "kernels_batch_fast_b1_c3.hip", "kernels_batch_fast_b1_c4.hip",
@@ -78,10 +80,12 @@ def build(verbose=False, changed_only=False):
     """Compiles every translation unit (changed_only: only those whose source or local
     headers are newer than their object, for development) and links the libraries."""
     os.makedirs(os.path.join(OUT, "obj"), exist_ok=True)
-    # the kernel translation units take minutes each: start the biggest first (the packed-byte
-    # ones, then the 16-bit-halves ones), so that the small ones fill in at the end
+    # the kernel translation units take minutes each: start the biggest first (16-bit samples,
+    # then the packed bytes, more channels before fewer), so that the small ones fill in at the end
     def cost(src):
-        return (0 if "_u8_" in src else 1 if "_fast_" in src else 2, src)
+        kind = 0 if "_fast_b2_" in src else 1 if "_u8_" in src else 2 if "_fast_" in src else 3
+        channels = int(src.split("_c")[1][0]) if "_c" in src else 0
+        return (kind, -channels, src)
     srcs = sorted({s for v in LIBS.values() for s in v}, key=cost)
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
         objs = dict(zip(srcs, ex.map(lambda s: _compile(s, changed_only), srcs)))

@@ -231,7 +231,7 @@ extern "C" CP_API int cp_batch_create(cp_ctx* ctx, const cp_job* jobs, uint32_t 
                 }
                 BatchJobK bj{};
                 bj.k = k;
-                const uint32_t P = group_tile_pixels(plan.family, plan.shape);
+                const uint32_t P = group_tile_pixels(plan.family, plan.shape, st->channels);
                 bj.tiles_x = (k.out_w + P - 1) / P;
                 bj.tiles = bj.tiles_x * k.out_h;
                 g->jobs.push_back(bj);
@@ -421,12 +421,12 @@ __global__ void autotune_fill_kernel(uint8_t* data, uint32_t bps, uint64_t n_ele
 // Public encoding of a kernel choice: (kernel << 24) | (pixels per lane << 16) | (lanes per
 // pixel << 8) | frames per lane; kernel 0: 16-bit halves, 1: 8-bit packed bytes with the byte
 // search, 2: 8-bit packed bytes with sorting-network ranks.
-static int32_t encode_choice(int choice) {
+static int32_t encode_choice(int choice, uint32_t channels) {
     if (choice >= kU8Base) {
         const U8Shape& u = kU8Shapes[choice - kU8Base];
         return ((u.S ? 2 : 1) << 24) | (u.X << 16) | (u.G << 8) | u.F;
     }
-    return (kShapes[choice].X << 16) | (kShapes[choice].G << 8) | kShapes[choice].F;
+    return (shape_px(choice, channels) << 16) | (kShapes[choice].G << 8) | kShapes[choice].F;
 }
 
 extern "C" CP_API int cp_tile_shapes_set(cp_ctx* ctx, uint32_t bps, uint32_t channels, const int32_t* shapes) {
@@ -441,7 +441,7 @@ extern "C" CP_API int cp_tile_shapes_set(cp_ctx* ctx, uint32_t bps, uint32_t cha
             if (want == 0) continue;
             for (int c = 0; c < kMaxCand; ++c) {
                 const int ch = kBucketCand[bps - 1][channels >= 3][b][c];
-                if (ch >= 0 && want == encode_choice(ch)) pick[kind][b] = (int8_t)ch;
+                if (ch >= 0 && want == encode_choice(ch, channels)) pick[kind][b] = (int8_t)ch;
             }
             if (pick[kind][b] < 0)
                 return fail(CP_ERR_INVALID_ARG, "shape 0x%07x is not a candidate for frame bucket %d", want, b);
@@ -538,7 +538,7 @@ extern "C" CP_API int cp_autotune(cp_ctx* ctx, uint32_t bps, uint32_t channels, 
             }
             if (!ok) break;
             ctx->tuned[bps - 1][channels - 1][kind][b] = (int8_t)best;
-            if (shapes) shapes[kb] = best >= 0 ? encode_choice(best) : 0;
+            if (shapes) shapes[kb] = best >= 0 ? encode_choice(best, channels) : 0;
         }
         (void)hipStreamSynchronize(s);
         if (d_pos) (void)hipFree(d_pos);

@@ -60,9 +60,9 @@ __device__ __forceinline__ uint32_t group_job(const BatchJobK* __restrict__ jobs
 template <int C, int G, int F, int X, int FS, bool ABS, bool SORT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, SORT))))
 outlier_u8_group_kernel(const BatchJobK* __restrict__ jobs, uint32_t njobs) {
-    __shared__ TileShared<C, G, F, X> sh;
+    __shared__ TileShared<C, G, F, X, false> sh;
     __shared__ uint64_t soff[FS > 0 ? G * (FS + 2) : 1];
-    __shared__ float odist[keeps_odist<G, F, X, FS, SORT>() ? (kOdistSlots + 1) * TileShared<C, G, F, X>::P : 1];
+    __shared__ float odist[keeps_odist<G, F, X, FS, SORT>() ? (kOdistSlots + 1) * TileShared<C, G, F, X, false>::P : 1];
     const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
     const BatchJobK& J = jobs[group_job(jobs, njobs, tile)];
     const OutlierK k = global_args(J.k);
@@ -77,19 +77,14 @@ outlier_u8_group_kernel(const BatchJobK* __restrict__ jobs, uint32_t njobs) {
 template <int B, int C, int G, int F, int X, bool ABS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint(F, C, ABS, X))))
 outlier_fast_group_kernel(const BatchJobK* __restrict__ jobs, uint32_t njobs) {
-    __shared__ TileShared<C, G, F, X> sh;
+    __shared__ TileShared<C, G, F, X, (X > 1)> sh;
+    __shared__ SampleTable<G, 0> ssh;
     const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
     const BatchJobK& J = jobs[group_job(jobs, njobs, tile)];
     const OutlierK k = global_args(J.k);
     const uint32_t t = tile - J.tile0, y = t / J.tiles_x;
-    if constexpr (X == 2) {
-        const uint32_t r = (uint32_t)((uintptr_t)k.stack + (uint64_t)y * k.stack_w * C * B) & 3u;
-        load_offsets_pair<B, F>(sh.off, sh.aoff, sh.sft, G * F, k.pos_off, k.n, r);
-    } else {
-        load_offsets<B, F>(sh.off, G * F, k.pos_off, k.n);
-    }
-    __syncthreads();
-    outlier_tile<B, C, G, F, X, ABS>(k, t % J.tiles_x, y, sh, threadIdx.x);
+    load_tables<B>(k, y, sh, ssh);
+    outlier_tile<B, C, G, F, X, 0, ABS>(k, t % J.tiles_x, y, sh, ssh, threadIdx.x);
 }
 
 template <int C, int G, int F, int X, int FS, bool SORT = false>
@@ -191,9 +186,9 @@ inline const void* group_kernel(int family, int shape, uint32_t bps, uint32_t ch
 }
 
 // Pixels per tile of a plan's shape.
-inline uint32_t group_tile_pixels(int family, int shape) {
+inline uint32_t group_tile_pixels(int family, int shape, uint32_t channels) {
     if (family == 2) return (uint32_t)(kU8Shapes[shape].X * 256 / kU8Shapes[shape].G);
-    return (uint32_t)(kShapes[shape].X * 256 / kShapes[shape].G);
+    return (uint32_t)(shape_px(shape, channels) * 256 / kShapes[shape].G);
 }
 
 }  // namespace cp

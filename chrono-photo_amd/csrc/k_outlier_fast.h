@@ -392,10 +392,12 @@ __device__ __forceinline__ uint32_t min_greater(const uint32_t (&r)[NW], uint32_
 }
 
 // Location estimate of a 16-bit channel: median-of-3 "remedian" over the lane's samples
-// (both halves of each dword at once), then a trimmed mean over the group's lanes.  It only
-// places the search window; exactness never depends on it.
+// (both halves of each dword at once), then a trimmed mean over the lanes whose block is at
+// least three quarters real frames (real: this lane's; pads are the largest value and would
+// pull the mean up, and the search window with it).  It only places the search window;
+// exactness never depends on it.
 template <int G, int NW>
-__device__ __forceinline__ uint32_t group_estimate(const uint32_t (&r)[NW]) {
+__device__ __forceinline__ uint32_t group_estimate(const uint32_t (&r)[NW], uint32_t real) {
     constexpr int L0 = NW / 3, L1 = L0 / 3, L2 = L1 / 3;
     static_assert(L0 >= 1, "estimate needs at least three dwords per lane");
     us2 a[L0];
@@ -411,9 +413,15 @@ __device__ __forceinline__ uint32_t group_estimate(const uint32_t (&r)[NW]) {
     }
     const uint32_t e = ((uint32_t)a[0].x + (uint32_t)a[0].y) >> 1;
     if constexpr (G == 1) return e;
-    const uint32_t s = (uint32_t)grp_sum<G>((int32_t)e);
-    if constexpr (G == 2) return s >> 1;
-    return (s - grp_min_u32<G>(e) - grp_max_u32<G>(e)) / (uint32_t)(G - 2);
+    const bool ok = real >= (uint32_t)(3 * NW / 2);
+    const uint32_t nv = (uint32_t)grp_sum<G>(ok ? 1 : 0);  // the same in every group
+    const uint32_t s = (uint32_t)grp_sum<G>((int32_t)(ok ? e : 0u));
+    if constexpr (G == 2) return nv == 2u ? s >> 1 : (nv == 1u ? s : grp_min_u32<G>(e));
+    if (nv == (uint32_t)G) return (s - grp_min_u32<G>(e) - grp_max_u32<G>(e)) / (uint32_t)(G - 2);
+    if (nv >= 3u)
+        return (uint32_t)((float)(s - grp_min_u32<G>(ok ? e : 0xFFFFu) - grp_max_u32<G>(ok ? e : 0u)) *
+                          __builtin_amdgcn_rcpf((float)(nv - 2u)));
+    return nv == 2u ? s >> 1 : (nv == 1u ? s : grp_min_u32<G>(e));
 }
 
 // Neighbour rank r1 = r0 + 1 from v0 and cle = #{x <= v0}.
@@ -464,7 +472,7 @@ __device__ __forceinline__ void rank_pairs(const uint32_t (&raw)[C][NW], uint32_
         uint32_t y[C][ND], lo[C];
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            const uint32_t est = group_estimate<G, NW>(raw[c]);
+            const uint32_t est = group_estimate<G, NW>(raw[c], real);
             lo[c] = min(est >= 63u ? est - 63u : 0u, LO_MAX);
             pack_window<NW, TOP>(raw[c], lo[c], y[c]);
         }
@@ -551,27 +559,28 @@ __device__ __forceinline__ float frame_dist(const uint32_t (&s)[4], const float 
 // an odd/even pair of offsets that spreads the even and odd pixels) so that the finishing
 // lanes (fixed g, consecutive p) and the writing lanes (the pixels of a wave x G blocks)
 // both spread over the banks; per-pixel values are stored channel-major.
-template <int C, int G, int F, int X = 1>
+// PAIR: the tile reads 16-bit samples of several pixels with one dword-aligned load.
+template <int C, int G, int F, int X = 1, bool PAIR = (X == 2)>
 struct TileShared {
     static constexpr int P = X * 256 / G;      // pixels per tile
     static constexpr int NS = G * P;           // lane summary slots (X per lane)
     static constexpr int MW = (F + 31) / 32;   // mask words per lane and pixel
     static constexpr int OS = F + 2;           // offset-table stride of a lane block
     uint64_t off[G * OS];      // frame byte offsets at oidx(t); positions >= N repeat N-1
-    // Two pixels per lane: with r the tile row's first sample address modulo 4 (shared by
-    // every pixel pair of the row, which start 12 or 16 bytes apart), aoff = (off + r) & ~3
-    // and sft = (off + r) & 3, so the lane whose pair starts at base loads 16 bytes at
-    // (base & ~3) + aoff and realigns them by sft.
-    uint64_t aoff[X == 2 ? G * OS : 1];
-    uint32_t sft[X == 2 ? G * OS : 1];
+    // PAIR: with r the tile row's first sample address modulo 4 (shared by every lane's pixels
+    // in the row, which start 8, 12 or 16 bytes apart), aoff = (off + r) & ~3 and
+    // sft = (off + r) & 3, so the lane whose pixels start at base loads from
+    // (base & ~3) + aoff and realigns by sft.
+    uint64_t aoff[PAIR ? G * OS : 1];
+    uint32_t sft[PAIR ? G * OS : 1];
     uint32_t mask[MW][NS];     // [w][slot]: outlier bits of frames g*F + 32w + b
     float lmax[NS];            // [slot]: the largest outlier distance (valid when lmaxi != ~0)
     uint32_t lmaxi[NS];        // [slot]: its first frame
-    float med[4][P];
-    float iqr_inv[4][P];
-    uint32_t s0[4][P];       // frame 0 samples
-    uint32_t sum_all[4][P];  // average modes
-    uint32_t sum_out[4][P];
+    float med[C][P];
+    float iqr_inv[C][P];
+    uint32_t s0[C][P];       // frame 0 samples
+    uint32_t sum_all[C][P];  // average modes
+    uint32_t sum_out[C][P];
     __device__ static __forceinline__ uint32_t oidx(uint32_t t) { return t + 2u * (t / (uint32_t)F); }
     __device__ static __forceinline__ uint32_t rot(uint32_t g) {
         return X == 1 ? 4u * g : (g & 1u) + (g >> 1) * (64u / (uint32_t)G);
@@ -590,8 +599,8 @@ __device__ __forceinline__ void load_offsets(uint64_t* off, uint32_t count, cons
     for (uint32_t i = threadIdx.x; i < count; i += 256) off[i + 2u * (i / (uint32_t)F)] = pos_off[min(i, n - 1)] * B;
 }
 
-// load_offsets plus the realignment tables of a two-pixel tile (TileShared::aoff, sft); r is
-// the tile row's first sample address modulo 4.
+// load_offsets plus the realignment tables of a PAIR tile (TileShared::aoff, sft); r is the tile
+// row's first sample address modulo 4.
 template <int B, int F>
 __device__ __forceinline__ void load_offsets_pair(uint64_t* off, uint64_t* aoff, uint32_t* sft, uint32_t count,
                                                   const uint64_t* __restrict__ pos_off, uint32_t n, uint32_t r) {
@@ -607,52 +616,54 @@ __device__ __forceinline__ void load_offsets_pair(uint64_t* off, uint64_t* aoff,
 // Loads the F frames of one lane block into raw[e*C + c][j/2] (pixel e of the lane, frame j
 // in half j&1); base is the lane's first pixel in stack slot 0 and off the block's F frame
 // byte offsets.
-// Two pixels per lane (16-bit stacks) take one 16-byte load per frame from the dword
-// boundary at or below the pair's first sample (3 channels: the pair's 12 bytes start 2-byte
-// aligned, so the load reads up to 4 bytes past them and v_alignbyte realigns by the address'
-// low bits).  All F loads are issued before the first is used, so a lane keeps its whole
-// block in flight; the byte shifts are read from the tile's shift table afterwards rather
-// than held in registers meanwhile.
+// Several pixels per lane (16-bit stacks) take one load per frame from the dword boundary at or
+// below the first sample: with an odd channel count the pixels start 2-byte aligned, so the
+// load covers one dword more than they fill and v_alignbyte realigns by the address' low bits
+// (3 channels: 16 bytes for a pair's 12; 1 channel: 12 bytes for four pixels' 8).  All F loads
+// are issued before the first is used, so a lane keeps its whole block in flight; the byte
+// shifts are read from the tile's shift table afterwards rather than held in registers
+// meanwhile.
 template <int B, int C, int F, int X>
 __device__ __forceinline__ void load_block(const uint8_t* __restrict__ base, const uint64_t* off,
                                            uint32_t (&raw)[X * C][F / 2], const uint64_t* aoff = nullptr,
                                            const uint32_t* sft = nullptr) {
-    static_assert(X == 1 || (X == 2 && B == 2 && C >= 3), "two pixels per lane: 16-bit, 3 or 4 channels");
-    if constexpr (X == 2) {
-        typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-        typedef const __attribute__((address_space(1))) u32x4 gu4;
+    static_assert(X == 1 || (B == 2 && X * C % 2 == 0 && X * C <= 8), "several pixels per lane: 16 bits");
+    if constexpr (X > 1) {
+        constexpr int NWD = X * C / 2;               // dwords a lane's pixels fill
+        constexpr int NQ = C % 2 ? NWD + 1 : NWD;    // dwords loaded
+        typedef unsigned int u32xq __attribute__((ext_vector_type(NQ)));
+        typedef unsigned int u32xq_a4 __attribute__((ext_vector_type(NQ), aligned(4)));
+        typedef const __attribute__((address_space(1))) u32xq_a4 guq;
         typedef const volatile __attribute__((address_space(3))) uint32_t lu32;
-        uint32_t q[F][4];
+        uint32_t q[F][NQ];
         const uintptr_t base_al = (uintptr_t)base & ~(uintptr_t)3;
 #pragma unroll
         for (int t = 0; t < F; ++t) {
-            const u32x4 v = *(gu4*)(base_al + aoff[t]);
-            q[t][0] = v.x;
-            q[t][1] = v.y;
-            q[t][2] = v.z;
-            q[t][3] = v.w;
+            const u32xq v = *(guq*)(base_al + aoff[t]);
+#pragma unroll
+            for (int h = 0; h < NQ; ++h) q[t][h] = v[h];
         }
         __builtin_amdgcn_sched_barrier(0);
         lu32* sft32 = (lu32*)sft;
 #pragma unroll
         for (int i = 0; i < F / 2; ++i) {
-            uint32_t a[4], b[4];
-            if constexpr (C == 3) {
+            uint32_t a[NWD], b[NWD];
+            if constexpr (NQ > NWD) {
                 const uint32_t s0 = sft32[2 * i], s1 = sft32[2 * i + 1];
 #pragma unroll
-                for (int h = 0; h < 3; ++h) {  // [c0|c1], [c2|c0'], [c1'|c2'] of pixels 0 and 1
+                for (int h = 0; h < NWD; ++h) {  // two samples per dword, in pixel and channel order
                     a[h] = __builtin_amdgcn_alignbyte(q[2 * i][h + 1], q[2 * i][h], s0);
                     b[h] = __builtin_amdgcn_alignbyte(q[2 * i + 1][h + 1], q[2 * i + 1][h], s1);
                 }
             } else {
 #pragma unroll
-                for (int h = 0; h < 4; ++h) {
+                for (int h = 0; h < NWD; ++h) {
                     a[h] = q[2 * i][h];
                     b[h] = q[2 * i + 1][h];
                 }
             }
 #pragma unroll
-            for (int h = 0; h < C; ++h) {
+            for (int h = 0; h < NWD; ++h) {
                 raw[2 * h][i] = __builtin_amdgcn_perm(b[h], a[h], 0x05040100u);
                 raw[2 * h + 1][i] = __builtin_amdgcn_perm(b[h], a[h], 0x07060302u);
             }
@@ -729,10 +740,10 @@ constexpr int kOdistSlots = 16;
 // the classification's squared distances of pixel p's outliers, slot s * P + p holding the
 // s-th outlier counted from the last frame, for up to kOdistSlots outliers; with it the
 // average mode takes the distances from there instead of re-reading the samples.
-template <int B, int C, int G, int F, int X, bool ABS>
+template <int B, int C, int G, int F, int X, bool ABS, bool PAIR>
 __device__ __forceinline__ void finish_pixel(const OutlierK& k, uint32_t bx, uint32_t y, uint32_t p,
-                                             const TileShared<C, G, F, X>& sh, const float* odist = nullptr) {
-    using TS = TileShared<C, G, F, X>;
+                                             const TileShared<C, G, F, X, PAIR>& sh, const float* odist = nullptr) {
+    using TS = TileShared<C, G, F, X, PAIR>;
     constexpr int P = TS::P;
     constexpr int MW = TS::MW;
     constexpr uint32_t MAXV = B == 1 ? 255u : 65535u;
@@ -749,8 +760,8 @@ __device__ __forceinline__ void finish_pixel(const OutlierK& k, uint32_t bx, uin
     const bool want_iqr = !ABS || k.stats != nullptr;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        med[c] = sh.med[c][p];
-        iqr_inv[c] = want_iqr ? sh.iqr_inv[c][p] : 0.0f;
+        med[c] = c < C ? sh.med[c < C ? c : 0][p] : 0.0f;
+        iqr_inv[c] = want_iqr && c < C ? sh.iqr_inv[c < C ? c : 0][p] : 0.0f;
         wi[c] = ABS ? k.w[c] : k.w[c] * iqr_inv[c];
         sg[c] = signum_f(k.w[c]);
     }
@@ -993,17 +1004,30 @@ __device__ __forceinline__ void finish_pixel(const OutlierK& k, uint32_t bx, uin
     }
 }
 
+// The sample positions' offsets of a `--sample` tile, laid out as TileShared's tables.
+template <int G, int FS>
+struct SampleTable {
+    static constexpr int N = FS > 0 ? G * (FS + 2) : 1;
+    uint64_t off[N];
+    uint64_t aoff[N];
+    uint32_t sft[N];
+};
+
 // One tile: P = X*256/G pixels of row y starting at pixel bx * P; lane (pl, g) holds frame
 // block g of pixels bx*P + pl*X + e, e < X.  sh.off must hold the tile's frame offsets
-// (load_offsets) and be visible to all lanes.  Every lane of the workgroup must call this
-// (it synchronises once).  With X = 2 the lanes read up to 16 bytes past their pixels'
-// samples (load12_a2, and pixel out_w of a row when out_w is odd); the launcher checks that
-// those bytes lie inside the stack allocation.  lane: threadIdx.x.
-template <int B, int C, int G, int F, int X, bool ABS>
+// (load_offsets) and be visible to all lanes; with FS > 0 (`--sample`) ssh holds those of the
+// sample positions, whose FS-frame block is loaded first: the ranks come from it, and its
+// registers are free again before the block of all frames is loaded.  Every lane of the
+// workgroup must call this (it synchronises once).  With X > 1 the lanes read up to 16 bytes
+// from their first sample (and pixels past out_w of a row whose width is no multiple of X); the
+// launcher checks that those bytes lie inside the stack allocation.  lane: threadIdx.x.
+template <int B, int C, int G, int F, int X, int FS, bool ABS, bool PAIR>
 __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uint32_t y,
-                                             TileShared<C, G, F, X>& sh, uint32_t lane) {
-    static_assert(F % 4 == 0 && F <= 64 && G <= 8 && (X == 1 || X == 2), "tile shape");
-    using TS = TileShared<C, G, F, X>;
+                                             TileShared<C, G, F, X, PAIR>& sh, const SampleTable<G, FS>& ssh,
+                                             uint32_t lane) {
+    static_assert(F % 4 == 0 && F <= 64 && G <= 32, "tile shape");
+    static_assert(FS == 0 || (X > 1 && FS % 4 == 0), "sample blocks go with several pixels per lane");
+    using TS = TileShared<C, G, F, X, PAIR>;
     constexpr int P = TS::P;
     constexpr int MW = TS::MW;
     constexpr int NW = F / 2;
@@ -1013,62 +1037,81 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
 
     const uint32_t g = lane % G;
     const uint32_t t0 = g * F;
-    const int32_t ntot = G * F;
+    const uint32_t real = N > t0 ? min(N - t0, (uint32_t)F) : 0u;  // real frames in this block
+    const bool full_tile = N == (uint32_t)(G * F);
     {
         const uint32_t pl = lane / G;
         const uint32_t x0 = bx * P + pl * X;
         const uint64_t pix = ((uint64_t)y * k.stack_w + (x0 < k.out_w ? x0 : 0u)) * C;
 
-        // ---- the lane's frame block; pads above N are set to MAXV
-        uint32_t raw[X * C][NW];
-        if constexpr (X == 2) load_block<B, C, F, X>(k.stack + pix * B, sh.off, raw, sh.aoff + g * TS::OS, sh.sft + g * TS::OS);
-        else load_block<B, C, F, X>(k.stack + pix * B, sh.off + g * TS::OS, raw);
-        if (N < (uint32_t)(G * F)) {  // grid-uniform: only stacks that do not fill the tile
+        // ---- medians / inverse IQR per pixel and channel
+        const RankPlan plan = rank_plan_core(FS > 0 ? k.n_sample : N, ABS);
+        uint32_t lowmed[X * C];  // the medians rounded down
+        float med[X][4], iqr_inv[X][4];
+        auto ranks = [&](auto nf_t, auto& blk, uint32_t blk_real) {
+            constexpr int NF = decltype(nf_t)::value, NFW = NF / 2;  // frames per lane in the ranked block
+            constexpr bool WINDOW = ABS && (B == 1 || NFW >= 3);
+            StaticFor<0, X>::run([&](auto e_t) {
+                constexpr int E = decltype(e_t)::value;
+                const uint32_t (&re)[C][NFW] = *reinterpret_cast<const uint32_t(*)[C][NFW]>(&blk[E * C][0]);
+                uint32_t m0[C], m1[C], a0[C], a1[C], b0[C], b1[C];
+                if constexpr (!ABS && B == 1) {
+                    rank_triples_u8<G, NFW, C>(re, plan, G * NF, blk_real, m0, m1, a0, a1, b0, b1);
+                } else {
+                    rank_pairs<B, G, NFW, C, WINDOW>(re, plan.m0, plan.m1, G * NF, blk_real, m0, m1);
+                    if constexpr (!ABS) {
+                        rank_pairs<B, G, NFW, C, false>(re, plan.a0, plan.a1, G * NF, blk_real, a0, a1);
+                        rank_pairs<B, G, NFW, C, false>(re, plan.b0, plan.b1, G * NF, blk_real, b0, b1);
+                    }
+                }
 #pragma unroll
-            for (int i = 0; i < NW; ++i) {
-                const uint32_t t = t0 + 2 * i;
+                for (int c = 0; c < 4; ++c) {
+                    med[E][c] = 0.0f;
+                    iqr_inv[E][c] = 0.0f;
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    float mc, ic;
+                    if constexpr (ABS) stats_from_values(plan, m0[c], m1[c], 0, 0, 0, 0, true, &mc, &ic);
+                    else stats_from_values(plan, m0[c], m1[c], a0[c], a1[c], b0[c], b1[c], false, &mc, &ic);
+                    // channels without weight keep zero statistics
+                    med[E][c] = k.w[c] == 0.0f ? 0.0f : mc;
+                    iqr_inv[E][c] = k.w[c] == 0.0f ? 0.0f : ic;
+                    lowmed[E * C + c] = (m0[c] + m1[c]) >> 1;
+                }
+            });
+        };
+        // pads from frame `count` of the block on take the largest value: the ranks below the
+        // frame count never see them
+        auto pad = [&](auto nf_t, auto& blk, uint32_t count) {
+            constexpr int NFW = decltype(nf_t)::value / 2;
+#pragma unroll
+            for (int i = 0; i < NFW; ++i) {
 #pragma unroll
                 for (int c = 0; c < X * C; ++c) {
-                    uint32_t r = raw[c][i];
-                    r = t + 1 >= N ? (r & 0xFFFFu) | (MAXV << 16) : r;
-                    r = t >= N ? MAXV | (MAXV << 16) : r;
-                    raw[c][i] = r;
+                    uint32_t r = blk[c][i];
+                    r = 2u * i + 1 >= count ? (r & 0xFFFFu) | (MAXV << 16) : r;
+                    r = 2u * i >= count ? MAXV | (MAXV << 16) : r;
+                    blk[c][i] = r;
                 }
             }
+        };
+        if constexpr (FS > 0) {
+            uint32_t smp[X * C][FS / 2];
+            load_block<B, C, FS, X>(k.stack + pix * B, ssh.off, smp, ssh.aoff + g * (FS + 2), ssh.sft + g * (FS + 2));
+            const uint32_t ts = g * FS, sreal = k.n_sample > ts ? min(k.n_sample - ts, (uint32_t)FS) : 0u;
+            if (k.n_sample < (uint32_t)(G * FS)) pad(std::integral_constant<int, FS>{}, smp, sreal);
+            ranks(std::integral_constant<int, FS>{}, smp, sreal);
         }
 
-        // ---- medians / inverse IQR per pixel and channel
-        const RankPlan plan = rank_plan_core(N, ABS);
-        const uint32_t real = N > t0 ? min(N - t0, (uint32_t)F) : 0u;  // real frames in this block
-        float med[X][4], iqr_inv[X][4];
-        StaticFor<0, X>::run([&](auto e_t) {
-            constexpr int E = decltype(e_t)::value;
-            const uint32_t (&re)[C][NW] = *reinterpret_cast<const uint32_t(*)[C][NW]>(&raw[E * C][0]);
-            uint32_t m0[C], m1[C], a0[C], a1[C], b0[C], b1[C];
-            if constexpr (!ABS && B == 1) {
-                rank_triples_u8<G, NW, C>(re, plan, ntot, real, m0, m1, a0, a1, b0, b1);
-            } else {
-                rank_pairs<B, G, NW, C, ABS>(re, plan.m0, plan.m1, ntot, real, m0, m1);
-                if constexpr (!ABS) {
-                    rank_pairs<B, G, NW, C, false>(re, plan.a0, plan.a1, ntot, real, a0, a1);
-                    rank_pairs<B, G, NW, C, false>(re, plan.b0, plan.b1, ntot, real, b0, b1);
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                med[E][c] = 0.0f;
-                iqr_inv[E][c] = 0.0f;
-            }
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                float mc, ic;
-                if constexpr (ABS) stats_from_values(plan, m0[c], m1[c], 0, 0, 0, 0, true, &mc, &ic);
-                else stats_from_values(plan, m0[c], m1[c], a0[c], a1[c], b0[c], b1[c], false, &mc, &ic);
-                // channels without weight keep zero statistics
-                med[E][c] = k.w[c] == 0.0f ? 0.0f : mc;
-                iqr_inv[E][c] = k.w[c] == 0.0f ? 0.0f : ic;
-            }
-        });
+        // ---- the lane's frame block
+        uint32_t raw[X * C][NW];
+        if constexpr (X > 1) load_block<B, C, F, X>(k.stack + pix * B, sh.off, raw, sh.aoff + g * TS::OS, sh.sft + g * TS::OS);
+        else load_block<B, C, F, X>(k.stack + pix * B, sh.off + g * TS::OS, raw);
+        if constexpr (FS == 0) {
+            if (!full_tile) pad(std::integral_constant<int, F>{}, raw, real);  // grid-uniform
+            ranks(std::integral_constant<int, F>{}, raw, real);
+        }
 
         // ---- classification over the lane's frames
         float wi[X][4], sg[4];
@@ -1086,7 +1129,6 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
         const float tsq = k.th.min * k.th.min;
         const bool want_max = k.outlier == 2 || k.stats != nullptr;
         const bool want_sums = k.background == 2 || k.outlier == 3;
-        const bool full_tile = N == (uint32_t)(G * F);
         uint32_t m[X][MW];
         float lmax[X];
         uint32_t lmaxi[X];
@@ -1100,24 +1142,40 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
 #pragma unroll
             for (int c = 0; c < 4; ++c) sum_all[e][c] = sum_out[e][c] = 0;
         }
+        // With non-negative weights the pads become the median rounded down: no sample lies
+        // nearer to the median, so a pad's distance is at most every real frame's, and as ties
+        // go to the lower frame a pad is never the largest of a lane with a real frame.  The
+        // passes below then need no test of the frame count, and the bound check holds for
+        // every tile.
+        uint32_t pad_v[X * C];
+#pragma unroll
+        for (int c = 0; c < X * C; ++c) pad_v[c] = pos ? lowmed[c] : MAXV;
+        if (!full_tile) {
+#pragma unroll
+            for (int i = 0; i < NW; ++i) {
+                const uint32_t mk = 2u * i >= real ? 0xFFFFFFFFu : (2u * i + 1 >= real ? 0xFFFF0000u : 0u);
+#pragma unroll
+                for (int c = 0; c < X * C; ++c)
+                    raw[c][i] = (raw[c][i] & ~mk) | (mk & (pad_v[c] | (pad_v[c] << 16)));
+            }
+        }
 
         // Frames run from last to first so that the mask shifts in bit j for frame j; the
         // largest distance keeps the lowest frame among ties (>=).  lmax starts at the
-        // threshold, so `d >= lmax` also implies that the frame is an outlier.
-        auto classify = [&](auto e_t, auto unit_t, auto pos_t, auto max_t, auto sums_t, auto check_t) {
+        // threshold, so `d >= lmax` also implies that the frame is an outlier.  CHECK: the pads
+        // are the largest value (negative weights).
+        auto classify = [&](auto e_t, auto unit_t, auto pos_t, auto max_t, auto check_t) {
             constexpr int E = decltype(e_t)::value;
             constexpr bool UNIT = decltype(unit_t)::value, POS = decltype(pos_t)::value;
-            constexpr bool MAXT = decltype(max_t)::value, SUMS = decltype(sums_t)::value;
-            constexpr bool CHECK = decltype(check_t)::value;
+            constexpr bool MAXT = decltype(max_t)::value, CHECK = decltype(check_t)::value;
 #pragma unroll
             for (int j = F - 1; j >= 0; --j) {
-                uint32_t xs[4];
                 float d = 0.0f;
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
                     const uint32_t w32 = raw[E * C + c][j >> 1];
-                    xs[c] = (j & 1) ? (w32 >> 16) : (w32 & 0xFFFFu);
-                    const float diff = med[E][c] - (float)xs[c];
+                    const uint32_t xs = (j & 1) ? (w32 >> 16) : (w32 & 0xFFFFu);
+                    const float diff = med[E][c] - (float)xs;
                     const float a = UNIT ? diff : wi[E][c] * diff;
                     float term = a * a;
                     if constexpr (!POS) term = sg[c] * term;
@@ -1126,25 +1184,9 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
                 const bool o = d >= tsq;  // pads are masked out after the loop
                 m[E][j >> 5] = (m[E][j >> 5] << 1) | (o ? 1u : 0u);
                 bool in = true;
-                if constexpr (CHECK) in = t0 + (uint32_t)j < N;
+                if constexpr (CHECK) in = (uint32_t)j < real;
                 if constexpr (MAXT) {
                     if (in && d >= lmax[E]) { lmax[E] = d; lmaxi[E] = t0 + (uint32_t)j; }
-                }
-                if constexpr (SUMS && CHECK) {
-#pragma unroll
-                    for (int c = 0; c < C; ++c) sum_out[E][c] += (o && in) ? xs[c] : 0u;
-                }
-            }
-            if constexpr (SUMS && !CHECK) {
-                // every frame is real: the outliers' sums from the mask, two frames per
-                // v_dot2_u32_u16 (the mask's two bits spread to one 0/1 half per frame)
-#pragma unroll
-                for (int i = 0; i < NW; ++i) {
-                    const uint32_t b = (m[E][i >> 4] >> (2 * (i & 15))) & 3u;
-                    const uint32_t sel = (b & 1u) | ((b & 2u) << 15);
-#pragma unroll
-                    for (int c = 0; c < C; ++c)
-                        sum_out[E][c] = __builtin_amdgcn_udot2(as_us2(raw[E * C + c][i]), as_us2(sel), sum_out[E][c], false);
                 }
             }
         };
@@ -1157,7 +1199,7 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
             // (correct rounding is monotone), so when that bound is below the threshold no
             // frame of this lane can be an outlier and the per-frame pass is skipped.
             bool may_outlier = true;
-            if (pos && full_tile) {
+            if (pos) {
                 float bound = 0.0f;
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
@@ -1176,53 +1218,57 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
                 may_outlier = bound >= tsq;
             }
             if (may_outlier) {
-                if (!full_tile) classify(e_t, F_{}, F_{}, T_{}, T_{}, T_{});
+                if (!pos) classify(e_t, F_{}, F_{}, T_{}, T_{});
                 else if (want_max) {
-                    if (want_sums) classify(e_t, F_{}, F_{}, T_{}, T_{}, F_{});
-                    else if (unit) classify(e_t, T_{}, T_{}, T_{}, F_{}, F_{});
-                    else if (pos) classify(e_t, F_{}, T_{}, T_{}, F_{}, F_{});
-                    else classify(e_t, F_{}, F_{}, T_{}, F_{}, F_{});
+                    if (unit) classify(e_t, T_{}, T_{}, T_{}, F_{});
+                    else classify(e_t, F_{}, T_{}, T_{}, F_{});
                 } else {
-                    if (want_sums) {
-                        if (pos) classify(e_t, F_{}, T_{}, F_{}, T_{}, F_{});
-                        else classify(e_t, F_{}, F_{}, F_{}, T_{}, F_{});
-                    } else if (unit) classify(e_t, T_{}, T_{}, F_{}, F_{}, F_{});
-                    else if (pos) classify(e_t, F_{}, T_{}, F_{}, F_{}, F_{});
-                    else classify(e_t, F_{}, F_{}, F_{}, F_{}, F_{});
+                    if (unit) classify(e_t, T_{}, T_{}, F_{}, F_{});
+                    else classify(e_t, F_{}, T_{}, F_{}, F_{});
                 }
             }
+#pragma unroll
+            for (int w = 0; w < MW; ++w) {
+                const int32_t nw = (int32_t)real - 32 * w;
+                m[E][w] &= nw >= 32 ? 0xFFFFFFFFu : (nw <= 0 ? 0u : (1u << nw) - 1u);
+            }
+            if (real == 0u) lmaxi[E] = NONE;
         });
         if (want_sums) {
-            // all-frame sums through v_sad_u16 against zero; pads (MAXV) are taken back out
-            const uint32_t npad = t0 + F > N ? min(t0 + F - N, (uint32_t)F) : 0u;
+            // all-frame sums through v_sad_u16 against zero, pads taken back out; the outliers'
+            // sums from the mask, two frames per v_dot2_u32_u16 (the mask's two bits spread to
+            // one 0/1 half per frame)
+            const uint32_t npad = (uint32_t)F - real;
 #pragma unroll
-            for (int e = 0; e < X; ++e)
+            for (int e = 0; e < X; ++e) {
+#pragma unroll
+                for (int i = 0; i < NW; ++i) {
+                    const uint32_t b = (m[e][i >> 4] >> (2 * (i & 15))) & 3u;
+                    const uint32_t sel = (b & 1u) | ((b & 2u) << 15);
+#pragma unroll
+                    for (int c = 0; c < C; ++c)
+                        sum_out[e][c] = __builtin_amdgcn_udot2(as_us2(raw[e * C + c][i]), as_us2(sel), sum_out[e][c], false);
+                }
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
                     uint32_t acc = 0;
 #pragma unroll
                     for (int i = 0; i < NW; ++i) acc = __builtin_amdgcn_sad_u16(raw[e * C + c][i], 0u, acc);
-                    sum_all[e][c] = (uint32_t)grp_sum<G>((int32_t)(acc - npad * MAXV));
+                    sum_all[e][c] = (uint32_t)grp_sum<G>((int32_t)(acc - npad * pad_v[e * C + c]));
                     sum_out[e][c] = (uint32_t)grp_sum<G>((int32_t)sum_out[e][c]);
                 }
+            }
         }
 
         // ---- leave the lane's summaries and the pixels' statistics in LDS
-        {
-            const int32_t nv = min((int32_t)N - (int32_t)t0, (int32_t)F);  // valid frames in this block
 #pragma unroll
-            for (int e = 0; e < X; ++e) {
-                const uint32_t sl = TS::slot(g, pl * X + e);
+        for (int e = 0; e < X; ++e) {
+            const uint32_t sl = TS::slot(g, pl * X + e);
 #pragma unroll
-                for (int w = 0; w < MW; ++w) {
-                    const int32_t nw = nv - 32 * w;
-                    const uint32_t vm = nw >= 32 ? 0xFFFFFFFFu : (nw <= 0 ? 0u : (1u << nw) - 1u);
-                    sh.mask[w][sl] = m[e][w] & vm;
-                }
-                if (want_max) {
-                    sh.lmax[sl] = lmax[e];
-                    sh.lmaxi[sl] = lmaxi[e];
-                }
+            for (int w = 0; w < MW; ++w) sh.mask[w][sl] = m[e][w];
+            if (want_max) {
+                sh.lmax[sl] = lmax[e];
+                sh.lmaxi[sl] = lmaxi[e];
             }
         }
         if (g == 0) {
@@ -1233,12 +1279,9 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
             for (int e = 0; e < X; ++e) {
                 const uint32_t p = pl * X + e;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
+                for (int c = 0; c < C; ++c) {
                     sh.med[c][p] = med[e][c];
                     if (want_iqr) sh.iqr_inv[c][p] = iqr_inv[e][c];
-                }
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
                     if (want_s0) sh.s0[c][p] = raw[e * C + c][0] & 0xFFFFu;
                     if (want_sums) {
                         sh.sum_all[c][p] = sum_all[e][c];
@@ -1262,26 +1305,40 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nb) {
 
 // Waves per SIMD the register allocator is asked to fit without spilling: 3-channel 32-frame
 // tiles fit five (absolute thresholds) or four (relative thresholds: three rank searches),
-// 4-channel tiles one fewer; two pixels per lane double the frame registers (three waves,
-// two for 4 channels or relative thresholds); the 64-frame tiles get the whole register file.
+// 4-channel tiles one fewer; two 3- or 4-channel pixels per lane double the frame registers
+// (three waves, two for 4 channels or relative thresholds), two or four pixels of two or one
+// channels take two thirds of that (three waves, four for two channels and absolute thresholds); the 64-frame
+// tiles get the whole register file.
 constexpr int waves_hint(int F, int C, bool absolute, int X = 1) {
-    return F > 32 ? 1 : X == 2 ? (absolute && C == 3 ? 3 : 2) : (absolute ? 5 : 4) - (C > 3 ? 1 : 0);
+    return F > 32   ? 1
+           : X == 1 ? (absolute ? 5 : 4) - (C > 3 ? 1 : 0)
+           : C == 1 ? 3
+           : C == 2 ? (absolute ? 4 : 3)
+                    : (absolute && C == 3 ? 3 : 2);
 }
 
-template <int B, int C, int G, int F, int X, bool ABS>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint(F, C, ABS, X))))
-outlier_fast_kernel(OutlierK k, uint32_t tiles_x) {
-    __shared__ TileShared<C, G, F, X> sh;
-    const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
-    const uint32_t y = tile / tiles_x;
-    if constexpr (X == 2) {
+template <int B, int C, int G, int F, int X, int FS>
+__device__ __forceinline__ void load_tables(const OutlierK& k, uint32_t y, TileShared<C, G, F, X, (X > 1)>& sh,
+                                            SampleTable<G, FS>& ssh) {
+    if constexpr (X > 1) {
         const uint32_t r = (uint32_t)((uintptr_t)k.stack + (uint64_t)y * k.stack_w * C * B) & 3u;
         load_offsets_pair<B, F>(sh.off, sh.aoff, sh.sft, G * F, k.pos_off, k.n, r);
+        if constexpr (FS > 0) load_offsets_pair<B, FS>(ssh.off, ssh.aoff, ssh.sft, G * FS, k.samp_off, k.n_sample, r);
     } else {
         load_offsets<B, F>(sh.off, G * F, k.pos_off, k.n);
     }
     __syncthreads();
-    outlier_tile<B, C, G, F, X, ABS>(k, tile % tiles_x, y, sh, threadIdx.x);
+}
+
+template <int B, int C, int G, int F, int X, int FS, bool ABS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint(F, C, ABS, X))))
+outlier_fast_kernel(OutlierK k, uint32_t tiles_x) {
+    __shared__ TileShared<C, G, F, X, (X > 1)> sh;
+    __shared__ SampleTable<G, FS> ssh;
+    const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+    const uint32_t y = tile / tiles_x;
+    load_tables<B>(k, y, sh, ssh);
+    outlier_tile<B, C, G, F, X, FS, ABS>(k, tile % tiles_x, y, sh, ssh, threadIdx.x);
 }
 
 }  // namespace cp

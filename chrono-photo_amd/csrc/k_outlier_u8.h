@@ -323,11 +323,11 @@ constexpr bool keeps_odist() {
 // * P floats of LDS when keeps_odist(), else unused.
 template <int C, int G, int F, int X, int FS, bool ABS, bool SORT = false>
 __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, uint32_t y,
-                                                TileShared<C, G, F, X>& sh, const uint64_t* soff, uint32_t lane,
+                                                TileShared<C, G, F, X, false>& sh, const uint64_t* soff, uint32_t lane,
                                                 float* odist = nullptr) {
     static_assert(F % 8 == 0 && F <= 64 && G <= 32 && FS % 4 == 0 && (X == 1 || X == 4), "tile shape");
     static_assert(!SORT || (G == 1 && X == 1 && FS == 0), "sorting-network ranks: one lane per pixel");
-    using TS = TileShared<C, G, F, X>;
+    using TS = TileShared<C, G, F, X, false>;
     constexpr int P = TS::P;
     constexpr int MW = TS::MW;
     constexpr int ND = F / 4;
@@ -662,12 +662,9 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
             for (int e = 0; e < X; ++e) {
                 const uint32_t p = pl * X + e;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
+                for (int c = 0; c < C; ++c) {
                     sh.med[c][p] = med[e][c];
                     if (want_iqr) sh.iqr_inv[c][p] = iqr_inv[e][c];
-                }
-#pragma unroll
-                for (int c = 0; c < C; ++c) {
                     if (want_s0) sh.s0[c][p] = yv[e * C + c][0] & 0xFFu;
                     if (want_sums) {
                         sh.sum_all[c][p] = sum_all[e][c];
@@ -692,9 +689,9 @@ constexpr int waves_hint_u8(int C, int F, int X, int FS, bool sort) {
 template <int C, int G, int F, int X, int FS, bool ABS, bool SORT = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, SORT))))
 outlier_u8_kernel(OutlierK k, uint32_t tiles_x) {
-    __shared__ TileShared<C, G, F, X> sh;
+    __shared__ TileShared<C, G, F, X, false> sh;
     __shared__ uint64_t soff[FS > 0 ? G * (FS + 2) : 1];
-    __shared__ float odist[keeps_odist<G, F, X, FS, SORT>() ? (kOdistSlots + 1) * TileShared<C, G, F, X>::P : 1];
+    __shared__ float odist[keeps_odist<G, F, X, FS, SORT>() ? (kOdistSlots + 1) * TileShared<C, G, F, X, false>::P : 1];
     const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
     load_offsets<1, F>(sh.off, G * F, k.pos_off, k.n);
     if constexpr (FS > 0) load_offsets<1, FS>(soff, G * FS, k.samp_off, k.n_sample);

@@ -23,8 +23,8 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
     // The register-resident kernels need exact integer sums for the average modes
     // (N * max sample < 2^24: always for 8-bit stacks).  8-bit composites take the packed-byte
     // kernel up to 1280 frames (and, with a `--sample` subset, up to 128 sample frames) or the
-    // tuned choice between the two kernels; 16-bit ones the 16-bit kernel up to 512 frames
-    // without a sample subset; the one-lane-per-pixel generic kernel takes the rest.  A
+    // tuned choice between the two kernels; 16-bit ones the 16-bit kernel up to 1024 frames (and
+    // up to 128 sample frames); the one-lane-per-pixel generic kernel takes the rest.  A
     // packed-byte choice whose wide loads would read past a borrowed stack's end falls back to
     // the bucket's 16-bit-halves shape, or to the generic kernel where the bucket has none.
     OutlierPlan p;
@@ -39,9 +39,15 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
             const int sh = u8_shape_for(k.n, true, k.n_sample);
             if (sh >= 0 && u8_fits(sh)) p = {kPlanU8, sh};
         }
+        if (st->bps == 2 && k.n <= kFastMaxFrames && k.n_sample <= kFastMaxSample && k.samp_off) {
+            const int sh = fast_sample_shape(k.n, k.n_sample);
+            if (sh >= 0 && pair_tile_fits(st->dev, st->alloc_bytes, st->bps, st->channels, k, max_pos))
+                p = {kPlanFast, sh};
+        }
         return p;
     }
     int choice = ctx->choice_for(st->bps, st->channels, k.n, k.th.absolute != 0);
+    if (choice < 0) choice = untuned_shape(st->bps, k.n);
     if (choice >= kU8Base) {
         if (u8_fits(choice - kU8Base)) return {kPlanU8, choice - kU8Base};
         // a borrowed stack the wide loads would overrun: the bucket's 16-bit-halves shape
@@ -51,8 +57,8 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
                      : -1;
     }
     if (choice >= 0) {
-        if (kShapes[choice].X == 2 && !pair_tile_fits(st->dev, st->alloc_bytes, st->bps, st->channels, k, max_pos))
-            choice = narrow_shape(choice);
+        if (kShapes[choice].X > 1 && !pair_tile_fits(st->dev, st->alloc_bytes, st->bps, st->channels, k, max_pos))
+            choice = st->channels >= 3 ? narrow_shape(choice) : -1;
         if (choice >= 0) p = {kPlanFast, choice};
     }
     return p;

@@ -11,16 +11,35 @@
 namespace cp {
 
 struct TileShape {
-    int G, F, X;
+    int G, F, X, FS;
 };
 
-// Shapes 10-14 put two pixels in each lane (16-bit stacks with 3 or 4 channels): one 12- or
-// 16-byte load per frame instead of one per pixel, which is what lets a wave's loads reach
-// HBM speed; narrow_shape gives the one-pixel shape with the same blocks.
-constexpr int kNumShapes = 15;
-constexpr TileShape kShapes[kNumShapes] = {{1, 16, 1}, {1, 32, 1}, {2, 16, 1}, {2, 32, 1}, {4, 16, 1},
-                                           {4, 32, 1}, {8, 16, 1}, {8, 32, 1}, {4, 64, 1}, {8, 64, 1},
-                                           {1, 16, 2}, {1, 32, 2}, {2, 32, 2}, {4, 32, 2}, {8, 32, 2}};
+// Shapes from 10 on put several pixels in each lane (16-bit stacks): one 8- to 16-byte load per
+// frame instead of one per pixel, which is what lets a wave's loads reach HBM speed; narrow_shape
+// gives the one-pixel shape with the same blocks (3 and 4 channels up to 256 frames).  X is 2
+// there, and 4 for one channel (wide_px).  Shapes from 17 on carry an FS-frame block of the
+// `--sample` positions.  Before the shapes for 1 and 2 channels, above 512 frames and with a
+// sample block, those stacks took the one-lane-per-pixel kernel, which reads every frame from
+// L2 once per value bit: 100 x 1937x1091 mono took 4.19 ms and takes 0.222 ms, 300 x 960x541 RGB
+// with 48 sample frames 4.42 and 0.440 ms.
+constexpr int kNumShapes = 21;
+constexpr TileShape kShapes[kNumShapes] = {
+    {1, 16, 1, 0}, {1, 32, 1, 0},  {2, 16, 1, 0},  {2, 32, 1, 0},  {4, 16, 1, 0},  {4, 32, 1, 0},  {8, 16, 1, 0},
+    {8, 32, 1, 0}, {4, 64, 1, 0},  {8, 64, 1, 0},  {1, 16, 2, 0},  {1, 32, 2, 0},  {2, 32, 2, 0},  {4, 32, 2, 0},
+    {8, 32, 2, 0}, {16, 32, 2, 0}, {32, 32, 2, 0}, {4, 32, 2, 16}, {8, 32, 2, 16}, {16, 32, 2, 8}, {32, 32, 2, 4}};
+constexpr int kSampleShape0 = 17;
+constexpr uint32_t kFastMaxFrames = 32 * 32, kFastMaxSample = 128;
+// Pixels per lane of the wide shapes, and of any shape, for a channel count.
+constexpr int wide_px(int channels) { return channels == 1 ? 4 : 2; }
+constexpr int shape_px(int shape, uint32_t channels) {
+    return kShapes[shape].X == 1 ? 1 : wide_px((int)channels);
+}
+// The smallest 16-bit shape with a sample block that holds n frames and s sample frames, or -1.
+inline int fast_sample_shape(uint32_t n, uint32_t s) {
+    for (int i = kSampleShape0; i < kNumShapes; ++i)
+        if ((uint32_t)(kShapes[i].G * kShapes[i].F) >= n && (uint32_t)(kShapes[i].G * kShapes[i].FS) >= s) return i;
+    return -1;
+}
 // Frame-count buckets of the tuned kernel choice.  A choice is a shape of this kernel
 // (kShapes index) or, from kU8Base on, a shape of the 8-bit packed-byte kernel (kU8Shapes
 // index + kU8Base, kernels_u8.h); each bucket has up to kMaxCand candidates, the first being
@@ -41,12 +60,12 @@ constexpr int kBucketCand[2][2][kNumBuckets][kMaxCand] = {
       {3, 4, kU8Base + 2, kU8Base + 16, kU8Base + 17}, {5, 6, kU8Base + 3, -1, -1},
       {7, 8, kU8Base + 4, -1, -1}, {9, kU8Base + 6, kU8Base + 5, -1, -1}, {kU8Base + 7, -1, -1, -1, -1},
       {kU8Base + 8, -1, -1, -1, -1}, {kU8Base + 9, -1, -1, -1, -1}}},
-    // 16-bit: 1-2 channels have no register-resident kernel; 3-4 channels up to 512 frames
+    // 16-bit: 1-2 channels and stacks over 512 frames have one shape each (untuned_shape)
     {{{-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1},
       {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1},
       {-1, -1, -1, -1, -1}},
      {{10, 0, -1, -1, -1}, {11, 1, -1, -1, -1}, {12, 3, -1, -1, -1}, {13, 5, -1, -1, -1}, {14, 7, -1, -1, -1},
-      {9, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}}}};
+      {15, 9, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}}}};
 // Default choice for relative thresholds where it differs from the bucket's first candidate
 // (-1: the first candidate): up to 64 frames of an 8-bit stack, one sort of a lane's bytes
 // gives the median and both quartiles at once, where the byte search runs three searches
@@ -62,73 +81,108 @@ inline int bucket_for(uint32_t n) {
     return -1;
 }
 
-inline int narrow_shape(int shape) {
-    for (int i = 0; i < kNumShapes; ++i)
-        if (kShapes[i].X == 1 && kShapes[i].G == kShapes[shape].G && kShapes[i].F == kShapes[shape].F) return i;
+// The shape of 16-bit stacks whose bucket has no candidates to choose from, or -1: the smallest
+// wide one that holds n frames.
+inline int untuned_shape(uint32_t bps, uint32_t n) {
+    for (int i = 10; bps == 2 && i < kSampleShape0; ++i)
+        if ((uint32_t)(kShapes[i].G * kShapes[i].F) >= n) return i;
     return -1;
 }
 
-template <int B, int C, int G, int F, int X>
+inline int narrow_shape(int shape) {
+    for (int i = 0; i < kNumShapes; ++i)
+        if (kShapes[i].X == 1 && kShapes[i].G == kShapes[shape].G && kShapes[i].F == kShapes[shape].F) return i;
+    return shape == 15 ? 9 : -1;  // 512 frames: 8 lanes of 64
+}
+
+template <bool ABS, int B, int C, int G, int F, int X, int FS = 0>
 inline void launch_fast_shape(const OutlierK& k, hipStream_t s) {
     constexpr int P = X * 256 / G;
     const uint32_t tiles_x = (k.out_w + P - 1) / P;
     dim3 grid(tiles_x * k.out_h), block(256);
-    if (k.th.absolute) hipLaunchKernelGGL((outlier_fast_kernel<B, C, G, F, X, true>), grid, block, 0, s, k, tiles_x);
-    else hipLaunchKernelGGL((outlier_fast_kernel<B, C, G, F, X, false>), grid, block, 0, s, k, tiles_x);
+    hipLaunchKernelGGL((outlier_fast_kernel<B, C, G, F, X, FS, ABS>), grid, block, 0, s, k, tiles_x);
 }
 
-template <int B, int C>
+// ABS: absolute thresholds (k.th.absolute).
+template <bool ABS, int B, int C>
 inline bool launch_fast_c(const OutlierK& k, int shape, hipStream_t s) {
-    switch (shape) {
-    case 0: launch_fast_shape<B, C, 1, 16, 1>(k, s); return true;
-    case 1: launch_fast_shape<B, C, 1, 32, 1>(k, s); return true;
-    case 2: launch_fast_shape<B, C, 2, 16, 1>(k, s); return true;
-    case 3: launch_fast_shape<B, C, 2, 32, 1>(k, s); return true;
-    case 4: launch_fast_shape<B, C, 4, 16, 1>(k, s); return true;
-    case 5: launch_fast_shape<B, C, 4, 32, 1>(k, s); return true;
-    case 6: launch_fast_shape<B, C, 8, 16, 1>(k, s); return true;
-    case 7: launch_fast_shape<B, C, 8, 32, 1>(k, s); return true;
-    case 8: launch_fast_shape<B, C, 4, 64, 1>(k, s); return true;
-    case 9: launch_fast_shape<B, C, 8, 64, 1>(k, s); return true;
-    default: break;
-    }
-    if constexpr (B == 2) {
+    if constexpr (C >= 3) {
         switch (shape) {
-        case 10: launch_fast_shape<B, C, 1, 16, 2>(k, s); return true;
-        case 11: launch_fast_shape<B, C, 1, 32, 2>(k, s); return true;
-        case 12: launch_fast_shape<B, C, 2, 32, 2>(k, s); return true;
-        case 13: launch_fast_shape<B, C, 4, 32, 2>(k, s); return true;
-        case 14: launch_fast_shape<B, C, 8, 32, 2>(k, s); return true;
+        case 0: launch_fast_shape<ABS, B, C, 1, 16, 1>(k, s); return true;
+        case 1: launch_fast_shape<ABS, B, C, 1, 32, 1>(k, s); return true;
+        case 3: launch_fast_shape<ABS, B, C, 2, 32, 1>(k, s); return true;
+        case 5: launch_fast_shape<ABS, B, C, 4, 32, 1>(k, s); return true;
+        case 7: launch_fast_shape<ABS, B, C, 8, 32, 1>(k, s); return true;
+        case 9: launch_fast_shape<ABS, B, C, 8, 64, 1>(k, s); return true;
+        default: break;
+        }
+    }
+    if constexpr (B == 1) {
+        switch (shape) {
+        case 2: launch_fast_shape<ABS, B, C, 2, 16, 1>(k, s); return true;
+        case 4: launch_fast_shape<ABS, B, C, 4, 16, 1>(k, s); return true;
+        case 6: launch_fast_shape<ABS, B, C, 8, 16, 1>(k, s); return true;
+        case 8: launch_fast_shape<ABS, B, C, 4, 64, 1>(k, s); return true;
+        default: break;
+        }
+    } else {
+        constexpr int X = wide_px(C);
+        switch (shape) {
+        case 10: launch_fast_shape<ABS, B, C, 1, 16, X>(k, s); return true;
+        case 11: launch_fast_shape<ABS, B, C, 1, 32, X>(k, s); return true;
+        case 12: launch_fast_shape<ABS, B, C, 2, 32, X>(k, s); return true;
+        case 13: launch_fast_shape<ABS, B, C, 4, 32, X>(k, s); return true;
+        case 14: launch_fast_shape<ABS, B, C, 8, 32, X>(k, s); return true;
+        case 15: launch_fast_shape<ABS, B, C, 16, 32, X>(k, s); return true;
+        case 16: launch_fast_shape<ABS, B, C, 32, 32, X>(k, s); return true;
+        case 17: launch_fast_shape<ABS, B, C, 4, 32, X, 16>(k, s); return true;
+        case 18: launch_fast_shape<ABS, B, C, 8, 32, X, 16>(k, s); return true;
+        case 19: launch_fast_shape<ABS, B, C, 16, 32, X, 8>(k, s); return true;
+        case 20: launch_fast_shape<ABS, B, C, 32, 32, X, 4>(k, s); return true;
         default: break;
         }
     }
     return false;
 }
 
-// Whether a two-pixel tile may run over this composite: the stack starts on an 8-byte
-// boundary (4-channel pairs are loaded as they lie, 3-channel pairs realigned from dword
-// boundaries), and every read stays inside the stack allocation: the last pixel pair of the
-// last row, at the largest frame offset, reads 16 bytes from its first sample.
+// Whether a tile of several pixels per lane may run over this composite: the stack starts on an
+// 8-byte boundary (pixels of an even channel count are loaded as they lie, the others realigned
+// from dword boundaries), and every read stays inside the stack allocation: the last lane of the
+// last row, at the largest frame offset, reads at most 16 bytes from its first sample.
 inline bool pair_tile_fits(const void* stack, uint64_t alloc_bytes, uint32_t bps, uint32_t channels,
                            const OutlierK& k, uint64_t max_pos) {
     if ((uintptr_t)stack & 7u) return false;
-    const uint64_t x_last = (uint64_t)((k.out_w - 1) / 2) * 2;
+    const uint64_t X = (uint64_t)wide_px((int)channels), x_last = (k.out_w - 1) / X * X;
     const uint64_t first = max_pos + ((uint64_t)(k.out_h - 1) * k.stack_w + x_last) * channels;
     return first * bps + 16 <= alloc_bytes;
 }
 
-// One translation unit per (sample bytes, channels): kernels_fast_b<B>_c<C>.hip.
+// One translation unit per (sample bytes, channels, and for 16 bits threshold kind):
+// kernels_fast_b<B>_c<C>[_abs|_rel].hip.
 bool launch_fast_b1_c3(const OutlierK& k, int shape, hipStream_t s);
 bool launch_fast_b1_c4(const OutlierK& k, int shape, hipStream_t s);
-bool launch_fast_b2_c3(const OutlierK& k, int shape, hipStream_t s);
-bool launch_fast_b2_c4(const OutlierK& k, int shape, hipStream_t s);
+bool launch_fast_b2_c1_abs(const OutlierK& k, int shape, hipStream_t s);
+bool launch_fast_b2_c1_rel(const OutlierK& k, int shape, hipStream_t s);
+bool launch_fast_b2_c2_abs(const OutlierK& k, int shape, hipStream_t s);
+bool launch_fast_b2_c2_rel(const OutlierK& k, int shape, hipStream_t s);
+bool launch_fast_b2_c3_abs(const OutlierK& k, int shape, hipStream_t s);
+bool launch_fast_b2_c3_rel(const OutlierK& k, int shape, hipStream_t s);
+bool launch_fast_b2_c4_abs(const OutlierK& k, int shape, hipStream_t s);
+bool launch_fast_b2_c4_rel(const OutlierK& k, int shape, hipStream_t s);
 
 inline bool launch_outlier_fast(uint32_t bps, uint32_t channels, const OutlierK& k, int shape, hipStream_t s) {
-    if (bps == 1 && channels == 3) return launch_fast_b1_c3(k, shape, s);
-    if (bps == 1 && channels == 4) return launch_fast_b1_c4(k, shape, s);
-    if (bps == 2 && channels == 3) return launch_fast_b2_c3(k, shape, s);
-    if (bps == 2 && channels == 4) return launch_fast_b2_c4(k, shape, s);
-    return false;
+    if (bps == 1) {
+        if (channels == 3) return launch_fast_b1_c3(k, shape, s);
+        return channels == 4 && launch_fast_b1_c4(k, shape, s);
+    }
+    const bool a = k.th.absolute != 0;
+    switch (channels) {
+    case 1: return a ? launch_fast_b2_c1_abs(k, shape, s) : launch_fast_b2_c1_rel(k, shape, s);
+    case 2: return a ? launch_fast_b2_c2_abs(k, shape, s) : launch_fast_b2_c2_rel(k, shape, s);
+    case 3: return a ? launch_fast_b2_c3_abs(k, shape, s) : launch_fast_b2_c3_rel(k, shape, s);
+    case 4: return a ? launch_fast_b2_c4_abs(k, shape, s) : launch_fast_b2_c4_rel(k, shape, s);
+    default: return false;
+    }
 }
 
 }  // namespace cp

@@ -3,6 +3,8 @@
 
 namespace cp {
 
-bool launch_fast_b1_c4(const OutlierK& k, int shape, hipStream_t s) { return launch_fast_c<1, 4>(k, shape, s); }
+bool launch_fast_b1_c4(const OutlierK& k, int shape, hipStream_t s) {
+    return k.th.absolute ? launch_fast_c<true, 1, 4>(k, shape, s) : launch_fast_c<false, 1, 4>(k, shape, s);
+}
 
 }  // namespace cp

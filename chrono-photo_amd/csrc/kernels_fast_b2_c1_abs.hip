@@ -1,0 +1,9 @@
+// kernels_fast_b2_c1_abs.hip -- register-resident outlier kernels, 16-bit, 1 channel(s), absolute
+// thresholds.
+#include "kernels_fast.h"
+
+namespace cp {
+
+bool launch_fast_b2_c1_abs(const OutlierK& k, int shape, hipStream_t s) { return launch_fast_c<true, 2, 1>(k, shape, s); }
+
+}  // namespace cp

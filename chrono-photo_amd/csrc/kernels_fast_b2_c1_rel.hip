@@ -1,0 +1,9 @@
+// kernels_fast_b2_c1_rel.hip -- register-resident outlier kernels, 16-bit, 1 channel(s), relative
+// thresholds.
+#include "kernels_fast.h"
+
+namespace cp {
+
+bool launch_fast_b2_c1_rel(const OutlierK& k, int shape, hipStream_t s) { return launch_fast_c<false, 2, 1>(k, shape, s); }
+
+}  // namespace cp

@@ -1,0 +1,9 @@
+// kernels_fast_b2_c3_abs.hip -- register-resident outlier kernels, 16-bit, 3 channel(s), absolute
+// thresholds.
+#include "kernels_fast.h"
+
+namespace cp {
+
+bool launch_fast_b2_c3_abs(const OutlierK& k, int shape, hipStream_t s) { return launch_fast_c<true, 2, 3>(k, shape, s); }
+
+}  // namespace cp
