@@ -33,9 +33,9 @@
 // candidate adds the workgroup's part to the frame's table.
 //
 // 256 x 4K RGB16, 5 anchors, r = 32, s = 12, per call: 0.78 ms with f64 products on the vector
-// units (bound by their issue), 0.245 ms with the matrix cores.  Staging, box sums and products
-// now take about a quarter each, one after another in a workgroup; three workgroups per CU
-// overlap them (16 window rows per workgroup: 12 or 13 measured alike, 22 leave two).
+// units (bound by their issue), 0.206 ms with the matrix cores (0.245 ms before the staging loads
+// were all in flight at once and the box sums of a candidate were added up once).  Staging, box
+// sums and products follow one another in a workgroup; three workgroups per CU overlap them.
 #pragma once
 #include "device_common.h"
 
@@ -90,16 +90,18 @@ __host__ __device__ inline ShakeLds shake_lds(int32_t rows, int32_t orows, int32
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
-// Eight samples from element e of a row that holds `len` (samples past it read as the centre),
-// centred, as bytes: hi and lo planes for 16-bit samples, lo alone for 8-bit ones.
+// Eight samples from element e of a row that holds `len` >= 8 or fewer samples, centred, as bytes
+// (hi and lo planes for 16-bit samples, lo alone for 8-bit ones); samples past len are zero.  A row
+// of eight samples or more is read without a branch: where the eight would pass its end, the
+// row's last eight are read and shifted.
 template <int B>
 __device__ __forceinline__ void load_centred8(const uint8_t* row, uint32_t e, uint32_t len, uint2& hi, uint2& lo) {
     typedef uint32_t words __attribute__((ext_vector_type(2 * B), aligned(B)));
     typedef const __attribute__((address_space(1))) words gwords;
+    const uint32_t at = min(e, len >= 8u ? len - 8u : 0u), past = min(e - at, 8u);  // samples to shift out
     uint32_t w[2 * B];
-    const uint8_t* at = row + e * B;
-    if (e + 8u <= len) {
-        const words v = *(gwords*)(uintptr_t)at;
+    if (len >= 8u) {  // the same for every lane
+        const words v = *(gwords*)(uintptr_t)(row + at * B);
 #pragma unroll
         for (int i = 0; i < 2 * B; ++i) w[i] = v[i];
     } else {
@@ -107,43 +109,56 @@ __device__ __forceinline__ void load_centred8(const uint8_t* row, uint32_t e, ui
         for (int i = 0; i < 2 * B; ++i) w[i] = 0x80808080u;
 #pragma unroll
         for (uint32_t i = 0; i < 8u; ++i) {
-            if (e + i >= len) break;
-            const uint32_t bit = 8u * B * i, v = load_sample<B>(at, i);
+            if (i >= len) break;
+            const uint32_t bit = 8u * B * i, v = load_sample<B>(row, i);
             w[bit / 32u] = (w[bit / 32u] & ~((B == 1 ? 0xFFu : 0xFFFFu) << (bit % 32u))) | (v << (bit % 32u));
         }
     }
+    auto shifted = [&](uint32_t a, uint32_t b) {  // the plane's eight bytes less `past`, zeros behind
+        const uint64_t v = (((uint64_t)(b ^ 0x80808080u) << 32) | (a ^ 0x80808080u));
+        const uint64_t r = past >= 8u ? 0ull : v >> (8u * past);
+        return uint2{(uint32_t)r, (uint32_t)(r >> 32)};
+    };
     if constexpr (B == 1) {
-        lo = uint2{w[0] ^ 0x80808080u, w[1] ^ 0x80808080u};
+        lo = shifted(w[0], w[1]);
         hi = uint2{0u, 0u};
     } else {
-        lo = uint2{__builtin_amdgcn_perm(w[1], w[0], 0x06040200u) ^ 0x80808080u,
-                   __builtin_amdgcn_perm(w[2 * B - 1], w[2 * B - 2], 0x06040200u) ^ 0x80808080u};
-        hi = uint2{__builtin_amdgcn_perm(w[1], w[0], 0x07050301u) ^ 0x80808080u,
-                   __builtin_amdgcn_perm(w[2 * B - 1], w[2 * B - 2], 0x07050301u) ^ 0x80808080u};
+        lo = shifted(__builtin_amdgcn_perm(w[1], w[0], 0x06040200u),
+                     __builtin_amdgcn_perm(w[2 * B - 1], w[2 * B - 2], 0x06040200u));
+        hi = shifted(__builtin_amdgcn_perm(w[1], w[0], 0x07050301u),
+                     __builtin_amdgcn_perm(w[2 * B - 1], w[2 * B - 2], 0x07050301u));
     }
 }
 
 // Stages `rows` rows of `len` samples (row y at base + y * stride bytes) as byte planes: plane p
 // of row y at dst + (p * rows + y) * pitch; samples past len are zero.  groups: eights of bytes
-// per row.  Sixteen lanes share a row, so that no lane divides and a row's loads are contiguous.
-template <int B>
+// per row.  Sixteen lanes share a row, so that no lane divides and a row's loads are contiguous;
+// the loads of R rows are all in flight before the first is used.
+template <int B, int R>
 __device__ __forceinline__ void stage_rows(const uint8_t* base, uint64_t stride, uint32_t rows, uint32_t len,
                                            uint32_t groups, uint8_t* dst, uint32_t pitch) {
-    constexpr int U = 4;  // groups in flight per lane
-    const uint32_t gx = threadIdx.x & 15u;
-    for (uint32_t y = threadIdx.x >> 4; y < rows; y += 16u) {
-        const uint8_t* row = base + y * stride;
-        uint8_t* out = dst + y * pitch;
-        for (uint32_t q0 = gx; q0 < groups; q0 += 16u * U) {
-            uint2 hi[U], lo[U];
+    constexpr uint32_t U = 3;  // groups of a row per lane and round
+    const uint32_t gx = threadIdx.x & 15u, y0 = threadIdx.x >> 4;
+    for (uint32_t yb = 0; yb < rows; yb += 16u * R) {
+        for (uint32_t qb = 0; qb < groups; qb += 16u * U) {
+            uint2 hi[R][U], lo[R][U];
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (q0 + 16u * u < groups) load_centred8<B>(row, (q0 + 16u * u) * 8u, len, hi[u], lo[u]);
+            for (uint32_t r = 0; r < R; ++r) {
+                const uint32_t y = min(yb + 16u * r + y0, rows - 1u);
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (q0 + 16u * u >= groups) break;
-                *reinterpret_cast<uint2*>(out + (q0 + 16u * u) * 8u) = lo[u];
-                if constexpr (B == 2) *reinterpret_cast<uint2*>(out + rows * pitch + (q0 + 16u * u) * 8u) = hi[u];
+                for (uint32_t u = 0; u < U; ++u)
+                    load_centred8<B>(base + y * stride, min(qb + 16u * u + gx, groups - 1u) * 8u, len, hi[r][u], lo[r][u]);
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < R; ++r) {
+                const uint32_t y = yb + 16u * r + y0;
+#pragma unroll
+                for (uint32_t u = 0; u < U; ++u) {
+                    const uint32_t q = qb + 16u * u + gx;
+                    if (y >= rows || q >= groups) continue;
+                    *reinterpret_cast<uint2*>(dst + y * pitch + q * 8u) = lo[r][u];
+                    if constexpr (B == 2) *reinterpret_cast<uint2*>(dst + (rows + y) * pitch + q * 8u) = hi[r][u];
+                }
             }
         }
     }
@@ -202,19 +217,18 @@ __global__ void __launch_bounds__(256) shake_ssd_kernel(ShakeK k) {
     const uint32_t srows = lay.srows, wsamples = (uint32_t)(size * C);
 
     // ---- stage: region rows oy0 + c0 .. of frame f, window rows c0 .. of frame 0 with zeros
-    // around them, the totals cleared
+    // around them
     {
         const uint64_t stride = (uint64_t)k.stack_w * C * B;
         const uint8_t* rbase =
             k.stack + (k.pos_off[f] + ((uint64_t)(cy - s - r + oy0 + c0) * k.stack_w + (cx - s - r + ox0)) * C) * B;
-        stage_rows<B>(rbase, stride, srows, lay.rlen, lay.slabs * 8u, region, lay.rpitch);
+        stage_rows<B, 3>(rbase, stride, srows, lay.rlen, lay.slabs * 8u, region, lay.rpitch);
         const uint8_t* wbase = k.stack + (k.pos_off[0] + ((uint64_t)(cy - r + c0) * k.stack_w + (cx - r)) * C) * B;
-        stage_rows<B>(wbase, stride, (uint32_t)crows, wsamples, (lay.wpitch - lay.wlead) / 8u, win + lay.wlead,
+        stage_rows<B, 1>(wbase, stride, (uint32_t)crows, wsamples, (lay.wpitch - lay.wlead) / 8u, win + lay.wlead,
                       lay.wpitch);
         const uint32_t lead = lay.wlead / 4u, wrows = (uint32_t)crows * PL;
         for (uint32_t i = tid; i < wrows * lead; i += 256u)
             *reinterpret_cast<uint32_t*>(win + (i / lead) * lay.wpitch + (i % lead) * 4u) = 0u;
-        for (uint32_t i = tid; i < (uint32_t)(orows * ocols); i += 256u) tot[i] = 0ull;
     }
     __syncthreads();
 
@@ -358,7 +372,14 @@ __global__ void __launch_bounds__(256) shake_ssd_kernel(ShakeK k) {
     }
     __syncthreads();  // the box sums are there
 
-    // ---- sum v^2 - 2 sum w * v of this wave's window rows
+    // ---- sum v^2 of every candidate, then each wave takes off twice its sum w * v
+    for (uint32_t i = tid; i < (uint32_t)(orows * ocols); i += 256u) {
+        long long v = 0;
+#pragma unroll 4
+        for (uint32_t dy = 0; dy < (uint32_t)crows; ++dy) v += rq[i + dy * (uint32_t)ocols];
+        tot[i] = (unsigned long long)v;
+    }
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -371,9 +392,7 @@ __global__ void __launch_bounds__(256) shake_ssd_kernel(ShakeK k) {
                 long long wv = acc[i][j][0][e];
                 if constexpr (B == 2)
                     wv += ((long long)acc[i][j][B == 2 ? 2 : 0][e] << 16) + ((long long)acc[i][j][B == 2 ? 1 : 0][e] << 8);
-                long long v = -2 * wv;
-                for (uint32_t dy = wave; dy < (uint32_t)crows; dy += 4u) v += rq[(oy + dy) * (uint32_t)ocols + ox];
-                atomicAdd(tot + oy * (uint32_t)ocols + ox, (unsigned long long)v);
+                atomicAdd(tot + oy * (uint32_t)ocols + ox, (unsigned long long)(-2 * wv));
             }
         }
     __syncthreads();
