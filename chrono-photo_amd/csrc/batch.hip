@@ -72,7 +72,7 @@ struct Tables {
 };
 
 void apply_fix(OutlierK& k, const TFix& f, uint8_t* base) {
-    k.pos_off = (const uint64_t*)(base + f.pos);
+    k.pos_off = PosK{(const uint64_t*)(base + f.pos), 0, 0};
     if (f.has_fade) k.fade.values = (const float*)(base + f.fade);
     if (f.has_mask) {
         k.sample_mask = (const uint32_t*)(base + f.mask);
@@ -334,7 +334,7 @@ extern "C" CP_API int cp_batch_create(cp_ctx* ctx, const cp_job* jobs, uint32_t 
             if (d.outlier) {
                 apply_fix(d.ko, d.fix, dbase);
             } else {
-                d.ks.pos_off = (const uint64_t*)(dbase + d.fix.pos);
+                d.ks.pos_off = PosK{(const uint64_t*)(dbase + d.fix.pos), 0, 0};
                 if (d.fix.has_fade) d.ks.fade.values = (const float*)(dbase + d.fix.fade);
             }
         }
@@ -506,7 +506,7 @@ extern "C" CP_API int cp_autotune(cp_ctx* ctx, uint32_t bps, uint32_t channels, 
                     const int c = step < nc ? step : 2 * nc - 1 - step;
                     OutlierK k{};
                     k.stack = st->dev;
-                    k.pos_off = d_pos;
+                    k.pos_off = PosK{d_pos, 0, 0};
                     k.n = kBucketMax[b];
                     k.n_sample = k.n;
                     k.stack_w = W;

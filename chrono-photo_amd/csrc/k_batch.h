@@ -34,7 +34,7 @@ __device__ __forceinline__ T* as_global(T* p) {
 __device__ __forceinline__ OutlierK global_args(const OutlierK& j) {
     OutlierK k = j;
     k.stack = as_global(k.stack);
-    k.pos_off = as_global(k.pos_off);
+    k.pos_off.table = as_global(k.pos_off.table);
     k.sample_mask = as_global(k.sample_mask);
     k.samp_off = as_global(k.samp_off);
     k.fade.values = as_global(k.fade.values);

@@ -593,17 +593,16 @@ struct TileShared {
 // Fills the frame-offset table of a tile (all 256 lanes take part): byte offsets of the
 // frame positions, the last one repeated up to `count` positions, at oidx(t) of a table
 // with blocks of F entries.
-template <int B, int F>
-__device__ __forceinline__ void load_offsets(uint64_t* off, uint32_t count, const uint64_t* __restrict__ pos_off,
-                                             uint32_t n) {
+template <int B, int F, typename Pos>
+__device__ __forceinline__ void load_offsets(uint64_t* off, uint32_t count, const Pos pos_off, uint32_t n) {
     for (uint32_t i = threadIdx.x; i < count; i += 256) off[i + 2u * (i / (uint32_t)F)] = pos_off[min(i, n - 1)] * B;
 }
 
 // load_offsets plus the realignment tables of a PAIR tile (TileShared::aoff, sft); r is the tile
 // row's first sample address modulo 4.
-template <int B, int F>
+template <int B, int F, typename Pos>
 __device__ __forceinline__ void load_offsets_pair(uint64_t* off, uint64_t* aoff, uint32_t* sft, uint32_t count,
-                                                  const uint64_t* __restrict__ pos_off, uint32_t n, uint32_t r) {
+                                                  const Pos pos_off, uint32_t n, uint32_t r) {
     for (uint32_t i = threadIdx.x; i < count; i += 256) {
         const uint32_t j = i + 2u * (i / (uint32_t)F);
         const uint64_t o = pos_off[min(i, n - 1)] * B;

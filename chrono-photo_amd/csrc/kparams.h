@@ -27,12 +27,24 @@ struct PixelStats {
     uint32_t pad;
 };
 
+// Element offsets of a composite's frame positions: a device table, or without one an even
+// spacing.  Whole stacks, video windows and frame ranges are evenly spaced, and their calls need
+// no copy of a table in front of the kernel.
+struct PosK {
+    const uint64_t* table;  // n offsets, or null
+    uint64_t first;
+    int64_t step;
+    __device__ __forceinline__ uint64_t operator[](uint32_t t) const {
+        return table ? table[t] : first + (uint64_t)(step * (int64_t)t);
+    }
+};
+
 // One composite over a device-resident stack.  Frame position t (0..n-1) reads sample
 // (x, y, ch) at element index pos_off[t] + (y * stack_w + x) * C + ch, where pos_off folds
 // the stack slot and the per-frame crop origin.
 struct OutlierK {
     const uint8_t* stack;
-    const uint64_t* pos_off;     // n element offsets
+    PosK pos_off;                // n element offsets
     const uint32_t* sample_mask; // bit t set: position t is in the median sample (null: all)
     const uint64_t* samp_off;    // element offsets of the n_sample sample positions (null: all)
     uint32_t n, n_sample;
@@ -53,7 +65,7 @@ struct OutlierK {
 
 struct SimpleK {
     const uint8_t* stack;
-    const uint64_t* pos_off;
+    PosK pos_off;
     uint32_t n;
     uint32_t stack_w;
     uint32_t out_w, out_h;

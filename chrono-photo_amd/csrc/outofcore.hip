@@ -229,7 +229,6 @@ CP_API int cp_simple_host(cp_ctx* ctx, const void* const* host_frames, uint32_t 
     if ((rc = plan_bands(ctx, host_frames, sel, width, C, B, g.n, g.out_h, band_bytes, &bp))) return rc;
     SimpleK k{};
     k.stack = bp.band.dev;
-    k.pos_off = (const uint64_t*)ctx->arena.put(bp.pos.data(), 8 * g.n, s);
     k.n = g.n;
     k.stack_w = width;
     k.out_w = g.out_w;
@@ -237,9 +236,10 @@ CP_API int cp_simple_host(cp_ctx* ctx, const void* const* host_frames, uint32_t 
     k.darker = darker ? 1 : 0;
     for (int i = 0; i < 4; ++i) k.w[i] = weights[i];
     k.fade = fade_to_device(ctx, fade, &rc);
-    if (rc || !k.pos_off) {
+    if (!rc) rc = stage_positions(ctx->arena, bp.pos, s, &k.pos_off);
+    if (rc) {
         free_bands(ctx, &bp, s);
-        return rc ? rc : fail(CP_ERR_HIP, "parameter staging failed");
+        return rc;
     }
     for (uint32_t r0 = 0; r0 < g.out_h; r0 += bp.bh) {
         const uint32_t rows = std::min(bp.bh, g.out_h - r0);

@@ -103,6 +103,9 @@ struct Geometry {
 };
 
 int resolve_frames(const cp_stack* st, const cp_frames* fr, Geometry* g);
+// The offsets `pos` as kernel arguments: their spacing where they are evenly spaced, else a copy
+// staged in `arena` on stream s.
+int stage_positions(ParamArena& arena, const std::vector<uint64_t>& pos, hipStream_t s, PosK* out);
 int check_weights(const float w[4]);
 
 // Validated arguments of one outlier composite; device pointers (pos_off, sample_mask,

@@ -202,8 +202,7 @@ int cp_server::start(Request* r, Slot& slot) {
         if ((rc = resolve_frames(st, &j.frames, &g))) return rc;
         SimpleK k{};
         k.stack = st->dev;
-        k.pos_off = (const uint64_t*)slot.arena.put(g.pos_off.data(), 8 * g.n, s);
-        if (!k.pos_off) return fail(CP_ERR_HIP, "server: parameter staging failed");
+        if ((rc = stage_positions(slot.arena, g.pos_off, s, &k.pos_off))) return rc;
         k.n = g.n;
         k.stack_w = st->width;
         k.out_w = g.out_w;
