@@ -560,6 +560,13 @@ __device__ __forceinline__ float frame_dist(const uint32_t (&s)[4], const float 
 // lanes (fixed g, consecutive p) and the writing lanes (the pixels of a wave x G blocks)
 // both spread over the banks; per-pixel values are stored channel-major.
 // PAIR: the tile reads 16-bit samples of several pixels with one dword-aligned load.
+// Whether a tile's waves finish their own pixels (finish_group): where a wave holds at most 16
+// pixels the finish by one lane per pixel of the whole tile would leave most of it idle.
+template <int G, int X>
+constexpr bool group_finishes() {
+    return (64 * X / G <= 8 || G >= 16) && X <= G;
+}
+
 template <int C, int G, int F, int X = 1, bool PAIR = (X == 2)>
 struct TileShared {
     static constexpr int P = X * 256 / G;      // pixels per tile
@@ -574,13 +581,16 @@ struct TileShared {
     uint64_t aoff[PAIR ? G * OS : 1];
     uint32_t sft[PAIR ? G * OS : 1];
     uint32_t mask[MW][NS];     // [w][slot]: outlier bits of frames g*F + 32w + b
-    float lmax[NS];            // [slot]: the largest outlier distance (valid when lmaxi != ~0)
-    uint32_t lmaxi[NS];        // [slot]: its first frame
-    float med[C][P];
-    float iqr_inv[C][P];
-    uint32_t s0[C][P];       // frame 0 samples
-    uint32_t sum_all[C][P];  // average modes
-    uint32_t sum_out[C][P];
+    // Tiles whose waves finish their own pixels (finish_group) keep nothing else here.
+    static constexpr bool OWN = group_finishes<G, X>();
+    static constexpr int PB = OWN ? 1 : P, NSB = OWN ? 1 : NS;
+    float lmax[NSB];           // [slot]: the largest outlier distance (valid when lmaxi != ~0)
+    uint32_t lmaxi[NSB];       // [slot]: its first frame
+    float med[C][PB];
+    float iqr_inv[C][PB];
+    uint32_t s0[C][PB];       // frame 0 samples
+    uint32_t sum_all[C][PB];  // average modes
+    uint32_t sum_out[C][PB];
     __device__ static __forceinline__ uint32_t oidx(uint32_t t) { return t + 2u * (t / (uint32_t)F); }
     __device__ static __forceinline__ uint32_t rot(uint32_t g) {
         return X == 1 ? 4u * g : (g & 1u) + (g >> 1) * (64u / (uint32_t)G);
@@ -1003,6 +1013,408 @@ __device__ __forceinline__ void finish_pixel(const OutlierK& k, uint32_t bx, uin
     }
 }
 
+// Inclusive prefix sum over the G lanes of a group (g: the lane's index in it).
+template <int G>
+__device__ __forceinline__ uint32_t grp_prefix(uint32_t v, uint32_t g) {
+    const uint32_t g16 = g & 15u;
+    auto up = [&](uint32_t moved, uint32_t d) { v += g16 >= d ? moved : 0u; };
+    if constexpr (G >= 2) up((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true), 1u);
+    if constexpr (G >= 4) up((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true), 2u);
+    if constexpr (G >= 8) up((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true), 4u);
+    if constexpr (G >= 16) up((uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true), 8u);
+    if constexpr (G >= 32) {
+        const uint32_t low = (uint32_t)__shfl((int)v, (int)((threadIdx.x & 32u) + 15u));
+        v += g >= 16u ? low : 0u;
+    }
+    return v;
+}
+
+// Orders a wave's own LDS accesses (they execute in order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The outlier lists of finish_group, one set per wave: kListCap outliers of each of the wave's PW
+// pixels at a time, entry (i, p) at i * PW + p.
+constexpr int kListCap = 16;
+template <int B, int C, int PW>
+struct WaveLists {
+    uint32_t num[PW];                // outliers of the pixel
+    float med[C][PW], wi[C][PW];
+    uint32_t frame[kListCap * PW];
+    float value[kListCap * PW];      // distance (average) or blend factor (forward, backward)
+    uint32_t smp[B][kListCap * PW];  // the samples, packed
+};
+
+// Finishes the X pixels of a lane group from the lanes' classifications: background and outlier
+// selection / blending (src/chrono.rs:290-493), output and statistics.  Counts, first and last
+// outliers and the largest distance are reduced over the group in registers; lane e < X of the
+// group then finishes pixel e.  The order-dependent modes list each pixel's outliers in frame
+// order (or reverse) in LDS, the whole wave fetches and weighs the listed samples, and the
+// finishing lane blends them from LDS.
+//
+// One lane per pixel of the tile after a barrier (finish_pixel) leaves a 32-lane-per-pixel tile
+// with 32 of its 256 lanes scanning 64 mask words and re-reading one sample after another, about
+// 0.7 ms of the 3.82 ms of 1200 x 1080p RGB8 (abs/0.05/0.2, extreme): 3.30 ms so; 400 frames 1.24
+// and 0.99 ms.  Tiles of 8 lanes and two 16-bit pixels finish faster the other way (256 x 4K RGB16
+// 3.11 against 3.21 ms): they have two waves of finishing lanes and few mask words.
+template <int B, int C, int G, int F, int X, bool ABS, int MW, bool PAIR>
+__device__ __forceinline__ void finish_group(const OutlierK& k, uint32_t bx, uint32_t y, uint32_t lane, uint32_t real,
+                                             const uint32_t (&m)[X][MW], const float (&lmax)[X],
+                                             const uint32_t (&lmaxi)[X], const uint32_t (&sum_all)[X][4],
+                                             const uint32_t (&sum_out)[X][4], const float (&med_all)[X][4],
+                                             const float (&iqr_all)[X][4], const uint32_t (&first)[X][C],
+                                             TileShared<C, G, F, X, PAIR>& sh,
+                                             WaveLists<B, C, 64 * X / G>& L) {
+    using TS = TileShared<C, G, F, X, PAIR>;
+    constexpr int PW = 64 * X / G;
+    constexpr uint32_t MAXV = B == 1 ? 255u : 65535u;
+    constexpr uint32_t NONE = 0xFFFFFFFFu;
+    const uint32_t N = k.n;
+    const uint32_t g = lane % G, t0 = g * F;
+    const uint32_t wl = lane & 63u, p = (wl / G) * X + g;  // the wave's pixel this lane finishes (g < X)
+    const uint32_t xw = bx * (uint32_t)TS::P + (lane >> 6) * (uint32_t)PW;
+    const bool want_iqr = !ABS || k.stats != nullptr;
+    const bool want_max = k.outlier == 2 || k.stats != nullptr;
+    const bool ordered = k.outlier >= 3;
+
+    // ---- summaries of each pixel; lane e keeps pixel e's
+    uint32_t num = 0, first_idx = NONE, last_idx = 0, first_non = NONE, max_index = 0;
+    float max_d = 0.0f, med[4] = {0, 0, 0, 0}, iqr_inv[4] = {0, 0, 0, 0}, wi[4], sg[4];
+    uint32_t s0[4] = {0, 0, 0, 0}, s_all[4] = {0, 0, 0, 0}, s_out[4] = {0, 0, 0, 0};
+    uint32_t num_e[X], ord_e[X];  // group-wide count; this lane's next place in its pixel's order
+#pragma unroll
+    for (int e = 0; e < X; ++e) {
+        uint32_t cnt = 0, fi = NONE, la = 0, fn = NONE;
+#pragma unroll
+        for (int w = 0; w < MW; ++w) {
+            const uint32_t mm = m[e][w];
+            cnt += __builtin_popcount(mm);
+            if (fi == NONE && mm) fi = t0 + 32u * w + __builtin_ctz(mm);
+            if (mm) la = t0 + 32u * w + 31u - __builtin_clz(mm);
+            const int32_t nw = (int32_t)real - 32 * w;
+            const uint32_t non = ~mm & (nw >= 32 ? 0xFFFFFFFFu : (nw <= 0 ? 0u : (1u << nw) - 1u));
+            if (fn == NONE && non) fn = t0 + 32u * w + __builtin_ctz(non);
+        }
+        num_e[e] = (uint32_t)grp_sum<G>((int32_t)cnt);
+        fi = grp_min_u32<G>(fi);
+        if (k.outlier == 1) la = grp_max_u32<G>(la);
+        if (k.background == 0) fn = grp_min_u32<G>(fn);
+        ord_e[e] = 0;
+        if (ordered) {
+            const uint32_t incl = grp_prefix<G>(cnt, g);
+            ord_e[e] = k.outlier == 5 ? num_e[e] - incl : incl - cnt;
+        }
+        uint32_t mxi = 0;
+        float mx = 0.0f;
+        if (want_max) {
+            const uint32_t bits = lmaxi[e] != NONE && lmax[e] > 0.0f ? __float_as_uint(lmax[e]) : 0u;
+            const uint32_t top = grp_max_u32<G>(bits);
+            const uint32_t at = grp_min_u32<G>(bits == top ? lmaxi[e] : NONE);
+            mx = __uint_as_float(top);
+            mxi = top != 0u ? at : 0u;
+        }
+        uint32_t f0[C];
+        if (k.background < 2) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) f0[c] = (uint32_t)__shfl((int)first[e][c], (int)(wl - g));
+        } else {
+#pragma unroll
+            for (int c = 0; c < C; ++c) f0[c] = 0;
+        }
+        if (g == (uint32_t)e) {
+            num = num_e[e];
+            first_idx = fi;
+            last_idx = la;
+            first_non = fn;
+            max_index = mxi;
+            max_d = mx;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                med[c] = med_all[e][c];
+                iqr_inv[c] = want_iqr ? iqr_all[e][c] : 0.0f;
+                s0[c] = f0[c];
+                s_all[c] = sum_all[e][c];
+                s_out[c] = sum_out[e][c];
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        wi[c] = ABS ? k.w[c] : k.w[c] * iqr_inv[c];
+        sg[c] = signum_f(k.w[c]);
+    }
+    if (first_idx == NONE) first_idx = 0;
+    const uint32_t x = xw + p;
+    const bool mine = g < (uint32_t)X && x < k.out_w;
+    const uint64_t row = (uint64_t)y * k.stack_w;
+    const uint64_t pix = (row + (mine ? x : 0u)) * C;
+    const uint64_t pix_id = (uint64_t)y * k.out_w + x;
+    auto sample = [&](uint32_t t, uint64_t at, uint32_t (&v)[4]) {
+#pragma unroll
+        for (int ch = 0; ch < C; ++ch) v[ch] = load_sample<B>(k.stack + sh.off[TS::oidx(t)], at + (uint64_t)ch);
+    };
+    // Sums of 16-bit samples over more than 256 frames can pass 2^24, where the reference's f32
+    // sums in frame order round: such a pixel's sums are taken again in that order.
+    const bool long_sums = B == 2 && N > 256u && (k.background == 2 || k.outlier == 3);
+    if (k.background == 1 || long_sums) {
+        // the random background's draw steps back through every outlier
+#pragma unroll
+        for (int e = 0; e < X; ++e)
+#pragma unroll
+            for (int w = 0; w < MW; ++w) sh.mask[w][TS::slot(g, (lane / G) * X + e)] = m[e][w];
+        wave_lds_order();
+    }
+
+    float f_all[4], f_out[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        f_all[c] = (float)s_all[c];
+        f_out[c] = (float)s_out[c];
+    }
+    if constexpr (B == 2) {
+        if (long_sums && mine) {
+            bool all_long = false, out_long = false;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                all_long = all_long || s_all[c] >= 1u << 24;
+                out_long = out_long || s_out[c] >= 1u << 24;
+            }
+            if (k.background == 2 && all_long) {
+                float acc[4] = {0, 0, 0, 0};
+#pragma unroll 8
+                for (uint32_t t = 0; t < N; ++t) {
+                    uint32_t v[4];
+                    sample(t, pix, v);
+#pragma unroll
+                    for (int c = 0; c < C; ++c) acc[c] += (float)v[c];
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c) f_all[c] = acc[c];
+            }
+            if (out_long) {
+                float acc[4] = {0, 0, 0, 0};
+                for (uint32_t q = 0; q < (uint32_t)G; ++q)
+#pragma unroll
+                    for (int w = 0; w < MW; ++w) {
+                        uint32_t mm = sh.mask[w][TS::slot(q, (lane / G) * X + g)];
+                        while (mm) {
+                            const uint32_t b = __builtin_ctz(mm);
+                            mm &= mm - 1u;
+                            uint32_t v[4];
+                            sample(q * F + 32u * w + b, pix, v);
+#pragma unroll
+                            for (int c = 0; c < C; ++c) acc[c] += (float)v[c];
+                        }
+                    }
+#pragma unroll
+                for (int c = 0; c < C; ++c) f_out[c] = acc[c];
+            }
+        }
+    }
+
+    // ---- background
+    uint32_t pixel[4] = {0, 0, 0, 0}, s[4] = {0, 0, 0, 0};
+    bool warning = false;
+    uint32_t bg_index = 0;
+    if (mine) {
+        if (k.background == 2) {
+            float mean[4];
+#pragma unroll
+            for (int c = 0; c < C; ++c) mean[c] = f_all[c] / (float)N;
+            if (num == 1) {
+                sample(first_idx, pix, s);
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                    pixel[c] = sat_cast(roundf(mean[c] * ((float)N / (float)(N - 1)) - (float)s[c] / (float)N), MAXV);
+            } else if (num > 1) {
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                    pixel[c] = sat_cast(roundf(mean[c] * ((float)N / (float)(N - num)) - f_out[c] / (float)N), MAXV);
+            } else {
+#pragma unroll
+                for (int c = 0; c < C; ++c) pixel[c] = sat_cast(roundf(mean[c]), MAXV);
+            }
+        } else if (k.background == 3) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) pixel[c] = sat_cast(roundf(med[c]), MAXV);
+        } else {
+            if (k.background == 0) {
+                if (num == N) warning = true;
+                else bg_index = num == 0 ? 0 : first_non;
+            } else if (num == 0 || num == N) {
+                bg_index = rng_range(k.seed, k.pix_base + pix_id, 0, N);
+                warning = num == N;
+            } else {
+                uint32_t pos = rng_range(k.seed, k.pix_base + pix_id, 0, N - num);
+                uint32_t j = num;
+                const uint32_t pt = (lane / G) * X + g;
+                for (int q = G - 1; q >= 0; --q) {
+#pragma unroll
+                    for (int w = MW - 1; w >= 0; --w) {
+                        uint32_t mm = sh.mask[w][TS::slot((uint32_t)q, pt)];
+                        while (mm) {
+                            const uint32_t b = 31 - __builtin_clz(mm);
+                            mm &= ~(1u << b);
+                            const uint32_t a = (uint32_t)q * F + (uint32_t)w * 32 + b;
+                            --j;
+                            const uint32_t bb = N - 1 - j;
+                            if (pos == a) pos = bb;
+                            else if (pos == bb) pos = a;
+                        }
+                    }
+                }
+                bg_index = pos;
+            }
+            if (bg_index == 0) {
+#pragma unroll
+                for (int c = 0; c < C; ++c) pixel[c] = s0[c];
+            } else {
+                sample(bg_index, pix, pixel);
+            }
+        }
+    }
+
+    // ---- outliers in frame order (average, forward) or reverse order (backward)
+    float pix_new[4] = {0, 0, 0, 0}, blend_inv = 1.0f, mean_dist = 0.0f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) pix_new[c] = (float)pixel[c];
+    if (ordered && __any(mine && num > 1)) {
+        const bool fwd = k.outlier != 5, blends = k.outlier != 3;
+        if (g < (uint32_t)X) {
+            L.num[p] = mine && num > 1 ? num : 0u;  // pixels with one outlier take no list
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                L.med[c][p] = med[c];
+                L.wi[c][p] = wi[c];
+            }
+        }
+        uint32_t cur[X][MW];
+#pragma unroll
+        for (int e = 0; e < X; ++e)
+#pragma unroll
+            for (int w = 0; w < MW; ++w) cur[e][w] = num_e[e] > 1 ? m[e][w] : 0u;
+        for (uint32_t base = 0; __any(mine && num > 1 && base < num); base += (uint32_t)kListCap) {
+            // list the outliers base .. base + kListCap - 1 of every pixel
+#pragma unroll
+            for (int e = 0; e < X; ++e) {
+                const uint32_t pe = (wl / G) * X + e;
+#pragma unroll
+                for (int ww = 0; ww < MW; ++ww) {
+                    const int w0 = ww, w1 = MW - 1 - ww;
+                    uint32_t mm = fwd ? cur[e][w0] : cur[e][w1];
+                    const uint32_t tw = t0 + 32u * (fwd ? w0 : w1);
+                    while (mm && ord_e[e] < base + (uint32_t)kListCap) {
+                        const uint32_t b = fwd ? __builtin_ctz(mm) : 31 - __builtin_clz(mm);
+                        mm &= ~(1u << b);
+                        L.frame[(ord_e[e] - base) * PW + pe] = tw + b;
+                        ++ord_e[e];
+                    }
+                    if (fwd) cur[e][w0] = mm;
+                    else cur[e][w1] = mm;
+                }
+            }
+            wave_lds_order();
+            // fetch and weigh them, one entry per lane
+            for (uint32_t i0 = 0; i0 < (uint32_t)(kListCap * PW); i0 += 64u) {
+                const uint32_t i = i0 + wl, pp = i % (uint32_t)PW;
+                const bool in = i < (uint32_t)(kListCap * PW) && base + i / (uint32_t)PW < L.num[pp];
+                if (!__any(in)) break;
+                if (in) {
+                    const uint32_t t = L.frame[i];
+                    float pm[4] = {0, 0, 0, 0}, pw[4] = {0, 0, 0, 0};
+#pragma unroll
+                    for (int c = 0; c < C; ++c) {
+                        pm[c] = L.med[c][pp];
+                        pw[c] = L.wi[c][pp];
+                    }
+                    uint32_t v[4] = {0, 0, 0, 0};
+                    sample(t, (row + xw + pp) * C, v);
+                    const float d = sqrtf(frame_dist<C>(v, pm, pw, sg));
+                    L.value[i] = blends ? fade_pick(k.fade, (int32_t)t, (int32_t)N, k.frame_offset) * blend_value(k.th, d)
+                                        : d;
+                    if (blends) {
+                        if constexpr (B == 1) {
+                            L.smp[0][i] = v[0] | (v[1] << 8) | (v[2] << 16) | (v[3] << 24);
+                        } else {
+                            L.smp[0][i] = v[0] | (v[1] << 16);
+                            L.smp[B - 1][i] = v[2] | (v[3] << 16);
+                        }
+                    }
+                }
+            }
+            wave_lds_order();
+            if (mine && num > 1 && base < num) {
+                const uint32_t n_here = min(num - base, (uint32_t)kListCap);
+                for (uint32_t i = 0; i < n_here; ++i) {
+                    const float val = L.value[i * PW + p];
+                    if (!blends) {
+                        mean_dist += val;
+                        continue;
+                    }
+                    const uint32_t q0 = L.smp[0][i * PW + p], q1 = B == 2 ? L.smp[B - 1][i * PW + p] : 0u;
+                    uint32_t v[4];
+                    if constexpr (B == 1) {
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) v[c] = (q0 >> (8 * c)) & 0xFFu;
+                    } else {
+                        v[0] = q0 & 0xFFFFu;
+                        v[1] = q0 >> 16;
+                        v[2] = q1 & 0xFFFFu;
+                        v[3] = q1 >> 16;
+                    }
+                    blend_into_f32<C>(pix_new, v, val);
+                    blend_inv *= 1.0f - val;
+                }
+            }
+            wave_lds_order();
+        }
+    }
+    if (!mine) return;
+    uint32_t blend_byte = 0;
+    if (num > 1 && (k.outlier == 4 || k.outlier == 5)) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) pixel[c] = sat_cast(roundf(pix_new[c]), MAXV);
+        blend_byte = sat_cast(roundf((1.0f - blend_inv) * 255.0f), 255u);
+    } else if (num > 0) {
+        uint32_t sel = 0;
+        float dist;
+        if (num > 1 && k.outlier == 3) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) s[c] = sat_cast(roundf(f_out[c] / (float)num), MAXV);
+            dist = mean_dist / (float)num;
+        } else {
+            sel = num == 1 || k.outlier == 0 ? first_idx : (k.outlier == 1 ? last_idx : max_index);
+            sample(sel, pix, s);
+            dist = sqrtf(frame_dist<C>(s, med, wi, sg));
+        }
+        const float fade = fade_pick(k.fade, (int32_t)sel, (int32_t)N, k.frame_offset);
+        const float blend = fade * blend_value(k.th, dist);
+        blend_into_px<C>(pixel, s, blend, MAXV);
+        blend_byte = sat_cast(roundf(blend * 255.0f), 255u);
+    }
+    const uint64_t o = pix_id * C;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        store_sample<B>(k.out_px, o + c, pixel[c]);
+        if (k.out_mask) k.out_mask[o + c] = c < 3 ? (uint8_t)blend_byte : (uint8_t)255;
+    }
+    if (warning && k.warnings) atomicAdd(k.warnings, 1ull);
+    if (k.stats) {
+        PixelStats st;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { st.median[i] = med[i]; st.iqr_inv[i] = iqr_inv[i]; }
+        st.num_outliers = num;
+        st.max_index = max_index;
+        st.max_dist_sq = max_d;
+        st.bg_index = bg_index;
+        st.warning = warning ? 1u : 0u;
+        st.pad = 0;
+        k.stats[pix_id] = st;
+    }
+}
+
 // The sample positions' offsets of a `--sample` tile, laid out as TileShared's tables.
 template <int G, int FS>
 struct SampleTable {
@@ -1257,6 +1669,18 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
                     sum_out[e][c] = (uint32_t)grp_sum<G>((int32_t)sum_out[e][c]);
                 }
             }
+        }
+
+        if constexpr (TS::OWN) {
+            __shared__ WaveLists<B, C, 64 * X / G> lists[4];
+            uint32_t first[X][C];
+#pragma unroll
+            for (int e = 0; e < X; ++e)
+#pragma unroll
+                for (int c = 0; c < C; ++c) first[e][c] = raw[e * C + c][0] & 0xFFFFu;
+            finish_group<B, C, G, F, X, ABS>(k, bx, y, lane, real, m, lmax, lmaxi, sum_all, sum_out, med, iqr_inv, first,
+                                             sh, lists[lane >> 6]);
+            return;
         }
 
         // ---- leave the lane's summaries and the pixels' statistics in LDS

@@ -642,6 +642,18 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
                 }
         }
 
+        if constexpr (TS::OWN) {
+            __shared__ WaveLists<1, C, 64 * X / G> lists[4];
+            uint32_t first[X][C];
+#pragma unroll
+            for (int e = 0; e < X; ++e)
+#pragma unroll
+                for (int c = 0; c < C; ++c) first[e][c] = yv[e * C + c][0] & 0xFFu;
+            finish_group<1, C, G, F, X, ABS>(k, bx, y, lane, real, m, lmax, lmaxi, sum_all, sum_out, med, iqr_inv, first,
+                                             sh, lists[lane >> 6]);
+            return;
+        }
+
         // ---- leave the lane's summaries and the pixels' statistics in LDS
         {
 #pragma unroll

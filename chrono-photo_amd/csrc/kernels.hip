@@ -20,8 +20,7 @@ static int launch_outlier_generic_b(const cp_stack* st, const OutlierK& k, hipSt
 }
 
 OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uint64_t max_pos, uint32_t flags) {
-    // The register-resident kernels need exact integer sums for the average modes
-    // (N * max sample < 2^24: always for 8-bit stacks).  8-bit composites take the packed-byte
+    // 8-bit composites take the packed-byte
     // kernel up to 1280 frames (and, with a `--sample` subset, up to 128 sample frames) or the
     // tuned choice between the two kernels; 16-bit ones the 16-bit kernel up to 1024 frames (and
     // up to 128 sample frames); the one-lane-per-pixel generic kernel takes the rest.  A
@@ -29,8 +28,7 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
     // the bucket's 16-bit-halves shape, or to the generic kernel where the bucket has none.
     OutlierPlan p;
     const bool sums = k.background == 2 || k.outlier == 3;
-    const bool exact_sums = st->bps == 1 || k.n <= 256;
-    if ((flags & CP_FLAG_FORCE_GENERIC) || (sums && !exact_sums)) return p;
+    if (flags & CP_FLAG_FORCE_GENERIC) return p;
     auto u8_fits = [&](int sh) {
         return u8_tile_fits(st->dev, st->alloc_bytes, st->channels, kU8Shapes[sh].X, k, max_pos);
     };
