@@ -226,13 +226,12 @@ int cp_ctx::ensure(cp::DeviceBuffer& b, size_t bytes) {
     return CP_OK;
 }
 
-int cp_ctx::choice_for(uint32_t bps, uint32_t channels, uint32_t n, bool absolute) const {
+int cp_ctx::choice_for(uint32_t bps, uint32_t channels, uint32_t n, bool absolute, bool sums) const {
     const int b = cp::bucket_for(n);
     if (b < 0 || bps < 1 || bps > 2 || channels < 1 || channels > 4) return -1;
     const int t = tuned[bps - 1][channels - 1][absolute ? 0 : 1][b];
     if (t >= 0) return t;
-    const int rel = absolute ? -1 : cp::kRelDefault[bps - 1][channels >= 3][b];
-    return rel >= 0 ? rel : cp::kBucketCand[bps - 1][channels >= 3][b][0];
+    return cp::default_choice(bps, channels, b, absolute, sums);
 }
 
 int cp_ctx::charge(uint64_t bytes) {

@@ -424,7 +424,7 @@ __global__ void autotune_fill_kernel(uint8_t* data, uint32_t bps, uint64_t n_ele
 static int32_t encode_choice(int choice, uint32_t channels) {
     if (choice >= kU8Base) {
         const U8Shape& u = kU8Shapes[choice - kU8Base];
-        return ((u.S ? 2 : 1) << 24) | (u.X << 16) | (u.G << 8) | u.F;
+        return ((u.S ? 2 : 1) << 24) | (u.load_px() << 16) | (u.G << 8) | u.F;
     }
     return (shape_px(choice, channels) << 16) | (kShapes[choice].G << 8) | kShapes[choice].F;
 }

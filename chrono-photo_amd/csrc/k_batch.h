@@ -57,8 +57,8 @@ __device__ __forceinline__ uint32_t group_job(const BatchJobK* __restrict__ jobs
 }
 
 // The packed-byte kernel over a group of jobs (k_outlier_u8.h).
-template <int C, int G, int F, int X, int FS, bool ABS, bool SORT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, SORT))))
+template <int C, int G, int F, int X, int FS, bool ABS, bool SORT, bool XCH>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, SORT, XCH))))
 outlier_u8_group_kernel(const BatchJobK* __restrict__ jobs, uint32_t njobs) {
     __shared__ TileShared<C, G, F, X, false> sh;
     __shared__ uint64_t soff[FS > 0 ? G * (FS + 2) : 1];
@@ -70,7 +70,7 @@ outlier_u8_group_kernel(const BatchJobK* __restrict__ jobs, uint32_t njobs) {
     if constexpr (FS > 0) load_offsets<1, FS>(soff, G * FS, k.samp_off, k.n_sample);
     __syncthreads();
     const uint32_t t = tile - J.tile0;
-    outlier_u8_tile<C, G, F, X, FS, ABS, SORT>(k, t % J.tiles_x, t / J.tiles_x, sh, soff, threadIdx.x, odist);
+    outlier_u8_tile<C, G, F, X, FS, ABS, SORT, XCH>(k, t % J.tiles_x, t / J.tiles_x, sh, soff, threadIdx.x, odist);
 }
 
 // The 16-bit-halves kernel over a group of jobs (k_outlier_fast.h).
@@ -87,10 +87,10 @@ outlier_fast_group_kernel(const BatchJobK* __restrict__ jobs, uint32_t njobs) {
     outlier_tile<B, C, G, F, X, 0, ABS>(k, t % J.tiles_x, y, sh, ssh, threadIdx.x);
 }
 
-template <int C, int G, int F, int X, int FS, bool SORT = false>
+template <int C, int G, int F, int X, int FS, bool SORT = false, bool XCH = false>
 constexpr const void* u8_group(bool absolute) {
-    return absolute ? (const void*)&outlier_u8_group_kernel<C, G, F, X, FS, true, SORT>
-                    : (const void*)&outlier_u8_group_kernel<C, G, F, X, FS, false, SORT>;
+    return absolute ? (const void*)&outlier_u8_group_kernel<C, G, F, X, FS, true, SORT, XCH>
+                    : (const void*)&outlier_u8_group_kernel<C, G, F, X, FS, false, SORT, XCH>;
 }
 
 // The group kernel of packed-byte shape `shape` (kU8Shapes index), or nullptr.
@@ -115,6 +115,16 @@ const void* u8_group_c(int shape, bool absolute) {
     case 15: return u8_group<C, 1, 32, 1, 0, true>(absolute);
     case 16: return u8_group<C, 1, 64, 1, 0, true>(absolute);
     case 17: return u8_group<C, 1, 64, 1, 0>(absolute);
+    case 18: return u8_group<C, 2, 64, 1, 0, false, true>(absolute);
+    case 19: return u8_group<C, 4, 64, 1, 0, false, true>(absolute);
+    case 20: return u8_group<C, 8, 64, 1, 0, false, true>(absolute);
+    case 21: return u8_group<C, 8, 96, 1, 0, false, true>(absolute);
+    case 22: return u8_group<C, 8, 128, 1, 0, false, true>(absolute);
+    case 23: return u8_group<C, 8, 160, 1, 0, false, true>(absolute);
+    case 24: return u8_group<C, 4, 64, 1, 32, false, true>(absolute);
+    case 25: return u8_group<C, 8, 64, 1, 16, false, true>(absolute);
+    case 26: return u8_group<C, 8, 160, 1, 16, false, true>(absolute);
+    case 27: return u8_group<C, 1, 64, 1, 0, false, true>(absolute);
     default: return nullptr;
     }
 }

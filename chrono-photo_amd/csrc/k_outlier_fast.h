@@ -391,13 +391,19 @@ __device__ __forceinline__ uint32_t min_greater(const uint32_t (&r)[NW], uint32_
     return grp_min_u32<G>(mm) + v + 1;
 }
 
+// Lanes of a group whose block of F frames is at least three quarters real, for `count` frames in
+// blocks of F (the same in every group).
+template <int G, int F>
+__device__ __forceinline__ uint32_t offering_lanes(uint32_t count) {
+    return min((count + (uint32_t)(F / 4)) / (uint32_t)F, (uint32_t)G);
+}
+
 // Location estimate of a 16-bit channel: median-of-3 "remedian" over the lane's samples
-// (both halves of each dword at once), then a trimmed mean over the lanes whose block is at
-// least three quarters real frames (real: this lane's; pads are the largest value and would
-// pull the mean up, and the search window with it).  It only places the search window;
-// exactness never depends on it.
+// (both halves of each dword at once), then a trimmed mean over the nv offering lanes (ok: this
+// lane is one; pads are the largest value and would pull the mean up, and the search window with
+// it).  It only places the search window; exactness never depends on it.
 template <int G, int NW>
-__device__ __forceinline__ uint32_t group_estimate(const uint32_t (&r)[NW], uint32_t real) {
+__device__ __forceinline__ uint32_t group_estimate(const uint32_t (&r)[NW], bool ok, uint32_t nv) {
     constexpr int L0 = NW / 3, L1 = L0 / 3, L2 = L1 / 3;
     static_assert(L0 >= 1, "estimate needs at least three dwords per lane");
     us2 a[L0];
@@ -413,11 +419,12 @@ __device__ __forceinline__ uint32_t group_estimate(const uint32_t (&r)[NW], uint
     }
     const uint32_t e = ((uint32_t)a[0].x + (uint32_t)a[0].y) >> 1;
     if constexpr (G == 1) return e;
-    const bool ok = real >= (uint32_t)(3 * NW / 2);
-    const uint32_t nv = (uint32_t)grp_sum<G>(ok ? 1 : 0);  // the same in every group
+    if (nv == (uint32_t)G) {
+        const uint32_t s = (uint32_t)grp_sum<G>((int32_t)e);
+        if constexpr (G == 2) return s >> 1;
+        return (s - grp_min_u32<G>(e) - grp_max_u32<G>(e)) / (uint32_t)(G > 2 ? G - 2 : 1);
+    }
     const uint32_t s = (uint32_t)grp_sum<G>((int32_t)(ok ? e : 0u));
-    if constexpr (G == 2) return nv == 2u ? s >> 1 : (nv == 1u ? s : grp_min_u32<G>(e));
-    if (nv == (uint32_t)G) return (s - grp_min_u32<G>(e) - grp_max_u32<G>(e)) / (uint32_t)(G - 2);
     if (nv >= 3u)
         return (uint32_t)((float)(s - grp_min_u32<G>(ok ? e : 0xFFFFu) - grp_max_u32<G>(ok ? e : 0u)) *
                           __builtin_amdgcn_rcpf((float)(nv - 2u)));
@@ -433,16 +440,16 @@ __device__ __forceinline__ uint32_t neighbour(const uint32_t (&r)[NW], uint32_t 
 // Values at ranks (r0, r1), r1 in {r0, r0 + 1}, of every channel.
 //  u8:  one byte level (WINDOW: in the 16-value window of byte_select_median, real = the lane
 //       block's frames below the stack's count); the neighbour is v0 or min{x > v0}.
-//  u16, WINDOW (medians of absolute thresholds): a 7-step byte search inside the window
-//       [lo, lo + 127] around the estimate; a channel's result is exact when it ends strictly
-//       inside (1..126).  Otherwise the rank lies below lo + 1 (result 0) or above lo + 126
-//       (result 127), and that channel searches the window next to it on that side, then, if
+//  u16, WINDOW (medians of absolute thresholds): a byte search inside a window of 128 or 256
+//       values around the estimate; a channel's result is exact when it ends strictly inside.
+//       Otherwise the rank lies at or below its first value or at or above its last, and that
+//       channel searches the window next to it on that side, then, if
 //       that one misses too, runs the exact two-level search.
 //  u16 otherwise: the exact two-level search.
 // Branches depend on group-uniform values only.
 template <int B, int G, int NW, int C, bool WINDOW>
 __device__ __forceinline__ void rank_pairs(const uint32_t (&raw)[C][NW], uint32_t r0, uint32_t r1, int32_t ntot,
-                                           uint32_t real, uint32_t (&v0)[C], uint32_t (&v1)[C]) {
+                                           uint32_t real, uint32_t count, uint32_t (&v0)[C], uint32_t (&v1)[C]) {
     constexpr int ND = NW / 2;
     constexpr uint32_t MAXV = B == 1 ? 255u : 65535u;
     const uint32_t kk[1] = {r0};
@@ -468,15 +475,21 @@ __device__ __forceinline__ void rank_pairs(const uint32_t (&raw)[C][NW], uint32_
             v1[c] = r1 == r0 ? v0[c] : neighbour<G, NW>(raw[c], v0[c], n1[c], r1);
         }
     } else if constexpr (WINDOW) {
-        constexpr uint32_t TOP = 127u, LO_MAX = 65535u - TOP;
+        // few lanes estimate the median more coarsely: a window of 256 values (one step more) up
+        // to 128 frames saves most of the second searches (100 x 1937x1091 mono: 219 us with 128
+        // values, 192 us so)
+        constexpr int WB = G <= 4 ? 8 : 7;
+        constexpr uint32_t TOP = (1u << WB) - 1u, LO_MAX = 65535u - TOP;
+        const uint32_t nv = offering_lanes<G, 2 * NW>(count);
+        const bool ok = real >= (uint32_t)(3 * NW / 2);
         uint32_t y[C][ND], lo[C];
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            const uint32_t est = group_estimate<G, NW>(raw[c], real);
-            lo[c] = min(est >= 63u ? est - 63u : 0u, LO_MAX);
+            const uint32_t est = group_estimate<G, NW>(raw[c], ok, nv);
+            lo[c] = min(est >= TOP / 2u ? est - TOP / 2u : 0u, LO_MAX);
             pack_window<NW, TOP>(raw[c], lo[c], y[c]);
         }
-        byte_select_multi<G, ND, C, 1, true, 7>(y, kk, ntot, sel, cle);
+        byte_select_multi<G, ND, C, 1, true, WB>(y, kk, ntot, sel, cle);
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             uint32_t ys = sel[c][0], base = lo[c];
@@ -485,7 +498,7 @@ __device__ __forceinline__ void rank_pairs(const uint32_t (&raw)[C][NW], uint32_
                 base = ys == 0u ? (base >= TOP - 1u ? base - (TOP - 1u) : 0u) : min(base + (TOP - 1u), LO_MAX);
                 uint32_t y1[1][ND], s1[1][1], c1[1][1];
                 pack_window<NW, TOP>(raw[c], base, y1[0]);
-                byte_select_multi<G, ND, 1, 1, true, 7>(y1, kk, ntot, s1, c1);
+                byte_select_multi<G, ND, 1, 1, true, WB>(y1, kk, ntot, s1, c1);
                 ys = s1[0][0];
                 le = c1[0][0];
             }
@@ -1461,6 +1474,7 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
         float med[X][4], iqr_inv[X][4];
         auto ranks = [&](auto nf_t, auto& blk, uint32_t blk_real) {
             constexpr int NF = decltype(nf_t)::value, NFW = NF / 2;  // frames per lane in the ranked block
+            const uint32_t blk_count = FS > 0 ? k.n_sample : N;
             constexpr bool WINDOW = ABS && (B == 1 || NFW >= 3);
             StaticFor<0, X>::run([&](auto e_t) {
                 constexpr int E = decltype(e_t)::value;
@@ -1469,10 +1483,10 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
                 if constexpr (!ABS && B == 1) {
                     rank_triples_u8<G, NFW, C>(re, plan, G * NF, blk_real, m0, m1, a0, a1, b0, b1);
                 } else {
-                    rank_pairs<B, G, NFW, C, WINDOW>(re, plan.m0, plan.m1, G * NF, blk_real, m0, m1);
+                    rank_pairs<B, G, NFW, C, WINDOW>(re, plan.m0, plan.m1, G * NF, blk_real, blk_count, m0, m1);
                     if constexpr (!ABS) {
-                        rank_pairs<B, G, NFW, C, false>(re, plan.a0, plan.a1, G * NF, blk_real, a0, a1);
-                        rank_pairs<B, G, NFW, C, false>(re, plan.b0, plan.b1, G * NF, blk_real, b0, b1);
+                        rank_pairs<B, G, NFW, C, false>(re, plan.a0, plan.a1, G * NF, blk_real, blk_count, a0, a1);
+                        rank_pairs<B, G, NFW, C, false>(re, plan.b0, plan.b1, G * NF, blk_real, blk_count, b0, b1);
                     }
                 }
 #pragma unroll
@@ -1638,12 +1652,14 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
                     else classify(e_t, F_{}, T_{}, F_{}, F_{});
                 }
             }
+            if (!full_tile) {
 #pragma unroll
-            for (int w = 0; w < MW; ++w) {
-                const int32_t nw = (int32_t)real - 32 * w;
-                m[E][w] &= nw >= 32 ? 0xFFFFFFFFu : (nw <= 0 ? 0u : (1u << nw) - 1u);
+                for (int w = 0; w < MW; ++w) {
+                    const int32_t nw = (int32_t)real - 32 * w;
+                    m[E][w] &= nw >= 32 ? 0xFFFFFFFFu : (nw <= 0 ? 0u : (1u << nw) - 1u);
+                }
+                if (real == 0u) lmaxi[E] = NONE;
             }
-            if (real == 0u) lmaxi[E] = NONE;
         });
         if (want_sums) {
             // all-frame sums through v_sad_u16 against zero, pads taken back out; the outliers'

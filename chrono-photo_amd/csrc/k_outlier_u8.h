@@ -101,26 +101,141 @@ __device__ __forceinline__ void load_quad_u8(const uint8_t* __restrict__ base, c
     }
 }
 
+// Pads of a lane block: the frames from `valid` on become 255.
+template <int XC, int ND>
+__device__ __forceinline__ void pad_block(uint32_t (&y)[XC][ND], uint32_t t0, uint32_t valid) {
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        const int32_t rem = (int32_t)valid - (int32_t)(t0 + 4 * i);  // valid frames in this dword
+        const uint32_t m = rem >= 4 ? 0u : (rem <= 0 ? 0xFFFFFFFFu : (0xFFFFFFFFu << (8 * rem)));
+#pragma unroll
+        for (int c = 0; c < XC; ++c) y[c][i] |= m;
+    }
+}
+
 // A lane's block of F frames (offsets off[0..F)) as packed bytes; frames from `valid` on are
 // set to 255 (valid is grid-uniform in the tile's block layout: N or the sample count).
 template <int C, int X, int F>
 __device__ __forceinline__ void load_block_u8(const uint8_t* __restrict__ base, const uint64_t* off,
                                               uint32_t (&y)[X * C][F / 4], uint32_t t0, uint32_t valid, bool pad) {
+    if constexpr (X == 1 && C <= 2) {
+        // One dword per frame: all of them are requested before the first is used.  Left to the
+        // scheduler a few are in flight at a time, which is best where the dwords are two per
+        // frame (3 channels: registers) and not here: 1080p mono, 64 frames 128 us with it,
+        // 74 us so.
+        uint32_t q[F];
 #pragma unroll
-    for (int i = 0; i < F / 4; ++i) {
-        uint32_t v[X * C];
-        load_quad_u8<C, X>(base, off + 4 * i, v);
-#pragma unroll
-        for (int c = 0; c < X * C; ++c) y[c][i] = v[c];
-    }
-    if (pad) {
+        for (int t = 0; t < F; ++t)
+            q[t] = *(const __attribute__((address_space(1))) uint32_t*)(((uintptr_t)base + off[t]) & ~(uintptr_t)3);
+        __builtin_amdgcn_sched_barrier(0);
+        // the shifts from the table again, not held in registers meanwhile
+        typedef const volatile __attribute__((address_space(3))) uint32_t lu32;
 #pragma unroll
         for (int i = 0; i < F / 4; ++i) {
-            const int32_t rem = (int32_t)valid - (int32_t)(t0 + 4 * i);  // valid frames in this dword
-            const uint32_t m = rem >= 4 ? 0u : (rem <= 0 ? 0xFFFFFFFFu : (0xFFFFFFFFu << (8 * rem)));
+            uint32_t in[4], out[4];
 #pragma unroll
-            for (int c = 0; c < X * C; ++c) y[c][i] |= m;
+            for (int f = 0; f < 4; ++f)
+                in[f] = __builtin_amdgcn_alignbyte(0u, q[4 * i + f], ((uint32_t)(uintptr_t)base + *(lu32*)(off + 4 * i + f)) & 3u);
+            transpose4(in, out);
+#pragma unroll
+            for (int c = 0; c < C; ++c) y[c][i] = out[c];
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < F / 4; ++i) {
+            uint32_t v[X * C];
+            load_quad_u8<C, X>(base, off + 4 * i, v);
+#pragma unroll
+            for (int c = 0; c < X * C; ++c) y[c][i] = v[c];
+        }
+    }
+    if (pad) pad_block<X * C, F / 4>(y, t0, valid);
+}
+
+// A workgroup barrier that orders LDS accesses alone: loads from memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Exchange tiles: 256 / G pixels, one pixel and F frames per lane, loaded in another layout.
+//
+// A lane with one pixel loads three useful bytes of eight, and with four pixels and few frames
+// each search step's reductions and bookkeeping, which are per lane, pixel and channel, outweigh
+// its counting (12 chains over 10 dwords of the 40-frame lanes).  So each lane loads a
+// quarter of the frames of four neighbouring pixels (one 16-byte load per frame; a wave covers
+// every pixel of the tile and 64 / (256 / G / 4) frame blocks), and the transposed dwords go
+// through LDS, four frames of every block at a time, to the lanes that own the pixels.
+// 1080p RGB8, abs/0.05/0.2, extreme, against the best tile without the exchange: 128 frames 257 ->
+// 221 us, 256 frames 588 -> 416 us, 512 frames 1006 -> 852 us, 1200 frames 3.30 -> 2.23 ms (loads
+// alone 2.07 ms at that pattern); rel/2.0/4.0, average: 518, 1043, 1971 us where 640, 1230 and
+// 2475 us were the best, and 700 x 720p rel/2.5/5.0 2.30 -> 1.19 ms.
+template <int C, int G, int BUFS>
+struct ExchangeLds {
+    static constexpr int NP = 256 / G;       // pixels
+    static constexpr int ROW = NP + (G > 1 ? 64 / G : 0);  // pads so that a wave's reads and writes spread over the banks
+    // [buffer][block of the lane's four * C + channel][lane of the pixel group * ROW + pixel]
+    uint32_t w[BUFS][4 * C][G * ROW];
+};
+// Tall lanes (many rounds) alternate between two buffers, one barrier a round; the others save the
+// LDS, which bounds how many of their workgroups a CU holds.
+constexpr int exchange_bufs(int F) { return F > 64 ? 2 : 1; }
+template <int C, int G, int F, int BUFS>
+__device__ __forceinline__ void load_block_exchange(const uint8_t* __restrict__ row, uint32_t x_tile, uint32_t out_w,
+                                                    const uint64_t* off, ExchangeLds<C, G, BUFS>& ex, uint32_t lane,
+                                                    uint32_t (&y)[C][F / 4]) {
+    using EX = ExchangeLds<C, G, BUFS>;
+    constexpr int NLG = EX::NP / 4;            // lanes across the tile
+    constexpr int FB = F / 4;                  // frames per loaded block
+    constexpr int NW = C, NQ = C == 4 ? 4 : C + 1;  // dwords of four pixels, dwords loaded
+    static_assert(F % 16 == 0, "whole quads per block");
+    typedef unsigned int vec __attribute__((ext_vector_type(NQ), aligned(4)));
+    const uint32_t lg = lane % (uint32_t)NLG, lb = lane / (uint32_t)NLG;
+    const uint32_t x = x_tile + lg * 4u;
+    const uintptr_t base = (uintptr_t)(row + (uint64_t)(x < out_w ? x : 0u) * C);
+    // frame lb * FB + j of the offset table, whose blocks of F entries are F + 2 apart
+    const uint64_t* o = off + lb * (uint32_t)FB + 2u * (lb / 4u);
+    vec raw[FB];
+#pragma unroll
+    for (int t = 0; t < FB; ++t)
+        raw[t] = *(const __attribute__((address_space(1))) vec*)((base + o[t]) & ~(uintptr_t)3);
+    __builtin_amdgcn_sched_barrier(0);
+    typedef const volatile __attribute__((address_space(3))) uint32_t lu32;  // the low halves, for the shifts
+    const uint32_t to = (lb / 4u) * (uint32_t)EX::ROW + lg * 4u;
+    const uint32_t from = (lane % (uint32_t)G) * (uint32_t)EX::ROW + lane / (uint32_t)G;
+#pragma unroll
+    for (int i = 0; i < FB / 4; ++i) {
+        uint32_t w[4][NW], v[4 * C];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            if constexpr (NQ > NW) {
+                const uint32_t sft = ((uint32_t)base + *(lu32*)(o + 4 * i + f)) & 3u;
+#pragma unroll
+                for (int h = 0; h < NW; ++h)
+                    w[f][h] = __builtin_amdgcn_alignbyte(raw[4 * i + f][h + 1], raw[4 * i + f][h], sft);
+            } else {
+#pragma unroll
+                for (int h = 0; h < NW; ++h) w[f][h] = raw[4 * i + f][h];
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < NW; ++h) {
+            const uint32_t in[4] = {w[0][h], w[1][h], w[2][h], w[3][h]};
+            uint32_t out[4];
+            transpose4(in, out);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) v[4 * h + b] = out[b];  // byte 4h + b of the 4 pixels x C
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            *reinterpret_cast<uint4*>(&ex.w[i % BUFS][(lb % 4u) * C + c][to]) = uint4{v[c], v[C + c], v[2 * C + c], v[3 * C + c]};
+        lds_barrier();
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int c = 0; c < C; ++c) y[c][b * (FB / 4) + i] = ex.w[i % BUFS][b * C + c][from];
+        if (BUFS == 1 || i == FB / 4 - 1) lds_barrier();  // the buffer is free again
     }
 }
 
@@ -321,11 +436,11 @@ constexpr bool keeps_odist() {
 // offsets (all positions) and soff the sample positions' offsets when FS > 0; every lane of
 // the workgroup calls this (it synchronises once).  lane: threadIdx.x.  odist: (kOdistSlots + 1)
 // * P floats of LDS when keeps_odist(), else unused.
-template <int C, int G, int F, int X, int FS, bool ABS, bool SORT = false>
+template <int C, int G, int F, int X, int FS, bool ABS, bool SORT = false, bool XCH = false>
 __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, uint32_t y,
                                                 TileShared<C, G, F, X, false>& sh, const uint64_t* soff, uint32_t lane,
                                                 float* odist = nullptr) {
-    static_assert(F % 8 == 0 && F <= 64 && G <= 32 && FS % 4 == 0 && (X == 1 || X == 4), "tile shape");
+    static_assert(F % 8 == 0 && (F <= 64 || (XCH && F <= 160)) && G <= 32 && FS % 4 == 0 && (X == 1 || X == 4), "tile shape");
     static_assert(!SORT || (G == 1 && X == 1 && FS == 0), "sorting-network ranks: one lane per pixel");
     using TS = TileShared<C, G, F, X, false>;
     constexpr int P = TS::P;
@@ -341,9 +456,21 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
         const uint32_t x0 = bx * P + pl * X;
         const uint64_t pix = ((uint64_t)y * k.stack_w + (x0 < k.out_w ? x0 : 0u)) * C;
         const uint8_t* base = k.stack + pix;
+        // the exchange buffer and, after the loads, the waves' outlier lists
+        using EX = ExchangeLds<C, XCH ? G : 8, exchange_bufs(F)>;
+        using WL = WaveLists<1, C, TS::OWN ? 64 * X / G : 1>;
+        constexpr size_t kExBytes = XCH ? sizeof(EX) : 16, kListBytes = TS::OWN ? 4 * sizeof(WL) : 16;
+        __shared__ __align__(16) uint8_t lds_mem[kExBytes > kListBytes ? kExBytes : kListBytes];
 
         uint32_t yv[XC][ND];
-        load_block_u8<C, X, F>(base, sh.off + g * TS::OS, yv, t0, N, N < (uint32_t)(G * F));
+        if constexpr (XCH) {
+            static_assert(X == 1, "exchange tiles hold one pixel per lane");
+            load_block_exchange<C, G, F>(k.stack + (uint64_t)y * k.stack_w * C, bx * P, k.out_w, sh.off,
+                                         *reinterpret_cast<EX*>(lds_mem), lane, yv);
+            if (N < (uint32_t)(G * F)) pad_block<XC, ND>(yv, t0, N);
+        } else {
+            load_block_u8<C, X, F>(base, sh.off + g * TS::OS, yv, t0, N, N < (uint32_t)(G * F));
+        }
 
         // ---- medians / inverse IQR over the sample set, every pixel and channel
         const RankPlan plan = rank_plan_core(k.n_sample, ABS);
@@ -353,8 +480,14 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
         } else if constexpr (FS > 0) {
             constexpr int NDS = FS / 4;
             uint32_t ys[XC][NDS];
-            load_block_u8<C, X, FS>(base, soff + g * (FS + 2), ys, g * FS, k.n_sample,
-                                    k.n_sample < (uint32_t)(G * FS));
+            if constexpr (XCH) {
+                load_block_exchange<C, G, FS>(k.stack + (uint64_t)y * k.stack_w * C, bx * P, k.out_w, soff,
+                                              *reinterpret_cast<EX*>(lds_mem), lane, ys);
+                if (k.n_sample < (uint32_t)(G * FS)) pad_block<XC, NDS>(ys, g * FS, k.n_sample);
+            } else {
+                load_block_u8<C, X, FS>(base, soff + g * (FS + 2), ys, g * FS, k.n_sample,
+                                        k.n_sample < (uint32_t)(G * FS));
+            }
             const uint32_t ts = g * FS, ns = k.n_sample;
             ranks_u8<G, NDS, XC, ABS>(ys, plan, G * FS, ns > ts ? min(ns - ts, (uint32_t)FS) : 0u, m0, m1, a0, a1,
                                       b0, b1);
@@ -471,6 +604,7 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
             // an outlier is 4 d >= 4 tsq, i.e. dot products' sum >= et
             const int32_t t4 = (int32_t)ceilf(fminf(4.0f * tsq, 8388608.0f));
             const int32_t et = (t4 - s4 + 3) >> 2;
+            constexpr int JB = F <= 64 ? 6 : 8, JM = (1 << JB) - 1;  // dev < 2^22: the frame goes below it
             int32_t best = (int32_t)0x80000000;
 #pragma unroll
             for (int i = ND - 1; i >= 0; --i) {
@@ -509,7 +643,7 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
                         __builtin_amdgcn_udot4(px[f], v1, __builtin_amdgcn_udot4(px[f], v0, 0u, false), false);
                     const uint32_t dev = xx - xm;  // as a signed number: >= 0 for an outlier
                     m[E][j >> 5] = __builtin_amdgcn_alignbit(m[E][j >> 5], dev, 31);
-                    if constexpr (MAXT) best = max(best, (int32_t)((dev << 6) | (uint32_t)(63 - j)));
+                    if constexpr (MAXT) best = max(best, (int32_t)((dev << JB) | (uint32_t)(JM - j)));
                     if constexpr (OD) {
                         const int32_t d4 = 4 * ((int32_t)dev + et) + s4;
                         put_dist((int32_t)dev >= 0 && (uint32_t)j < real, 0.25f * (float)d4);
@@ -520,8 +654,8 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
             for (int w = 0; w < MW; ++w) m[E][w] = ~m[E][w];  // the sign bits mark the others
             if constexpr (MAXT) {
                 if (best >= 0) {
-                    lmax[E] = 0.25f * (float)(4 * ((best >> 6) + et) + s4);
-                    lmaxi[E] = t0 + 63u - ((uint32_t)best & 63u);
+                    lmax[E] = 0.25f * (float)(4 * ((best >> JB) + et) + s4);
+                    lmaxi[E] = t0 + (uint32_t)JM - ((uint32_t)best & (uint32_t)JM);
                 }
             }
         };
@@ -643,14 +777,13 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
         }
 
         if constexpr (TS::OWN) {
-            __shared__ WaveLists<1, C, 64 * X / G> lists[4];
             uint32_t first[X][C];
 #pragma unroll
             for (int e = 0; e < X; ++e)
 #pragma unroll
                 for (int c = 0; c < C; ++c) first[e][c] = yv[e * C + c][0] & 0xFFu;
             finish_group<1, C, G, F, X, ABS>(k, bx, y, lane, real, m, lmax, lmaxi, sum_all, sum_out, med, iqr_inv, first,
-                                             sh, lists[lane >> 6]);
+                                             sh, reinterpret_cast<WL*>(lds_mem)[lane >> 6]);
             return;
         }
 
@@ -693,13 +826,17 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
 
 // VGPRs the frame blocks take, for the occupancy hint: X * C * (F + FS) / 4, plus F for the
 // pairs a sorting network works on, plus working registers.
-constexpr int waves_hint_u8(int C, int F, int X, int FS, bool sort) {
+constexpr int waves_hint_u8(int C, int F, int X, int FS, bool sort, bool xch = false) {
+    if (xch) {
+        const int v = 512 / (C * (F + FS) / 4 + 48);
+        return v < 2 ? 2 : (v > 6 ? 6 : v);
+    }
     const int w = 448 / (X * C * (F + FS) / 4 + (sort ? F : 0) + 64);
     return w < 1 ? 1 : (w > 8 ? 8 : w);
 }
 
-template <int C, int G, int F, int X, int FS, bool ABS, bool SORT = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, SORT))))
+template <int C, int G, int F, int X, int FS, bool ABS, bool SORT = false, bool XCH = false>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, SORT, XCH))))
 outlier_u8_kernel(OutlierK k, uint32_t tiles_x) {
     __shared__ TileShared<C, G, F, X, false> sh;
     __shared__ uint64_t soff[FS > 0 ? G * (FS + 2) : 1];
@@ -708,7 +845,7 @@ outlier_u8_kernel(OutlierK k, uint32_t tiles_x) {
     load_offsets<1, F>(sh.off, G * F, k.pos_off, k.n);
     if constexpr (FS > 0) load_offsets<1, FS>(soff, G * FS, k.samp_off, k.n_sample);
     __syncthreads();
-    outlier_u8_tile<C, G, F, X, FS, ABS, SORT>(k, tile % tiles_x, tile / tiles_x, sh, soff, threadIdx.x, odist);
+    outlier_u8_tile<C, G, F, X, FS, ABS, SORT, XCH>(k, tile % tiles_x, tile / tiles_x, sh, soff, threadIdx.x, odist);
 }
 
 // Whether the packed-byte tiles may run over this composite: every lane's load of a frame

@@ -30,11 +30,12 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
     const bool sums = k.background == 2 || k.outlier == 3;
     if (flags & CP_FLAG_FORCE_GENERIC) return p;
     auto u8_fits = [&](int sh) {
-        return u8_tile_fits(st->dev, st->alloc_bytes, st->channels, kU8Shapes[sh].X, k, max_pos);
+        return u8_tile_fits(st->dev, st->alloc_bytes, st->channels, kU8Shapes[sh].load_px(), k, max_pos);
     };
     if (k.sample_mask != nullptr) {
         if (st->bps == 1 && k.n <= kU8MaxFrames && k.n_sample <= kU8MaxSample && k.samp_off) {
-            const int sh = u8_shape_for(k.n, true, k.n_sample);
+            int sh = u8_shape_for(k.n, true, k.n_sample, true);
+            if (sh < 0 || !u8_fits(sh)) sh = u8_shape_for(k.n, true, k.n_sample, false);
             if (sh >= 0 && u8_fits(sh)) p = {kPlanU8, sh};
         }
         if (st->bps == 2 && k.n <= kFastMaxFrames && k.n_sample <= kFastMaxSample && k.samp_off) {
@@ -44,15 +45,17 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
         }
         return p;
     }
-    int choice = ctx->choice_for(st->bps, st->channels, k.n, k.th.absolute != 0);
+    int choice = ctx->choice_for(st->bps, st->channels, k.n, k.th.absolute != 0, sums);
     if (choice < 0) choice = untuned_shape(st->bps, k.n);
     if (choice >= kU8Base) {
         if (u8_fits(choice - kU8Base)) return {kPlanU8, choice - kU8Base};
         // a borrowed stack the wide loads would overrun: the bucket's 16-bit-halves shape
         const int b = bucket_for(k.n);
-        choice = b >= 0 && kBucketCand[st->bps - 1][st->channels >= 3][b][0] < kU8Base
-                     ? kBucketCand[st->bps - 1][st->channels >= 3][b][0]
-                     : -1;
+        choice = -1;
+        for (int c = kMaxCand - 1; b >= 0 && c >= 0; --c) {
+            const int cand = kBucketCand[st->bps - 1][st->channels >= 3][b][c];
+            if (cand >= 0 && cand < kU8Base) choice = cand;  // the first of them
+        }
     }
     if (choice >= 0) {
         if (kShapes[choice].X > 1 && !pair_tile_fits(st->dev, st->alloc_bytes, st->bps, st->channels, k, max_pos))

@@ -47,33 +47,67 @@ inline int fast_sample_shape(uint32_t n, uint32_t s) {
 constexpr int kNumBuckets = 9;
 constexpr uint32_t kBucketMax[kNumBuckets] = {16, 32, 64, 128, 256, 512, 768, 1024, 1280};
 constexpr int kU8Base = 64;
-constexpr int kMaxCand = 5;
+constexpr int kMaxCand = 6;
 // [sample bytes - 1][channels >= 3][bucket][candidate]; -1: none
 constexpr int kBucketCand[2][2][kNumBuckets][kMaxCand] = {
     // 8-bit, 1-2 channels: the packed-byte kernel only
-    {{{kU8Base + 0, kU8Base + 14, -1, -1, -1}, {kU8Base + 1, kU8Base + 15, -1, -1, -1},
-      {kU8Base + 2, kU8Base + 16, kU8Base + 17, -1, -1}, {kU8Base + 3, -1, -1, -1, -1},
-      {kU8Base + 4, -1, -1, -1, -1}, {kU8Base + 6, kU8Base + 5, -1, -1, -1}, {kU8Base + 7, -1, -1, -1, -1},
-      {kU8Base + 8, -1, -1, -1, -1}, {kU8Base + 9, -1, -1, -1, -1}},
+    {{{kU8Base + 0, kU8Base + 14, -1, -1, -1, -1},
+      {kU8Base + 1, kU8Base + 15, -1, -1, -1, -1},
+      {kU8Base + 2, kU8Base + 16, kU8Base + 17, kU8Base + 27, -1, -1},
+      {kU8Base + 3, kU8Base + 18, -1, -1, -1, -1},
+      {kU8Base + 4, kU8Base + 19, -1, -1, -1, -1},
+      {kU8Base + 6, kU8Base + 5, kU8Base + 20, -1, -1, -1},
+      {kU8Base + 7, kU8Base + 21, -1, -1, -1, -1},
+      {kU8Base + 8, kU8Base + 22, -1, -1, -1, -1},
+      {kU8Base + 9, kU8Base + 23, -1, -1, -1, -1}},
      // 8-bit, 3-4 channels
-     {{0, kU8Base + 0, kU8Base + 14, -1, -1}, {1, 2, kU8Base + 1, kU8Base + 15, -1},
-      {3, 4, kU8Base + 2, kU8Base + 16, kU8Base + 17}, {5, 6, kU8Base + 3, -1, -1},
-      {7, 8, kU8Base + 4, -1, -1}, {9, kU8Base + 6, kU8Base + 5, -1, -1}, {kU8Base + 7, -1, -1, -1, -1},
-      {kU8Base + 8, -1, -1, -1, -1}, {kU8Base + 9, -1, -1, -1, -1}}},
+     {{0, kU8Base + 0, kU8Base + 14, -1, -1, -1},
+      {1, 2, kU8Base + 1, kU8Base + 15, -1, -1},
+      {3, 4, kU8Base + 2, kU8Base + 16, kU8Base + 17, kU8Base + 27},
+      {5, 6, kU8Base + 3, kU8Base + 18, -1, -1},
+      {7, 8, kU8Base + 4, kU8Base + 19, -1, -1},
+      {9, kU8Base + 6, kU8Base + 5, kU8Base + 20, -1, -1},
+      {kU8Base + 7, kU8Base + 21, -1, -1, -1, -1},
+      {kU8Base + 8, kU8Base + 22, -1, -1, -1, -1},
+      {kU8Base + 9, kU8Base + 23, -1, -1, -1, -1}}},
     // 16-bit: 1-2 channels and stacks over 512 frames have one shape each (untuned_shape)
-    {{{-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1},
-      {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1},
-      {-1, -1, -1, -1, -1}},
-     {{10, 0, -1, -1, -1}, {11, 1, -1, -1, -1}, {12, 3, -1, -1, -1}, {13, 5, -1, -1, -1}, {14, 7, -1, -1, -1},
-      {15, 9, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}}}};
-// Default choice for relative thresholds where it differs from the bucket's first candidate
-// (-1: the first candidate): up to 64 frames of an 8-bit stack, one sort of a lane's bytes
-// gives the median and both quartiles at once, where the byte search runs three searches
-// (64 × 1080p RGB8, rel/2/4: 0.339 ms against 0.428 ms for the best byte-search tile).
-constexpr int kRelDefault[2][2][kNumBuckets] = {
-    {{kU8Base + 14, kU8Base + 15, kU8Base + 16, -1, -1, -1, -1, -1, -1},
-     {kU8Base + 14, kU8Base + 15, kU8Base + 16, -1, -1, -1, -1, -1, -1}},
-    {{-1, -1, -1, -1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1, -1, -1, -1}}};
+    {{{-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1},
+      {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1},
+      {-1, -1, -1, -1, -1, -1}},
+     {{10, 0, -1, -1, -1, -1}, {11, 1, -1, -1, -1, -1}, {12, 3, -1, -1, -1, -1}, {13, 5, -1, -1, -1, -1}, {14, 7, -1, -1, -1, -1},
+      {15, 9, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1}}}};
+// The choice of a context that was not tuned, [sample bytes - 1][channels >= 3][relative][bucket]
+// (-1: none): the fastest of the bucket's candidates over 1080p stacks of the scene generator at
+// the bucket's limit and at counts inside it, extreme, forward and average modes.  us at 1080p
+// RGB, the choice and the first candidate, abs/0.05/0.2 extreme, then rel/2.0/4.0 average:
+//   8 bits    16: 40, 49 and 76, 110      32: 68, 81 and 140, 174    64: 132, 180 and 272, 368
+//            128: 221, 349 and 518, 703  256: 416, 901 and 1043, 1502  512: 852, 2004 and 1971, 4042
+//            768: 1190, 1958 and 3002, 6050   1024: 1603, 2401 and 4324, 7801
+//   16 bits   16: 108, 121 and 186, 202   64: 233, 268 and 611, 751
+//            128: 437 and 1267, 1497     256: 790 and 2606, 2983
+// (two 16-bit pixels per lane load better, one leaves more waves: the three full searches of
+// relative thresholds and the few loads of short stacks want the waves).
+constexpr int kDefault[2][2][2][kNumBuckets] = {
+    {{{kU8Base + 0, kU8Base + 1, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+       kU8Base + 23},
+      {kU8Base + 14, kU8Base + 15, kU8Base + 17, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+       kU8Base + 23}},
+     {{kU8Base + 14, kU8Base + 1, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+       kU8Base + 23},
+      {kU8Base + 14, kU8Base + 15, kU8Base + 16, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+       kU8Base + 23}}},
+    {{{-1, -1, -1, -1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1, -1, -1, -1}},
+     {{0, 1, 3, 13, 14, 15, -1, -1, -1}, {0, 1, 3, 5, 7, 9, -1, -1, -1}}}};
+// The same with the mode: sums: an average mode.
+inline int default_choice(uint32_t bps, uint32_t channels, int bucket, bool absolute, bool sums) {
+    const int c = kDefault[bps - 1][channels >= 3][absolute ? 0 : 1][bucket];
+    // 64 frames, relative: the network of one lane ranks fastest, but its tile keeps the average
+    // modes' distances in LDS, and four channels take two networks; the byte search then wins
+    if (c == kU8Base + 16 && (channels == 4 || sums)) return kU8Base + 17;
+    // four channels fill the exchanged dwords, and one lane's loads are already 4 bytes each
+    if (c == kU8Base + 27 && channels == 4) return kU8Base + 17;
+    return c;
+}
 
 inline int bucket_for(uint32_t n) {
     for (int b = 0; b < kNumBuckets; ++b)

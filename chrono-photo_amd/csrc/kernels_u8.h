@@ -10,40 +10,46 @@ namespace cp {
 
 struct U8Shape {
     int G, F, X, FS, S;  // S: ranks from a sorting network (G = 1) instead of the byte search
+    int L = 0;           // exchange tile (X = 1): L pixels per load
+    constexpr int load_px() const { return L ? L : X; }
 };
 
 // One pixel per lane for short stacks; four pixels per lane (one 16-byte load per frame)
 // for tall ones; `--sample` shapes carry an FS-frame block of the sample positions; shapes
 // 14-16 rank one lane's whole pixel with a sorting network; shape 17 holds a 64-frame pixel
 // in one lane for the byte search (a candidate only: u8_shape_for meets shape 2 first).
-constexpr int kNumU8Shapes = 18;
+// Shapes from 18 on are exchange tiles, 24-26 with a block of up to 128 sample frames.
+constexpr int kNumU8Shapes = 28;
 constexpr U8Shape kU8Shapes[kNumU8Shapes] = {
-    {1, 16, 1, 0, 0},  {1, 32, 1, 0, 0},  {2, 32, 1, 0, 0},  {4, 32, 1, 0, 0}, {8, 32, 1, 0, 0},
-    {16, 32, 1, 0, 0}, {16, 32, 4, 0, 0}, {32, 24, 4, 0, 0}, {32, 32, 4, 0, 0}, {32, 40, 4, 0, 0},
-    {4, 32, 1, 8, 0},  {8, 32, 1, 8, 0},  {16, 32, 4, 8, 0}, {32, 40, 4, 4, 0}, {1, 16, 1, 0, 1},
-    {1, 32, 1, 0, 1},  {1, 64, 1, 0, 1},  {1, 64, 1, 0, 0}};
+    {1, 16, 1, 0, 0},      {1, 32, 1, 0, 0},      {2, 32, 1, 0, 0},      {4, 32, 1, 0, 0},     {8, 32, 1, 0, 0},
+    {16, 32, 1, 0, 0},     {16, 32, 4, 0, 0},     {32, 24, 4, 0, 0},     {32, 32, 4, 0, 0},    {32, 40, 4, 0, 0},
+    {4, 32, 1, 8, 0},      {8, 32, 1, 8, 0},      {16, 32, 4, 8, 0},     {32, 40, 4, 4, 0},    {1, 16, 1, 0, 1},
+    {1, 32, 1, 0, 1},      {1, 64, 1, 0, 1},      {1, 64, 1, 0, 0},      {2, 64, 1, 0, 0, 4},  {4, 64, 1, 0, 0, 4},
+    {8, 64, 1, 0, 0, 4},   {8, 96, 1, 0, 0, 4},   {8, 128, 1, 0, 0, 4},  {8, 160, 1, 0, 0, 4}, {4, 64, 1, 32, 0, 4},
+    {8, 64, 1, 16, 0, 4},  {8, 160, 1, 16, 0, 4}, {1, 64, 1, 0, 0, 4}};
 constexpr uint32_t kU8MaxFrames = 32 * 40;
 constexpr uint32_t kU8MaxSample = 128;
 
-// The smallest shape that holds n frames (and s sample frames when sampled), or -1.
-inline int u8_shape_for(uint32_t n, bool sampled, uint32_t s) {
+// The smallest shape that holds n frames (and s sample frames when sampled), or -1; exchange:
+// among the exchange tiles or among the others.
+inline int u8_shape_for(uint32_t n, bool sampled, uint32_t s, bool exchange) {
     for (int i = 0; i < kNumU8Shapes; ++i) {
         const U8Shape& sh = kU8Shapes[i];
-        if ((sh.FS > 0) != sampled || sh.S) continue;
+        if ((sh.FS > 0) != sampled || sh.S || (sh.L > 0) != exchange) continue;
         if ((uint32_t)(sh.G * sh.F) >= n && (!sampled || (uint32_t)(sh.G * sh.FS) >= s)) return i;
     }
     return -1;
 }
 
-template <int C, int G, int F, int X, int FS, bool SORT = false>
+template <int C, int G, int F, int X, int FS, bool SORT = false, bool XCH = false>
 inline void launch_u8_shape(const OutlierK& k, hipStream_t s) {
     constexpr int P = X * 256 / G;
     const uint32_t tiles_x = (k.out_w + P - 1) / P;
     dim3 grid(tiles_x * k.out_h), block(256);
     if (k.th.absolute)
-        hipLaunchKernelGGL((outlier_u8_kernel<C, G, F, X, FS, true, SORT>), grid, block, 0, s, k, tiles_x);
+        hipLaunchKernelGGL((outlier_u8_kernel<C, G, F, X, FS, true, SORT, XCH>), grid, block, 0, s, k, tiles_x);
     else
-        hipLaunchKernelGGL((outlier_u8_kernel<C, G, F, X, FS, false, SORT>), grid, block, 0, s, k, tiles_x);
+        hipLaunchKernelGGL((outlier_u8_kernel<C, G, F, X, FS, false, SORT, XCH>), grid, block, 0, s, k, tiles_x);
 }
 
 template <int C>
@@ -67,6 +73,16 @@ inline bool launch_u8_c(const OutlierK& k, int shape, hipStream_t s) {
     case 15: launch_u8_shape<C, 1, 32, 1, 0, true>(k, s); return true;
     case 16: launch_u8_shape<C, 1, 64, 1, 0, true>(k, s); return true;
     case 17: launch_u8_shape<C, 1, 64, 1, 0>(k, s); return true;
+    case 18: launch_u8_shape<C, 2, 64, 1, 0, false, true>(k, s); return true;
+    case 19: launch_u8_shape<C, 4, 64, 1, 0, false, true>(k, s); return true;
+    case 20: launch_u8_shape<C, 8, 64, 1, 0, false, true>(k, s); return true;
+    case 21: launch_u8_shape<C, 8, 96, 1, 0, false, true>(k, s); return true;
+    case 22: launch_u8_shape<C, 8, 128, 1, 0, false, true>(k, s); return true;
+    case 23: launch_u8_shape<C, 8, 160, 1, 0, false, true>(k, s); return true;
+    case 24: launch_u8_shape<C, 4, 64, 1, 32, false, true>(k, s); return true;
+    case 25: launch_u8_shape<C, 8, 64, 1, 16, false, true>(k, s); return true;
+    case 26: launch_u8_shape<C, 8, 160, 1, 16, false, true>(k, s); return true;
+    case 27: launch_u8_shape<C, 1, 64, 1, 0, false, true>(k, s); return true;
     default: return false;
     }
 }

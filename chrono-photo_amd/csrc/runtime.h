@@ -71,8 +71,9 @@ struct cp_ctx {
     // autotuned kernel choice per (sample bytes - 1, channels - 1, threshold kind (0: absolute,
     // 1: relative), frame bucket); -1 = default
     int8_t tuned[2][4][2][16];
-    // the register-resident kernel choice for n frames (kernels_fast.h), or -1: none
-    int choice_for(uint32_t bps, uint32_t channels, uint32_t n, bool absolute) const;
+    // the register-resident kernel choice for n frames (kernels_fast.h), or -1: none; sums: an
+    // average mode
+    int choice_for(uint32_t bps, uint32_t channels, uint32_t n, bool absolute, bool sums) const;
     int ensure(cp::DeviceBuffer& b, size_t bytes);
     int charge(uint64_t bytes);
     void uncharge(uint64_t bytes) { used = used >= bytes ? used - bytes : 0; }
