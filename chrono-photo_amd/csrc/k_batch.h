@@ -58,7 +58,7 @@ __device__ __forceinline__ uint32_t group_job(const BatchJobK* __restrict__ jobs
 
 // The packed-byte kernel over a group of jobs (k_outlier_u8.h).
 template <int C, int G, int F, int X, int FS, bool ABS, bool SORT, bool XCH>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, SORT, XCH))))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, ABS, SORT, XCH))))
 outlier_u8_group_kernel(const BatchJobK* __restrict__ jobs, uint32_t njobs) {
     __shared__ TileShared<C, G, F, X, false> sh;
     __shared__ uint64_t soff[FS > 0 ? G * (FS + 2) : 1];

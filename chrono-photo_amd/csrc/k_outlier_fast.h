@@ -12,17 +12,23 @@
 //
 // Order statistics (src/chrono.rs:228-255 sorts each weighted channel; any exact selection
 // gives the same values).  The r-th smallest value is found MSB-first: keep the largest
-// prefix v with #{y < v} <= r.  Counts come from the sum of absolute differences:
-//     sum_y |y - v| - sum_y |y - (v-1)| = 2 #{y < v} - n
-// so one search step costs two v_sad_u8 per four byte-samples plus a G-lane DPP reduction.
-// All channels (and, for relative thresholds, all ranks) advance through the same step, so
-// the independent chains interleave.  8-bit stacks need one 8-step level, which their medians
-// first try as 4 steps in a 16-value window around an estimate and their quartiles as 4 steps
-// next to the median; 16-bit stacks run one level on the high bytes and one on the low bytes
-// clamped into the winning high-byte bucket (values below map to 0, above to 255, which
-// leaves every count #{y < v}, v in [1,255], exact); their medians first try a single 7-step
-// level inside a 128-wide window around an estimate, then the window next to it, and fall
-// back to the two levels when the result lands on a window's edge.  The neighbour order statistic of an even-sized median
+// prefix v with #{y < v} <= r.  There are two ways to count.
+//  - The sum of absolute differences over packed bytes (byte_select_multi):
+//        sum_y |y - v| - sum_y |y - (v-1)| = 2 #{y < v} - n
+//    so one search step costs two v_sad_u8 per four samples plus a G-lane DPP reduction.
+//  - Bit planes (plane_select): once 32 samples' bits are transposed, a step costs one AND and
+//    one bit count per 32 samples.  The transposition pays where it serves several ranks or
+//    many steps.
+// The chains of different channels and ranks are independent and interleave.  8-bit medians try
+// 4 SAD steps in a 16-value window around an estimate before the 8 of the whole range, and the
+// ranks of relative thresholds come from bit planes (plane_ranks; other blocks search 4 steps
+// next to the median).  16-bit medians search 7 or 8 bit planes inside a window around an
+// estimate, then in the window next to it, and fall back to two SAD levels, one on the high
+// bytes and one on the low bytes clamped into the winning high-byte bucket (values below map
+// to 0, above to 255, which leaves every count #{y < v}, v in [1,255], exact), when the result
+// lands on a window's edge; the ranks of relative thresholds come from all 16 bit planes.
+// Blocks of fewer than 32 frames per lane use SAD counts throughout.  The neighbour order
+// statistic of an even-sized median
 // (and the quartile interpolation partners) is either the same value (when #{x <= v} covers
 // it) or min{x > v} (packed u16 min).  Frames beyond N are padded with the maximum sample
 // value, which never changes the ranks below N.
@@ -147,6 +153,112 @@ __device__ __forceinline__ void byte_select_multi(const uint32_t (&y)[C][ND], co
 // A byte in all four bytes (a multiply by 0x01010101 takes four times as long to issue).
 __device__ __forceinline__ uint32_t splat4(uint32_t v) { return __builtin_amdgcn_perm(v, v, 0u); }
 
+// Bits of x where m is set, of y elsewhere (v_bfi_b32).
+__device__ __forceinline__ uint32_t bit_merge(uint32_t m, uint32_t x, uint32_t y) { return (x & m) | (y & ~m); }
+
+// One stage of a bit transposition over dwords: of each pair (a[i], a[i + S]) the first keeps the
+// fields' low S bits of both, the second their high S bits (m: the low S bits of every field of
+// 2 S bits).
+template <int S, int NB>
+__device__ __forceinline__ void plane_stage(uint32_t (&a)[NB], uint32_t m) {
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        if (i & S) continue;
+        const uint32_t x = a[i], z = a[i + S];
+        if constexpr (S == 8) {  // whole bytes: one v_perm_b32 each
+            a[i] = __builtin_amdgcn_perm(z, x, 0x06020400u);
+            a[i + S] = __builtin_amdgcn_perm(z, x, 0x07030501u);
+        } else {
+            a[i] = bit_merge(m, x, z << S);
+            a[i + S] = bit_merge(~m, z, x >> S);
+        }
+    }
+}
+
+// NB dwords of 32 / NB-byte-packed samples (NB = 8: four bytes, NB = 16: two 16-bit halves) become
+// NB bit planes: plane b holds bit b of all 32 samples, every plane with the same sample order.
+template <int NB>
+__device__ __forceinline__ void to_planes(uint32_t (&a)[NB]) {
+    static_assert(NB == 8 || NB == 16, "planes of 8- or 16-bit samples");
+    if constexpr (NB == 16) plane_stage<8, NB>(a, 0x00FF00FFu);
+    plane_stage<4, NB>(a, 0x0F0F0F0Fu);
+    plane_stage<2, NB>(a, 0x33333333u);
+    plane_stage<1, NB>(a, 0x55555555u);
+}
+
+// For every channel c and rank k[r] the k[r]-th smallest (out) of the group's samples and, with
+// CNT, #{samples <= it} (cnt), read from bit planes.  The search keeps the set of the samples
+// that agree with the value's bits so far as one bit per sample and descends a bit per step: the
+// samples of the set with a 1 here number n1 over the group; with q = the samples of the set
+// ranked above the value, n1 > q means that the value has a 1 too, otherwise those n1 lie above
+// it and the set keeps the others.  A step is an AND and a bit count per 32 samples and the
+// G-lane sum, against 16 SAD instructions of byte_select_multi; the transposition (48 instructions
+// per 32 bytes, 112 per 32 16-bit samples) pays when it serves several ranks or at least 7 steps.
+// Bound by VALU issue like the tiles around it, SAD counts and planes: 256 x 3840x2160 RGB16
+// abs/0.05/0.2, forward, 2691 and 2424 VALU instructions per wave, 3184 and 2946 us (the loads
+// alone are 1.9 ms at a streaming read's rate); 64 x 1080p RGB8 rel/2.0/4.0, average, 275 and
+// 241 us; 256 x 1080p RGB16 rel/2.0/4.0, average, 2592 and 1628 us.
+template <int G, int NG, int NB, int C, int R, bool CNT, int BITS = NB>
+__device__ __forceinline__ void plane_select(const uint32_t (&pl)[C][NG][NB], const uint32_t (&k)[R], int32_t ntot,
+                                             uint32_t (&out)[C][R], uint32_t (&cnt)[C][R]) {
+    uint32_t set[C][R][NG];
+    int32_t q[C][R];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            out[c][r] = 0;
+            q[c][r] = ntot - 1 - (int32_t)k[r];
+#pragma unroll
+            for (int g = 0; g < NG; ++g) set[c][r][g] = ~0u;
+        }
+#pragma unroll
+    for (int bit = BITS - 1; bit >= 0; --bit) {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                uint32_t ones[NG];
+                int32_t n = 0;
+#pragma unroll
+                for (int g = 0; g < NG; ++g) {
+                    ones[g] = set[c][r][g] & pl[c][g][bit];
+                    n += __popc(ones[g]);
+                }
+                n = grp_sum<G>(n);
+                const bool one = n > q[c][r];
+                q[c][r] = one ? q[c][r] : q[c][r] - n;
+                out[c][r] = (out[c][r] << 1) | (one ? 1u : 0u);
+#pragma unroll
+                for (int g = 0; g < NG; ++g) set[c][r][g] = one ? ones[g] : set[c][r][g] ^ ones[g];
+            }
+    }
+    if constexpr (CNT) {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int r = 0; r < R; ++r)  // q0 - q samples lie above the value
+                cnt[c][r] = (uint32_t)((int32_t)k[r] + 1 + q[c][r]);
+    }
+}
+
+// plane_select over packed bytes (below 2^BITS).
+template <int G, int ND, int C, int R, bool CNT, int BITS = 8>
+__device__ __forceinline__ void byte_planes_select(const uint32_t (&y)[C][ND], const uint32_t (&k)[R], int32_t ntot,
+                                                   uint32_t (&out)[C][R], uint32_t (&cnt)[C][R]) {
+    static_assert(ND % 8 == 0, "whole planes");
+    uint32_t pl[C][ND / 8][8];
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int g = 0; g < ND / 8; ++g) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pl[c][g][i] = y[c][8 * g + i];
+            to_planes<8>(pl[c][g]);
+        }
+    plane_select<G, ND / 8, 8, C, R, CNT, BITS>(pl, k, ntot, out, cnt);
+}
+
 // 2 #{y < v} - ntot over the group's packed bytes, for v in 1..255.
 template <int G, int ND>
 __device__ __forceinline__ int32_t count_below(const uint32_t (&y)[ND], uint32_t v) {
@@ -255,9 +367,16 @@ __device__ __forceinline__ void byte_select_median(const uint32_t (&y)[C][ND], u
     }
 }
 
+// Whether the three ranks of relative thresholds come from bit planes, for ND dwords of packed
+// bytes per lane and channel: whole planes, and few enough of them to stay in registers beside
+// the block (planes of 128 and more frames would take 32 registers to the windows' none, and
+// those of 96 frames do not fit beside four channels).
+constexpr bool plane_ranks(int ND, int C) { return ND % 8 == 0 && (ND <= 16 || (ND == 24 && C <= 3)); }
+
 // The median and both quartiles of every channel's packed bytes: k = {median rank, first quartile
-// rank <= it, third quartile rank >= it}; out and cnt as byte_select_multi's.  The median comes
-// from byte_select_median (real as there).  The first quartile then lies in the 16 values
+// rank <= it, third quartile rank >= it}; out and cnt as byte_select_multi's.  Blocks that
+// plane_ranks admits descend their bit planes.  For the others the median comes from
+// byte_select_median (real as there).  The first quartile then lies in the 16 values
 // [lo, lo + 15] with lo = max(0, median - 15) when #{y < lo} <= its rank (the window's top,
 // median + 1 or above, already counts more than the median's rank), and the third quartile in
 // [lo, lo + 15] with lo = min(median, 240) when #{y < lo + 16} > its rank (#{y < lo} is at most
@@ -267,6 +386,22 @@ __device__ __forceinline__ void byte_select_median(const uint32_t (&y)[C][ND], u
 template <int G, int ND, int C>
 __device__ __forceinline__ void byte_select_quartiles(const uint32_t (&y)[C][ND], const uint32_t (&k)[3], int32_t ntot,
                                                       uint32_t real, uint32_t (&out)[C][3], uint32_t (&cnt)[C][3]) {
+    if constexpr (plane_ranks(ND, C)) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {  // one channel's planes at a time
+            uint32_t one[1][ND], o[1][3], n[1][3];
+#pragma unroll
+            for (int i = 0; i < ND; ++i) one[0][i] = y[c][i];
+            byte_planes_select<G, ND, 1, 3, true>(one, k, ntot, o, n);
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                out[c][r] = o[0][r];
+                cnt[c][r] = n[0][r];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+    }
     {
         uint32_t o[C], n[C];
         byte_select_median<G, ND, C>(y, k[0], ntot, real, o, n);
@@ -443,8 +578,8 @@ __device__ __forceinline__ uint32_t neighbour(const uint32_t (&r)[NW], uint32_t 
 //  u16, WINDOW (medians of absolute thresholds): a byte search inside a window of 128 or 256
 //       values around the estimate; a channel's result is exact when it ends strictly inside.
 //       Otherwise the rank lies at or below its first value or at or above its last, and that
-//       channel searches the window next to it on that side, then, if
-//       that one misses too, runs the exact two-level search.
+//       channel searches the window next to it on that side, then, if that one misses too, runs
+//       the exact two-level search.
 //  u16 otherwise: the exact two-level search.
 // Branches depend on group-uniform values only.
 template <int B, int G, int NW, int C, bool WINDOW>
@@ -489,7 +624,8 @@ __device__ __forceinline__ void rank_pairs(const uint32_t (&raw)[C][NW], uint32_
             lo[c] = min(est >= TOP / 2u ? est - TOP / 2u : 0u, LO_MAX);
             pack_window<NW, TOP>(raw[c], lo[c], y[c]);
         }
-        byte_select_multi<G, ND, C, 1, true, WB>(y, kk, ntot, sel, cle);
+        if constexpr (ND % 8 == 0) byte_planes_select<G, ND, C, 1, true, WB>(y, kk, ntot, sel, cle);
+        else byte_select_multi<G, ND, C, 1, true, WB>(y, kk, ntot, sel, cle);
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             uint32_t ys = sel[c][0], base = lo[c];
@@ -527,7 +663,7 @@ __device__ __forceinline__ void rank_pairs(const uint32_t (&raw)[C][NW], uint32_
 }
 
 // The three rank pairs of a relative threshold (median, first and third quartile) of an
-// 8-bit stack in one byte search: the bytes are packed once and the 3*C chains interleave.
+// 8-bit stack (byte_select_quartiles); the bytes are packed once.
 template <int G, int NW, int C>
 __device__ __forceinline__ void rank_triples_u8(const uint32_t (&raw)[C][NW], const RankPlan& plan, int32_t ntot,
                                                 uint32_t real, uint32_t (&m0)[C], uint32_t (&m1)[C], uint32_t (&a0)[C],
@@ -546,6 +682,31 @@ __device__ __forceinline__ void rank_triples_u8(const uint32_t (&raw)[C][NW], co
         m1[c] = plan.m1 == plan.m0 ? m0[c] : neighbour<G, NW>(raw[c], m0[c], cle[c][0], plan.m1);
         a1[c] = plan.a1 == plan.a0 ? a0[c] : neighbour<G, NW>(raw[c], a0[c], cle[c][1], plan.a1);
         b1[c] = plan.b1 == plan.b0 ? b0[c] : neighbour<G, NW>(raw[c], b0[c], cle[c][2], plan.b1);
+    }
+}
+
+// The same of a 16-bit stack: all ranks of a channel from its 16 bit planes.
+template <int G, int NW, int C>
+__device__ __forceinline__ void rank_triples_u16(const uint32_t (&raw)[C][NW], const RankPlan& plan, int32_t ntot,
+                                                 uint32_t (&m0)[C], uint32_t (&m1)[C], uint32_t (&a0)[C],
+                                                 uint32_t (&a1)[C], uint32_t (&b0)[C], uint32_t (&b1)[C]) {
+    const uint32_t kk[3] = {plan.m0, plan.a0, plan.b0};
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        uint32_t pl[1][NW / 16][16], sel[1][3], cle[1][3];
+#pragma unroll
+        for (int g = 0; g < NW / 16; ++g) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) pl[0][g][i] = raw[c][16 * g + i];
+            to_planes<16>(pl[0][g]);
+        }
+        plane_select<G, NW / 16, 16, 1, 3, true>(pl, kk, ntot, sel, cle);
+        m0[c] = sel[0][0];
+        a0[c] = sel[0][1];
+        b0[c] = sel[0][2];
+        m1[c] = plan.m1 == plan.m0 ? m0[c] : neighbour<G, NW>(raw[c], m0[c], cle[0][0], plan.m1);
+        a1[c] = plan.a1 == plan.a0 ? a0[c] : neighbour<G, NW>(raw[c], a0[c], cle[0][1], plan.a1);
+        b1[c] = plan.b1 == plan.b0 ? b0[c] : neighbour<G, NW>(raw[c], b0[c], cle[0][2], plan.b1);
     }
 }
 
@@ -1480,7 +1641,9 @@ __device__ __forceinline__ void outlier_tile(const OutlierK& k, uint32_t bx, uin
                 constexpr int E = decltype(e_t)::value;
                 const uint32_t (&re)[C][NFW] = *reinterpret_cast<const uint32_t(*)[C][NFW]>(&blk[E * C][0]);
                 uint32_t m0[C], m1[C], a0[C], a1[C], b0[C], b1[C];
-                if constexpr (!ABS && B == 1) {
+                if constexpr (!ABS && B == 2 && NFW % 16 == 0) {
+                    rank_triples_u16<G, NFW, C>(re, plan, G * NF, m0, m1, a0, a1, b0, b1);
+                } else if constexpr (!ABS && B == 1) {
                     rank_triples_u8<G, NFW, C>(re, plan, G * NF, blk_real, m0, m1, a0, a1, b0, b1);
                 } else {
                     rank_pairs<B, G, NFW, C, WINDOW>(re, plan.m0, plan.m1, G * NF, blk_real, blk_count, m0, m1);

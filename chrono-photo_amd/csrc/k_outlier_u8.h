@@ -826,9 +826,12 @@ __device__ __forceinline__ void outlier_u8_tile(const OutlierK& k, uint32_t bx, 
 
 // VGPRs the frame blocks take, for the occupancy hint: X * C * (F + FS) / 4, plus F for the
 // pairs a sorting network works on, plus working registers.
-constexpr int waves_hint_u8(int C, int F, int X, int FS, bool sort, bool xch = false) {
+constexpr int waves_hint_u8(int C, int F, int X, int FS, bool ABS, bool sort, bool xch) {
     if (xch) {
-        const int v = 512 / (C * (F + FS) / 4 + 48);
+        // the bit planes of one channel and, with four channels, what the load keeps beside them:
+        // 256 x 1080p RGB8 relative took 817 us at the 5 waves that spill them and 760 us at 4
+        const int planes = ABS || !plane_ranks(F / 4, C) ? 0 : F / 4 + (C == 4 ? 16 : 0);
+        const int v = 512 / (C * (F + FS) / 4 + 48 + planes);
         return v < 2 ? 2 : (v > 6 ? 6 : v);
     }
     const int w = 448 / (X * C * (F + FS) / 4 + (sort ? F : 0) + 64);
@@ -836,7 +839,7 @@ constexpr int waves_hint_u8(int C, int F, int X, int FS, bool sort, bool xch = f
 }
 
 template <int C, int G, int F, int X, int FS, bool ABS, bool SORT = false, bool XCH = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, SORT, XCH))))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint_u8(C, F, X, FS, ABS, SORT, XCH))))
 outlier_u8_kernel(OutlierK k, uint32_t tiles_x) {
     __shared__ TileShared<C, G, F, X, false> sh;
     __shared__ uint64_t soff[FS > 0 ? G * (FS + 2) : 1];

@@ -80,32 +80,32 @@ constexpr int kBucketCand[2][2][kNumBuckets][kMaxCand] = {
 // (-1: none): the fastest of the bucket's candidates over 1080p stacks of the scene generator at
 // the bucket's limit and at counts inside it, extreme, forward and average modes.  us at 1080p
 // RGB, the choice and the first candidate, abs/0.05/0.2 extreme, then rel/2.0/4.0 average:
-//   8 bits    16: 40, 49 and 76, 110      32: 68, 81 and 140, 174    64: 132, 180 and 272, 368
-//            128: 221, 349 and 518, 703  256: 416, 901 and 1043, 1502  512: 852, 2004 and 1971, 4042
+//   8 bits    16: 40, 49 and 76, 113      32: 68, 81 and 133, 153    64: 132, 180 and 240, 357
+//            128: 221, 349 and 502, 661  256: 416, 901 and 988, 1461  512: 852, 2004 and 1910, 2850
 //            768: 1190, 1958 and 3002, 6050   1024: 1603, 2401 and 4324, 7801
-//   16 bits   16: 108, 121 and 186, 202   64: 233, 268 and 611, 751
-//            128: 437 and 1267, 1497     256: 790 and 2606, 2983
-// (two 16-bit pixels per lane load better, one leaves more waves: the three full searches of
-// relative thresholds and the few loads of short stacks want the waves).
+//   16 bits   16: 108, 121 and 184, 202   64: 233, 268 and 381, 434
+//            128: 437 and 740, 904       256: 790 and 1627, 1850
+// (two 16-bit pixels per lane load better, one leaves more waves: the three ranks of relative
+// thresholds and the few loads of short stacks want the waves).
 constexpr int kDefault[2][2][2][kNumBuckets] = {
     {{{kU8Base + 0, kU8Base + 1, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
        kU8Base + 23},
-      {kU8Base + 14, kU8Base + 15, kU8Base + 17, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+      {kU8Base + 14, kU8Base + 15, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
        kU8Base + 23}},
      {{kU8Base + 14, kU8Base + 1, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
        kU8Base + 23},
-      {kU8Base + 14, kU8Base + 15, kU8Base + 16, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+      {kU8Base + 14, kU8Base + 15, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
        kU8Base + 23}}},
     {{{-1, -1, -1, -1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1, -1, -1, -1}},
      {{0, 1, 3, 13, 14, 15, -1, -1, -1}, {0, 1, 3, 5, 7, 9, -1, -1, -1}}}};
 // The same with the mode: sums: an average mode.
 inline int default_choice(uint32_t bps, uint32_t channels, int bucket, bool absolute, bool sums) {
     const int c = kDefault[bps - 1][channels >= 3][absolute ? 0 : 1][bucket];
-    // 64 frames, relative: the network of one lane ranks fastest, but its tile keeps the average
-    // modes' distances in LDS, and four channels take two networks; the byte search then wins
-    if (c == kU8Base + 16 && (channels == 4 || sums)) return kU8Base + 17;
-    // four channels fill the exchanged dwords, and one lane's loads are already 4 bytes each
-    if (c == kU8Base + 27 && channels == 4) return kU8Base + 17;
+    // 64 frames, the exchange tile and the one whose lanes load their own pixel: four channels
+    // fill the exchanged dwords, and one lane's loads are already 4 bytes each (1080p RGBA
+    // relative: 286 and 277 us); three channels, relative: 206 and 211 us, but 248 and 240 us in
+    // the average modes
+    if (c == kU8Base + 27 && (channels == 4 || (channels == 3 && !absolute && sums))) return kU8Base + 17;
     return c;
 }
 
