@@ -109,8 +109,8 @@ const void* u8_group_c(int shape, bool absolute) {
     case 9: return u8_group<C, 32, 40, 4, 0>(absolute);
     case 10: return u8_group<C, 4, 32, 1, 8>(absolute);
     case 11: return u8_group<C, 8, 32, 1, 8>(absolute);
-    case 12: return u8_group<C, 16, 32, 4, 8>(absolute);
-    case 13: return u8_group<C, 32, 40, 4, 4>(absolute);
+    case 12: return u8_group<C, 4, 64, 1, 32, false, true>(absolute);
+    case 13: return u8_group<C, 8, 64, 1, 16, false, true>(absolute);
     case 14: return u8_group<C, 1, 16, 1, 0, true>(absolute);
     case 15: return u8_group<C, 1, 32, 1, 0, true>(absolute);
     case 16: return u8_group<C, 1, 64, 1, 0, true>(absolute);
@@ -121,10 +121,8 @@ const void* u8_group_c(int shape, bool absolute) {
     case 21: return u8_group<C, 8, 96, 1, 0, false, true>(absolute);
     case 22: return u8_group<C, 8, 128, 1, 0, false, true>(absolute);
     case 23: return u8_group<C, 8, 160, 1, 0, false, true>(absolute);
-    case 24: return u8_group<C, 4, 64, 1, 32, false, true>(absolute);
-    case 25: return u8_group<C, 8, 64, 1, 16, false, true>(absolute);
-    case 26: return u8_group<C, 8, 160, 1, 16, false, true>(absolute);
-    case 27: return u8_group<C, 1, 64, 1, 0, false, true>(absolute);
+    case 24: return u8_group<C, 8, 160, 1, 16, false, true>(absolute);
+    case 25: return u8_group<C, 1, 64, 1, 0, false, true>(absolute);
     default: return nullptr;
     }
 }

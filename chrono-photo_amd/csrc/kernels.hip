@@ -20,12 +20,12 @@ static int launch_outlier_generic_b(const cp_stack* st, const OutlierK& k, hipSt
 }
 
 OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uint64_t max_pos, uint32_t flags) {
-    // 8-bit composites take the packed-byte
-    // kernel up to 1280 frames (and, with a `--sample` subset, up to 128 sample frames) or the
-    // tuned choice between the two kernels; 16-bit ones the 16-bit kernel up to 1024 frames (and
-    // up to 128 sample frames); the one-lane-per-pixel generic kernel takes the rest.  A
-    // packed-byte choice whose wide loads would read past a borrowed stack's end falls back to
-    // the bucket's 16-bit-halves shape, or to the generic kernel where the bucket has none.
+    // 8-bit composites take the packed-byte kernel up to 1280 frames (and, with a `--sample`
+    // subset, up to 128 sample frames) or the tuned choice between the two kernels; 16-bit ones
+    // the 16-bit kernel up to 1024 frames (and up to 128 sample frames); the one-lane-per-pixel
+    // generic kernel takes the rest.  A packed-byte choice whose wide loads would read past a
+    // borrowed stack's end falls back to the bucket's 16-bit-halves shape, or to the generic
+    // kernel where the bucket has none.
     OutlierPlan p;
     const bool sums = k.background == 2 || k.outlier == 3;
     if (flags & CP_FLAG_FORCE_GENERIC) return p;
@@ -34,8 +34,8 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
     };
     if (k.sample_mask != nullptr) {
         if (st->bps == 1 && k.n <= kU8MaxFrames && k.n_sample <= kU8MaxSample && k.samp_off) {
-            int sh = u8_shape_for(k.n, true, k.n_sample, true);
-            if (sh < 0 || !u8_fits(sh)) sh = u8_shape_for(k.n, true, k.n_sample, false);
+            int sh = u8_sample_shape(k.n, k.n_sample, true);
+            if (sh < 0 || !u8_fits(sh)) sh = u8_sample_shape(k.n, k.n_sample, false);
             if (sh >= 0 && u8_fits(sh)) p = {kPlanU8, sh};
         }
         if (st->bps == 2 && k.n <= kFastMaxFrames && k.n_sample <= kFastMaxSample && k.samp_off) {

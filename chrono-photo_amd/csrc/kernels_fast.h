@@ -53,7 +53,7 @@ constexpr int kBucketCand[2][2][kNumBuckets][kMaxCand] = {
     // 8-bit, 1-2 channels: the packed-byte kernel only
     {{{kU8Base + 0, kU8Base + 14, -1, -1, -1, -1},
       {kU8Base + 1, kU8Base + 15, -1, -1, -1, -1},
-      {kU8Base + 2, kU8Base + 16, kU8Base + 17, kU8Base + 27, -1, -1},
+      {kU8Base + 2, kU8Base + 16, kU8Base + 17, kU8Base + 25, -1, -1},
       {kU8Base + 3, kU8Base + 18, -1, -1, -1, -1},
       {kU8Base + 4, kU8Base + 19, -1, -1, -1, -1},
       {kU8Base + 6, kU8Base + 5, kU8Base + 20, -1, -1, -1},
@@ -63,7 +63,7 @@ constexpr int kBucketCand[2][2][kNumBuckets][kMaxCand] = {
      // 8-bit, 3-4 channels
      {{0, kU8Base + 0, kU8Base + 14, -1, -1, -1},
       {1, 2, kU8Base + 1, kU8Base + 15, -1, -1},
-      {3, 4, kU8Base + 2, kU8Base + 16, kU8Base + 17, kU8Base + 27},
+      {3, 4, kU8Base + 2, kU8Base + 16, kU8Base + 17, kU8Base + 25},
       {5, 6, kU8Base + 3, kU8Base + 18, -1, -1},
       {7, 8, kU8Base + 4, kU8Base + 19, -1, -1},
       {9, kU8Base + 6, kU8Base + 5, kU8Base + 20, -1, -1},
@@ -88,13 +88,13 @@ constexpr int kBucketCand[2][2][kNumBuckets][kMaxCand] = {
 // (two 16-bit pixels per lane load better, one leaves more waves: the three ranks of relative
 // thresholds and the few loads of short stacks want the waves).
 constexpr int kDefault[2][2][2][kNumBuckets] = {
-    {{{kU8Base + 0, kU8Base + 1, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+    {{{kU8Base + 0, kU8Base + 1, kU8Base + 25, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
        kU8Base + 23},
-      {kU8Base + 14, kU8Base + 15, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+      {kU8Base + 14, kU8Base + 15, kU8Base + 25, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
        kU8Base + 23}},
-     {{kU8Base + 14, kU8Base + 1, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+     {{kU8Base + 14, kU8Base + 1, kU8Base + 25, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
        kU8Base + 23},
-      {kU8Base + 14, kU8Base + 15, kU8Base + 27, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
+      {kU8Base + 14, kU8Base + 15, kU8Base + 25, kU8Base + 18, kU8Base + 19, kU8Base + 20, kU8Base + 21, kU8Base + 22,
        kU8Base + 23}}},
     {{{-1, -1, -1, -1, -1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1, -1, -1, -1, -1}},
      {{0, 1, 3, 13, 14, 15, -1, -1, -1}, {0, 1, 3, 5, 7, 9, -1, -1, -1}}}};
@@ -105,7 +105,7 @@ inline int default_choice(uint32_t bps, uint32_t channels, int bucket, bool abso
     // fill the exchanged dwords, and one lane's loads are already 4 bytes each (1080p RGBA
     // relative: 286 and 277 us); three channels, relative: 206 and 211 us, but 248 and 240 us in
     // the average modes
-    if (c == kU8Base + 27 && (channels == 4 || (channels == 3 && !absolute && sums))) return kU8Base + 17;
+    if (c == kU8Base + 25 && (channels == 4 || (channels == 3 && !absolute && sums))) return kU8Base + 17;
     return c;
 }
 

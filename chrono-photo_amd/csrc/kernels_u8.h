@@ -17,26 +17,26 @@ struct U8Shape {
 // One pixel per lane for short stacks; four pixels per lane (one 16-byte load per frame)
 // for tall ones; `--sample` shapes carry an FS-frame block of the sample positions; shapes
 // 14-16 rank one lane's whole pixel with a sorting network; shape 17 holds a 64-frame pixel
-// in one lane for the byte search (a candidate only: u8_shape_for meets shape 2 first).
-// Shapes from 18 on are exchange tiles, 24-26 with a block of up to 128 sample frames.
-constexpr int kNumU8Shapes = 28;
+// in one lane.  Shapes 12, 13 and from 18 on are exchange tiles, 12, 13 and 24 with a block of
+// up to 128 sample frames.
+constexpr int kNumU8Shapes = 26;
 constexpr U8Shape kU8Shapes[kNumU8Shapes] = {
     {1, 16, 1, 0, 0},      {1, 32, 1, 0, 0},      {2, 32, 1, 0, 0},      {4, 32, 1, 0, 0},     {8, 32, 1, 0, 0},
     {16, 32, 1, 0, 0},     {16, 32, 4, 0, 0},     {32, 24, 4, 0, 0},     {32, 32, 4, 0, 0},    {32, 40, 4, 0, 0},
-    {4, 32, 1, 8, 0},      {8, 32, 1, 8, 0},      {16, 32, 4, 8, 0},     {32, 40, 4, 4, 0},    {1, 16, 1, 0, 1},
+    {4, 32, 1, 8, 0},      {8, 32, 1, 8, 0},      {4, 64, 1, 32, 0, 4},  {8, 64, 1, 16, 0, 4}, {1, 16, 1, 0, 1},
     {1, 32, 1, 0, 1},      {1, 64, 1, 0, 1},      {1, 64, 1, 0, 0},      {2, 64, 1, 0, 0, 4},  {4, 64, 1, 0, 0, 4},
-    {8, 64, 1, 0, 0, 4},   {8, 96, 1, 0, 0, 4},   {8, 128, 1, 0, 0, 4},  {8, 160, 1, 0, 0, 4}, {4, 64, 1, 32, 0, 4},
-    {8, 64, 1, 16, 0, 4},  {8, 160, 1, 16, 0, 4}, {1, 64, 1, 0, 0, 4}};
+    {8, 64, 1, 0, 0, 4},   {8, 96, 1, 0, 0, 4},   {8, 128, 1, 0, 0, 4},  {8, 160, 1, 0, 0, 4}, {8, 160, 1, 16, 0, 4},
+    {1, 64, 1, 0, 0, 4}};
 constexpr uint32_t kU8MaxFrames = 32 * 40;
 constexpr uint32_t kU8MaxSample = 128;
 
-// The smallest shape that holds n frames (and s sample frames when sampled), or -1; exchange:
-// among the exchange tiles or among the others.
-inline int u8_shape_for(uint32_t n, bool sampled, uint32_t s, bool exchange) {
+// The smallest shape with a sample block that holds n frames and s sample frames, or -1;
+// exchange: among the exchange tiles or among the others.
+inline int u8_sample_shape(uint32_t n, uint32_t s, bool exchange) {
     for (int i = 0; i < kNumU8Shapes; ++i) {
         const U8Shape& sh = kU8Shapes[i];
-        if ((sh.FS > 0) != sampled || sh.S || (sh.L > 0) != exchange) continue;
-        if ((uint32_t)(sh.G * sh.F) >= n && (!sampled || (uint32_t)(sh.G * sh.FS) >= s)) return i;
+        if (sh.FS > 0 && (sh.L > 0) == exchange && (uint32_t)(sh.G * sh.F) >= n && (uint32_t)(sh.G * sh.FS) >= s)
+            return i;
     }
     return -1;
 }
@@ -67,8 +67,8 @@ inline bool launch_u8_c(const OutlierK& k, int shape, hipStream_t s) {
     case 9: launch_u8_shape<C, 32, 40, 4, 0>(k, s); return true;
     case 10: launch_u8_shape<C, 4, 32, 1, 8>(k, s); return true;
     case 11: launch_u8_shape<C, 8, 32, 1, 8>(k, s); return true;
-    case 12: launch_u8_shape<C, 16, 32, 4, 8>(k, s); return true;
-    case 13: launch_u8_shape<C, 32, 40, 4, 4>(k, s); return true;
+    case 12: launch_u8_shape<C, 4, 64, 1, 32, false, true>(k, s); return true;
+    case 13: launch_u8_shape<C, 8, 64, 1, 16, false, true>(k, s); return true;
     case 14: launch_u8_shape<C, 1, 16, 1, 0, true>(k, s); return true;
     case 15: launch_u8_shape<C, 1, 32, 1, 0, true>(k, s); return true;
     case 16: launch_u8_shape<C, 1, 64, 1, 0, true>(k, s); return true;
@@ -79,10 +79,8 @@ inline bool launch_u8_c(const OutlierK& k, int shape, hipStream_t s) {
     case 21: launch_u8_shape<C, 8, 96, 1, 0, false, true>(k, s); return true;
     case 22: launch_u8_shape<C, 8, 128, 1, 0, false, true>(k, s); return true;
     case 23: launch_u8_shape<C, 8, 160, 1, 0, false, true>(k, s); return true;
-    case 24: launch_u8_shape<C, 4, 64, 1, 32, false, true>(k, s); return true;
-    case 25: launch_u8_shape<C, 8, 64, 1, 16, false, true>(k, s); return true;
-    case 26: launch_u8_shape<C, 8, 160, 1, 16, false, true>(k, s); return true;
-    case 27: launch_u8_shape<C, 1, 64, 1, 0, false, true>(k, s); return true;
+    case 24: launch_u8_shape<C, 8, 160, 1, 16, false, true>(k, s); return true;
+    case 25: launch_u8_shape<C, 1, 64, 1, 0, false, true>(k, s); return true;
     default: return false;
     }
 }
