@@ -196,10 +196,15 @@ __device__ __forceinline__ void load_block_exchange(const uint8_t* __restrict__ 
     const uintptr_t base = (uintptr_t)(row + (uint64_t)(x < out_w ? x : 0u) * C);
     // frame lb * FB + j of the offset table, whose blocks of F entries are F + 2 apart
     const uint64_t* o = off + lb * (uint32_t)FB + 2u * (lb / 4u);
+    // Forty frames of three channels leave no room for the loads' addresses at three waves per
+    // SIMD; the last quad's loads then wait until the first quad has left its registers.  All at
+    // once spilled 7 dwords per lane: 1200 x 1080p RGB8 wrote 412 MB instead of 13 and took 2228
+    // us, 2070 us so.
+    constexpr int HELD = FB >= 40 && C == 3 ? 4 : 0;
     vec raw[FB];
+    auto load = [&](int t) { raw[t] = *(const __attribute__((address_space(1))) vec*)((base + o[t]) & ~(uintptr_t)3); };
 #pragma unroll
-    for (int t = 0; t < FB; ++t)
-        raw[t] = *(const __attribute__((address_space(1))) vec*)((base + o[t]) & ~(uintptr_t)3);
+    for (int t = 0; t < FB - HELD; ++t) load(t);
     __builtin_amdgcn_sched_barrier(0);
     typedef const volatile __attribute__((address_space(3))) uint32_t lu32;  // the low halves, for the shifts
     const uint32_t to = (lb / 4u) * (uint32_t)EX::ROW + lg * 4u;
@@ -230,6 +235,12 @@ __device__ __forceinline__ void load_block_exchange(const uint8_t* __restrict__ 
 #pragma unroll
         for (int c = 0; c < C; ++c)
             *reinterpret_cast<uint4*>(&ex.w[i % BUFS][(lb % 4u) * C + c][to]) = uint4{v[c], v[C + c], v[2 * C + c], v[3 * C + c]};
+        if (HELD > 0 && i == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = FB - HELD; t < FB; ++t) load(t);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         lds_barrier();
 #pragma unroll
         for (int b = 0; b < 4; ++b)
@@ -831,7 +842,10 @@ constexpr int waves_hint_u8(int C, int F, int X, int FS, bool ABS, bool sort, bo
         // the bit planes of one channel and, with four channels, what the load keeps beside them:
         // 256 x 1080p RGB8 relative took 817 us at the 5 waves that spill them and 760 us at 4
         const int planes = ABS || !plane_ranks(F / 4, C) ? 0 : F / 4 + (C == 4 ? 16 : 0);
-        const int v = 512 / (C * (F + FS) / 4 + 48 + planes);
+        // a block of sample frames comes after the block of all frames and needs no registers when
+        // that one's loads peak: 1200 x 1080p RGB8 with 64 sample frames 2490 us at 2 waves, 2034
+        // us at 3
+        const int v = 512 / (C * F / 4 + 48 + planes);
         return v < 2 ? 2 : (v > 6 ? 6 : v);
     }
     const int w = 448 / (X * C * (F + FS) / 4 + (sort ? F : 0) + 64);
