@@ -157,6 +157,7 @@ const void* fast_group_bc(int shape, bool absolute) {
     case 12: return fast_group<B, C, 2, 32, 2, 2>(absolute);
     case 13: return fast_group<B, C, 4, 32, 2, 2>(absolute);
     case 14: return fast_group<B, C, 8, 32, 2, 2>(absolute);
+    case 15: return fast_group<B, C, 16, 32, 2, 2>(absolute);
     default: return nullptr;
     }
 }

@@ -109,3 +109,35 @@ def test_u16_sums_past_24_bits(ctx, n, c):
     for mode in ((True, 0.3, 0.5, 2, 3), (True, 0.02, 0.1, 2, 2), (False, 1.0, 2.0, 2, 3)):
         gpu, ref = run_both(ctx, x, *mode)
         assert_same(gpu, ref, f"n={n} c={c} mode={mode}")
+
+
+@pytest.mark.parametrize("c", [3, 4])
+def test_u16_batch_group_to_512_frames(ctx, c):
+    """16-bit 3/4-channel jobs of 257 to 512 frames share a group launch, absolute thresholds on the
+    two-pixel tile and relative ones on the one-pixel tile; widths inside a pixel pair."""
+    import oracle_py as O
+    from chrono_photo_amd import hip as H
+    jobs, keep = [], []
+    for i, (n, w) in enumerate(((257, 33), (300, 40), (449, 18), (512, 35))):
+        x = make_stack(8800 + n + c, n, 5, w, c, bits=16, outlier_frac=0.1)
+        st = cpa.Stack.from_array(ctx, x)
+        thr = cpa.Threshold.abs(0.05, 0.2) if i % 2 == 0 else cpa.Threshold.rel(2.0, 4.0)
+        px, mask = H.DeviceBuffer(x[0].nbytes), H.DeviceBuffer(x[0].size)
+        jobs.append(cpa.Job(cpa.CP_MODE_OUTLIER, st, px.ptr, mask.ptr, processor=cpa.OutlierProcessor(thr, i, i + 1, seed=3)))
+        keep.append((x, st, px, mask))
+    batch = cpa.Batch(ctx, jobs, graph=True)
+    info = batch.info()
+    assert info["group_jobs"] == 4 and info["group_launches"] == 2, info
+    for rep in range(3):
+        batch.launch()
+        ctx.synchronize()
+        for i, (x, st, px, mask) in enumerate(keep):
+            lo, hi = ((0.05, 0.2), (2.0, 4.0))[i % 2]
+            oimg, omask, _ = O.outlier(x, O.threshold(i % 2 == 0, lo, hi, 2), i, i + 1, seed=3)
+            assert np.array_equal(px.to_host(np.zeros(x[0].shape, x.dtype)), oimg), (rep, i)
+            assert np.array_equal(mask.to_host(np.zeros(x[0].shape, np.uint8)), omask), (rep, i)
+    batch.close()
+    for x, st, px, mask in keep:
+        st.close()
+        px.free()
+        mask.free()
