@@ -926,7 +926,7 @@ def tile_shapes_set(ctx: Context, bytes_per_sample: int, channels: int, shapes, 
     """cp_tile_shapes_set: pins the kernel choice per frame bucket (TILE_BUCKETS) for absolute
     thresholds (`shapes`) and relative ones (`rel_shapes`, default: the same); each entry is
     (lanes_per_pixel, frames_per_lane, pixels_per_lane[, kernel]) as autotune returns it
-    (kernel 1: the 8-bit packed-byte kernel with the byte search, 2: the same with a sorting
+    (kernel 1: the 8-bit packed-byte kernel with rank searches, 2: the same with a sorting
     network for the ranks, 0 or absent: the 16-bit-halves kernel), or None for the bucket's
     default.  Missing trailing buckets take their defaults."""
     nb = len(TILE_BUCKETS)
@@ -939,7 +939,7 @@ def tile_shapes_set(ctx: Context, bytes_per_sample: int, channels: int, shapes, 
 def autotune(ctx: Context, bytes_per_sample: int, channels: int):
     """Runs the kernel autotuner; returns {"abs": [...], "rel": [...]}: per bucket of
     TILE_BUCKETS and threshold kind, the chosen (lanes_per_pixel, frames_per_lane,
-    pixels_per_lane, kernel), or None where no register-resident kernel covers the bucket."""
+    pixels_per_lane, kernel), or None where the bucket has no candidates to choose from."""
     nb = len(TILE_BUCKETS)
     out = (C.c_int32 * (2 * nb))()
     _check(ctx.lib.cp_autotune(ctx.handle, bytes_per_sample, channels, out))

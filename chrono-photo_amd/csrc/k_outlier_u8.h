@@ -168,8 +168,8 @@ __device__ __forceinline__ void lds_barrier() {
 // every pixel of the tile and 64 / (256 / G / 4) frame blocks), and the transposed dwords go
 // through LDS, four frames of every block at a time, to the lanes that own the pixels.
 // 1080p RGB8, abs/0.05/0.2, extreme, against the best tile without the exchange: 128 frames 257 ->
-// 221 us, 256 frames 588 -> 416 us, 512 frames 1006 -> 852 us, 1200 frames 3.30 -> 2.23 ms (loads
-// alone 2.07 ms at that pattern); rel/2.0/4.0, average: 518, 1043, 1971 us where 640, 1230 and
+// 221 us, 256 frames 588 -> 416 us, 512 frames 1006 -> 852 us, 1200 frames 3.30 -> 2.08 ms (a
+// streaming read of the bytes 1.12 ms); rel/2.0/4.0, average: 518, 1043, 1971 us where 640, 1230 and
 // 2475 us were the best, and 700 x 720p rel/2.5/5.0 2.30 -> 1.19 ms.
 template <int C, int G, int BUFS>
 struct ExchangeLds {

@@ -270,13 +270,16 @@ CP_API int cp_batch_run(cp_ctx* ctx, const cp_job* jobs, uint32_t n_jobs, uint32
 /* Autotuner: for each threshold kind (absolute, relative) and frame-count bucket of the
  * register-resident outlier kernels (<= 16, 32, 64, 128, 256, 512, 768, 1024, 1280 frames:
  * CP_TILE_BUCKETS buckets) time the candidate kernel choices on a synthetic stack of this
- * sample width and channel count (1-4) and keep the fastest for the context.  A choice is a tile shape of the 16-bit-halves kernel or of
- * the 8-bit packed-byte kernel, whose one-lane-per-pixel shapes rank either by the byte
- * search or by a sorting network; shapes (nullable, 2 * CP_TILE_BUCKETS entries: absolute
- * thresholds' buckets, then relative thresholds') receives
- * (kernel << 24) | (pixels_per_lane << 16) | (lanes_per_pixel << 8) | frames_per_lane per
- * bucket (kernel 0: 16-bit halves, 1: packed bytes with the byte search, 2: packed bytes
- * with the sorting network), or 0 where no register-resident kernel covers the bucket. */
+ * sample width and channel count (1-4) and keep the fastest for the context.  A choice is a
+ * tile shape of the 16-bit-halves kernel or of the 8-bit packed-byte kernel, whose
+ * one-lane-per-pixel shapes rank either by searches or by a sorting network; shapes (nullable,
+ * 2 * CP_TILE_BUCKETS entries: absolute thresholds' buckets, then relative thresholds')
+ * receives (kernel << 24) | (pixels_per_lane << 16) | (lanes_per_pixel << 8) | frames_per_lane
+ * per bucket (kernel 0: 16-bit halves, 1: packed bytes with rank searches, 2: packed bytes
+ * with the sorting network; pixels_per_lane counts the pixels of one load, which the lanes of
+ * kernel 1's tiles with 64 and more frames per lane exchange so that each keeps one), or 0
+ * where the bucket has no candidates (16-bit stacks with 1-2 channels or over 512 frames have
+ * one shape each, or none). */
 #define CP_TILE_BUCKETS 9
 CP_API int cp_autotune(cp_ctx* ctx, uint32_t bytes_per_sample, uint32_t channels, int32_t* shapes);
 /* Sets the context's kernel choice per bucket without timing anything (no reference
