@@ -104,6 +104,11 @@ int launch_simple(cp_ctx* ctx, const cp_stack* st, const SimpleK& k_in, hipStrea
     // whole-number steps (k_simple.h) where every weight is one and nothing fades
     bool plain = k.fade.is_none != 0;
     for (uint32_t c = 0; c < st->channels; ++c) plain = plain && k.w[c] == 1.0f;
+    // Tall 8-bit stacks of up to three channels stream faster through the general step, whose waves
+    // stay closer together in the stack (us, general and whole-number step, 1280x721 mono, then RGB:
+    // 128 frames 65 and 50, 89 and 80; 300 frames 131 and 135, 183 and 185; 1100 frames 412 and 553,
+    // 599 and 680); four channels do not (1100 frames 777 and 731).
+    if (st->bps == 1 && st->channels < 4 && k.n > 256) plain = false;
     if (st->bps == 1) plain ? launch_simple_b<1, 4, true>(st, k, s) : launch_simple_b<1, 4, false>(st, k, s);
     else plain ? launch_simple_b<2, 2, true>(st, k, s) : launch_simple_b<2, 2, false>(st, k, s);
     hipError_t e = hipGetLastError();
