@@ -17,8 +17,8 @@
 // number that f32 holds exactly, and a new extreme replaces the pixel: PlainPixels keeps the
 // pixels packed as they lie in memory and takes one or two dot products, a compare and two
 // selects per pixel and frame.  Bound by HBM.  The general step (about 28 VALU instructions per
-// pixel and frame) was bound by VALU issue: 64 x 1080p RGB8, per call, 93 us with it and 72.5 us
-// (5.6 TB/s) without.
+// pixel and frame) was bound by VALU issue: 64 x 1080p RGB8, per call, 93 us with it and 67.5 us
+// (6.0 TB/s) without.
 #pragma once
 #include "device_common.h"
 
