@@ -42,7 +42,7 @@ constexpr uint32_t psel(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3) {
 // NW words of bytes from byte address a: word h holds bytes a + 4h .. a + 4h + 3.  They come
 // from the NQ dwords at or below a, realigned by a's offset in its dword: NQ = NW + 1 in
 // general, NQ = NW when a is dword-aligned (4-channel samples), NQ = NW = 1 when the bytes
-// needed lie in a's dword (one pixel of 1 or 2 channels).
+// needed lie in a's dword (one pixel of 1 channel, or of 2 at an even address).
 template <int NQ, int NW>
 __device__ __forceinline__ void load_realigned(const uint8_t* a, uint32_t (&w)[NW]) {
     static_assert(NQ <= 4, "at most 16 bytes per load");
@@ -867,10 +867,13 @@ outlier_u8_kernel(OutlierK k, uint32_t tiles_x) {
 
 // Whether the packed-byte tiles may run over this composite: every lane's load of a frame
 // (X * C bytes read with up to 8 bytes around them from the dword at or below them) stays
-// inside the stack allocation, and 4-channel stacks start on a dword boundary.
+// inside the stack allocation, and 4-channel stacks start on a dword boundary.  X: the pixels of
+// a load.  One pixel of 2 channels is read as the dword of its first byte, which holds the second
+// one too where the stack starts on an even address; on an odd one a pixel in four straddles two.
 inline bool u8_tile_fits(const void* stack, uint64_t alloc_bytes, uint32_t channels, int X, const OutlierK& k,
                          uint64_t max_pos) {
     if (channels == 4 && ((uintptr_t)stack & 3u)) return false;
+    if (channels == 2 && X == 1 && ((uintptr_t)stack & 1u)) return false;
     const uint64_t x_last = (uint64_t)((k.out_w - 1) / X) * X;
     const uint64_t first = max_pos + ((uint64_t)(k.out_h - 1) * k.stack_w + x_last) * channels;
     return first + (uint64_t)X * channels + 8 <= alloc_bytes;
