@@ -138,12 +138,12 @@ struct PlainPixels {
     typedef unsigned short us2s __attribute__((ext_vector_type(2)));
 };
 
-// PLAIN: unit weights and no fade.
-// (The general step of 8-bit frames needs more registers than eight waves leave: held to them, 90 x
-// 1280x721 RGBA8 with weights took 139 us instead of 118, with crops 202 instead of 117.  That of
-// 16-bit frames fits: 90 x RGB16 with weights and crops 96 us, 117 without the bound.)
-template <int B, int C, int PX, bool PLAIN>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PLAIN || B == 2 ? 8 : 1))) simple_kernel(SimpleK k) {
+// PLAIN: unit weights and no fade.  TABLE: the frame positions' offsets come from a table (crops,
+// uneven selections) or from their spacing; a test of that per frame waited for each entry before
+// it asked for the next (20 x 1280x721 mono lighter with weights and crops 23.3 us, 22.4 us without
+// it; 700 x 16 bits, two channels, 512 and 453 us with the register bound below gone as well).
+template <int B, int C, int PX, bool PLAIN, bool TABLE>
+__device__ __forceinline__ void simple_pixels(const SimpleK& k) {
     const uint32_t x0 = (blockIdx.x * blockDim.x + threadIdx.x) * PX;
     const uint32_t y = blockIdx.y;
     if (x0 >= k.out_w || y >= k.out_h) return;
@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PLAIN 
             int32_t t = 0;
             for (; t + UF <= N; t += UF) {
 #pragma unroll
-                for (int u = 0; u < UF; ++u) load(u, k.pos_off[t + u]);
+                for (int u = 0; u < UF; ++u) load(u, k.pos_off.wave_at<TABLE>(t + u));
 #pragma unroll
                 for (int u = 0; u < UF; ++u) {
                     uint32_t w[ND];
@@ -194,7 +194,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PLAIN 
                 }
             }
             for (; t < N; ++t) {
-                load(0, k.pos_off[t]);
+                load(0, k.pos_off.wave_at<TABLE>(t));
                 uint32_t w[ND];
 #pragma unroll
                 for (int i = 0; i < ND; ++i) w[i] = __builtin_amdgcn_alignbyte(d[0][i + 1], d[0][i], sh[0]);
@@ -214,7 +214,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PLAIN 
         for (; t + UF <= N; t += UF) {
             uint32_t d[UF][NB / 4 + 1];
 #pragma unroll
-            for (int u = 0; u < UF; ++u) load_segment<B, NB>(k.stack + (k.pos_off[t + u] + pix) * B, d[u]);
+            for (int u = 0; u < UF; ++u) load_segment<B, NB>(k.stack + (k.pos_off.wave_at<TABLE>(t + u) + pix) * B, d[u]);
 #pragma unroll
             for (int u = 0; u < UF; ++u) {
                 uint32_t in[PX][4];
@@ -224,14 +224,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PLAIN 
         }
         for (; t < N; ++t) {
             uint32_t d[NB / 4 + 1];
-            load_segment<B, NB>(k.stack + (k.pos_off[t] + pix) * B, d);
+            load_segment<B, NB>(k.stack + (k.pos_off.wave_at<TABLE>(t) + pix) * B, d);
             uint32_t in[PX][4];
             unpack_segment<B, C, PX>(d, in);
             simple_step<B, C, PX>(k, darker, t, N, in, ext, out);
         }
     } else {
         for (int32_t t = 0; t < N; ++t) {
-            const uint64_t base = k.pos_off[t] + pix;
+            const uint64_t base = k.pos_off.wave_at<TABLE>(t) + pix;
             uint32_t in[PX][4];
 #pragma unroll
             for (int e = 0; e < PX * C; ++e)
@@ -246,6 +246,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PLAIN 
 #pragma unroll
         for (int ch = 0; ch < C; ++ch) store_sample<B>(k.out_px, o + p * C + ch, out[p][ch]);
     }
+}
+
+// The general step takes the registers it needs (22 to 82); held to the 64 of eight waves per SIMD,
+// four 16-bit channels spilled (64 x 1280x721 RGBA16 lighter with weights and crops 99.9 us, 95.9 us
+// without the bound; 90 x RGBA8 139 and 118 us).  The whole-number step fits eight waves.
+template <int B, int C, int PX, bool TABLE>
+__global__ void __launch_bounds__(256) simple_kernel(SimpleK k) {
+    simple_pixels<B, C, PX, false, TABLE>(k);
+}
+
+template <int B, int C, int PX, bool TABLE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) simple_plain_kernel(SimpleK k) {
+    simple_pixels<B, C, PX, true, TABLE>(k);
 }
 
 }  // namespace cp

@@ -80,15 +80,21 @@ int launch_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uint64_t 
     return CP_OK;
 }
 
-template <int B, int PX, bool PLAIN>
-static void launch_simple_b(const cp_stack* st, const SimpleK& k, hipStream_t s) {
+template <int B, int C, int PX, bool TABLE>
+static void launch_simple_c(const SimpleK& k, bool plain, hipStream_t s) {
     const uint32_t lanes = (k.out_w + PX - 1) / PX;
     dim3 block(256), grid((lanes + 255) / 256, k.out_h);
+    if (plain) hipLaunchKernelGGL((simple_plain_kernel<B, C, PX, TABLE>), grid, block, 0, s, k);
+    else hipLaunchKernelGGL((simple_kernel<B, C, PX, TABLE>), grid, block, 0, s, k);
+}
+
+template <int B, int PX, bool TABLE>
+static void launch_simple_b(const cp_stack* st, const SimpleK& k, bool plain, hipStream_t s) {
     switch (st->channels) {
-    case 1: hipLaunchKernelGGL((simple_kernel<B, 1, PX, PLAIN>), grid, block, 0, s, k); break;
-    case 2: hipLaunchKernelGGL((simple_kernel<B, 2, PX, PLAIN>), grid, block, 0, s, k); break;
-    case 3: hipLaunchKernelGGL((simple_kernel<B, 3, PX, PLAIN>), grid, block, 0, s, k); break;
-    default: hipLaunchKernelGGL((simple_kernel<B, 4, PX, PLAIN>), grid, block, 0, s, k); break;
+    case 1: launch_simple_c<B, 1, PX, TABLE>(k, plain, s); break;
+    case 2: launch_simple_c<B, 2, PX, TABLE>(k, plain, s); break;
+    case 3: launch_simple_c<B, 3, PX, TABLE>(k, plain, s); break;
+    default: launch_simple_c<B, 4, PX, TABLE>(k, plain, s); break;
     }
 }
 
@@ -109,8 +115,9 @@ int launch_simple(cp_ctx* ctx, const cp_stack* st, const SimpleK& k_in, hipStrea
     // 128 frames 65 and 50, 89 and 80; 300 frames 131 and 135, 183 and 185; 1100 frames 412 and 553,
     // 599 and 680); four channels do not (1100 frames 777 and 731).
     if (st->bps == 1 && st->channels < 4 && k.n > 256) plain = false;
-    if (st->bps == 1) plain ? launch_simple_b<1, 4, true>(st, k, s) : launch_simple_b<1, 4, false>(st, k, s);
-    else plain ? launch_simple_b<2, 2, true>(st, k, s) : launch_simple_b<2, 2, false>(st, k, s);
+    const bool table = k.pos_off.table != nullptr;
+    if (st->bps == 1) table ? launch_simple_b<1, 4, true>(st, k, plain, s) : launch_simple_b<1, 4, false>(st, k, plain, s);
+    else table ? launch_simple_b<2, 2, true>(st, k, plain, s) : launch_simple_b<2, 2, false>(st, k, plain, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(CP_ERR_HIP, "simple kernel launch: %s", hipGetErrorString(e));
     return CP_OK;

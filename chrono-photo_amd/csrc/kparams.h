@@ -37,6 +37,20 @@ struct PosK {
     __device__ __forceinline__ uint64_t operator[](uint32_t t) const {
         return table ? table[t] : first + (uint64_t)(step * (int64_t)t);
     }
+    // The same for a kernel that knows at compile time which of the two it was given.
+    template <bool TABLE>
+    __device__ __forceinline__ uint64_t at(uint32_t t) const {
+        return TABLE ? table[t] : first + (uint64_t)(step * (int64_t)t);
+    }
+    // at() for a position that a wave's lanes share.  The offset stays scalar: left to itself the
+    // compiler turns the spacing into a pointer per lane and frame in flight (80 vector registers
+    // instead of 64 in the widest darker/lighter kernel).
+    template <bool TABLE>
+    __device__ __forceinline__ uint64_t wave_at(uint32_t t) const {
+        const uint64_t o = at<TABLE>(t);
+        return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(o >> 32)) << 32 |
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)o);
+    }
 };
 
 // One composite over a device-resident stack.  Frame position t (0..n-1) reads sample
