@@ -165,6 +165,7 @@ __device__ __forceinline__ void simple_pixels(const SimpleK& k) {
         if (npx == (uint32_t)PX) {
             constexpr int UF = 8, ND = NB / 4;  // UF frames in flight
             typedef uint32_t words __attribute__((ext_vector_type(ND), aligned(4)));
+            typedef uint32_t words1 __attribute__((ext_vector_type(ND + 1), aligned(4)));
             const uintptr_t base = (uintptr_t)k.stack + pix * B;
             const uint32_t base_sh = __builtin_amdgcn_readfirstlane((uint32_t)base & 3u);  // of the whole row
             PlainPixels<B, C, PX> px;
@@ -172,14 +173,23 @@ __device__ __forceinline__ void simple_pixels(const SimpleK& k) {
             uint32_t d[UF][ND + 1], sh[UF];
             auto load = [&](int u, uint64_t off) {
                 // whole dwords from the one that holds the first byte to the one that holds the
-                // last; the lanes of a wave share the shift
+                // last; the lanes of a wave share the shift.  One load for a shifted segment too
+                // (700 x 1280x721 RGB16 with crops 708 us with a second load for its last dword,
+                // 680 us so)
                 const uintptr_t a = base + off * B;
                 sh[u] = (base_sh + (uint32_t)off * B) & 3u;
-                const words v = *(const __attribute__((address_space(1))) words*)(a & ~(uintptr_t)3);
+                const uintptr_t w = a & ~(uintptr_t)3;
+                if (ND < 4 && sh[u] != 0u) {
+                    const words1 v = *(const __attribute__((address_space(1))) words1*)w;
+#pragma unroll
+                    for (int i = 0; i <= ND; ++i) d[u][i] = v[i];
+                    return;
+                }
+                const words v = *(const __attribute__((address_space(1))) words*)w;
 #pragma unroll
                 for (int i = 0; i < ND; ++i) d[u][i] = v[i];
                 d[u][ND] = 0u;
-                if (sh[u] != 0u) d[u][ND] = *(const __attribute__((address_space(1))) uint32_t*)((a & ~(uintptr_t)3) + NB);
+                if (ND >= 4 && sh[u] != 0u) d[u][ND] = *(const __attribute__((address_space(1))) uint32_t*)(w + NB);
             };
             int32_t t = 0;
             for (; t + UF <= N; t += UF) {
