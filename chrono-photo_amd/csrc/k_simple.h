@@ -144,9 +144,19 @@ struct PlainPixels {
 // it; 700 x 16 bits, two channels, 512 and 453 us with the register bound below gone as well).
 template <int B, int C, int PX, bool PLAIN, bool TABLE>
 __device__ __forceinline__ void simple_pixels(const SimpleK& k) {
-    const uint32_t x0 = (blockIdx.x * blockDim.x + threadIdx.x) * PX;
+    uint32_t x0 = (blockIdx.x * blockDim.x + threadIdx.x) * PX;
     const uint32_t y = blockIdx.y;
     if (x0 >= k.out_w || y >= k.out_h) return;
+    // A row that ends inside a lane's pixels: the lanes of its last wave all step back to end with
+    // it, so that every lane holds whole segments and the wave keeps one shift.  The pixels that
+    // lane 0 then shares with the wave before are that wave's to store.  Only a row of a single
+    // wave keeps a partial lane, which loads one frame's samples after another's (a latency
+    // each: 48 x 1281x721 RGB8 took 43.6 us with one at the end of the frame and takes 23.5 us so,
+    // 300 frames 315 and 148 us; the same at 1280x721 22.8 and 152 us).
+    const uint32_t part = k.out_w % PX;
+    const uint32_t wave_x0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 256u + (threadIdx.x & ~63u)) * PX);
+    const bool back = part != 0u && wave_x0 != 0u && k.out_w - wave_x0 <= 64u * PX;
+    if (back) x0 -= PX - part;
     const uint32_t npx = min((uint32_t)PX, k.out_w - x0);
     const bool darker = k.darker != 0;
     float ext[PX];
@@ -210,11 +220,21 @@ __device__ __forceinline__ void simple_pixels(const SimpleK& k) {
                 for (int i = 0; i < ND; ++i) w[i] = __builtin_amdgcn_alignbyte(d[0][i + 1], d[0][i], sh[0]);
                 px.step(w, darker);
             }
+            const uint64_t at = ((uint64_t)y * k.out_w + x0) * C;
+            const uint32_t skip = back && __lane_id() == 0u ? PX - part : 0u;
+            if (skip != 0u) {
+                uint32_t v[PX][4];
+                unpack_segment<B, C, PX>(px.out, v);
+#pragma unroll
+                for (int e = 0; e < PX * C; ++e)
+                    if ((uint32_t)(e / C) >= skip) store_sample<B>(k.out_px, at + e, v[e / C][e % C]);
+                return;
+            }
             typedef uint32_t out_words __attribute__((ext_vector_type(ND), aligned(B)));
             out_words o;
 #pragma unroll
             for (int i = 0; i < ND; ++i) o[i] = px.out[i];
-            *(__attribute__((address_space(1))) out_words*)((uintptr_t)k.out_px + ((uint64_t)y * k.out_w + x0) * C * B) = o;
+            *(__attribute__((address_space(1))) out_words*)((uintptr_t)k.out_px + at * B) = o;
             return;
         }
     }
@@ -249,10 +269,12 @@ __device__ __forceinline__ void simple_pixels(const SimpleK& k) {
             simple_step<B, C, PX>(k, darker, t, N, in, ext, out);
         }
     }
+    const uint32_t skip = back && __lane_id() == 0u ? PX - part : 0u;
     const uint64_t o = ((uint64_t)y * k.out_w + x0) * C;
 #pragma unroll
     for (int p = 0; p < PX; ++p) {
         if ((uint32_t)p >= npx) break;
+        if ((uint32_t)p < skip) continue;
 #pragma unroll
         for (int ch = 0; ch < C; ++ch) store_sample<B>(k.out_px, o + p * C + ch, out[p][ch]);
     }
