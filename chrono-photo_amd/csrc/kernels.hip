@@ -7,16 +7,21 @@
 
 namespace cp {
 
-template <int B>
-static int launch_outlier_generic_b(const cp_stack* st, const OutlierK& k, hipStream_t s) {
+template <int B, int C>
+static void launch_outlier_generic_c(const OutlierK& k, hipStream_t s) {
     dim3 block(256), grid((k.out_w + 255) / 256, k.out_h);
+    if (k.pos_off.table) hipLaunchKernelGGL((outlier_generic_kernel<B, C, true>), grid, block, 0, s, k);
+    else hipLaunchKernelGGL((outlier_generic_kernel<B, C, false>), grid, block, 0, s, k);
+}
+
+template <int B>
+static void launch_outlier_generic_b(const cp_stack* st, const OutlierK& k, hipStream_t s) {
     switch (st->channels) {
-    case 1: hipLaunchKernelGGL((outlier_generic_kernel<B, 1>), grid, block, 0, s, k); break;
-    case 2: hipLaunchKernelGGL((outlier_generic_kernel<B, 2>), grid, block, 0, s, k); break;
-    case 3: hipLaunchKernelGGL((outlier_generic_kernel<B, 3>), grid, block, 0, s, k); break;
-    default: hipLaunchKernelGGL((outlier_generic_kernel<B, 4>), grid, block, 0, s, k); break;
+    case 1: launch_outlier_generic_c<B, 1>(k, s); break;
+    case 2: launch_outlier_generic_c<B, 2>(k, s); break;
+    case 3: launch_outlier_generic_c<B, 3>(k, s); break;
+    default: launch_outlier_generic_c<B, 4>(k, s); break;
     }
-    return CP_OK;
 }
 
 OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uint64_t max_pos, uint32_t flags) {
