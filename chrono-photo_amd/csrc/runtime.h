@@ -66,7 +66,7 @@ struct cp_ctx {
     int cu_count = 0;
     cp::ParamArena arena;
     cp::DeviceBuffer out_px, out_mask, out_stats, warn;  // host-output staging
-    cp::DeviceBuffer shake_ws;                           // kept by cp_shake (not charged to the budget)
+    cp::DeviceBuffer shake_ws;                           // kept by cp_shake where there is no budget
     std::mutex mu;
     // autotuned kernel choice per (sample bytes - 1, channels - 1, threshold kind (0: absolute,
     // 1: relative), frame bucket); -1 = default

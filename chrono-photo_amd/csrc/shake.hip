@@ -13,7 +13,8 @@ namespace {
 // it (shake_scratch_init) and only that address is used on the host.
 constexpr uint64_t kShakeScratchBytes = 8ull << 20;
 constexpr int kMaxDevices = 64;
-// Sum tables and offsets up to this size live in a workspace that the context keeps.
+// Sum tables and offsets up to this size live in a workspace that a context without a memory
+// budget keeps.
 constexpr uint64_t kShakeKeepBytes = 4ull << 20;
 // Window rows per workgroup (a multiple of its four waves)
 constexpr int32_t kShakeRows = 16;
@@ -50,8 +51,9 @@ int cp::shake_scratch_init(int device) {
     return CP_OK;
 }
 
-// The search of cp_shake.  scratch_dev == nullptr: the sum table comes from hipMalloc; else it
-// lives in scratch_dev (kShakeScratchBytes).  dev_out: offsets is a device array written
+// The search of cp_shake.  scratch_dev == nullptr: the sum table lives in the context's kept
+// workspace, or comes from hipMalloc where it does not fit there; else it lives in scratch_dev
+// (kShakeScratchBytes).  dev_out: offsets is a device array written
 // asynchronously on the context stream; else a host array and the call waits.
 static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, uint32_t n,
                      const int32_t* anchors_xy, uint32_t n_anchors, uint32_t anchor_radius,
@@ -129,8 +131,10 @@ static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, ui
         const uint64_t offs_bytes = dev_out ? 0 : 8ull * n;
         if ((rc = ctx->charge(sums_bytes + offs_bytes))) return rc;
         // The context keeps one small workspace (an allocation and its release cost more than the
-        // search of a short stack); this call holds it until the stream has drained below.
-        kept = sums_al + offs_bytes <= kShakeKeepBytes &&
+        // search of a short stack); this call holds it until the stream has drained below.  With a
+        // memory budget it does not: memory held between calls would be missing from a later
+        // allocation that fits the budget.
+        kept = ctx->budget == 0 && sums_al + offs_bytes <= kShakeKeepBytes &&
                (ctx->shake_ws.ptr || hipMalloc(&ctx->shake_ws.ptr, kShakeKeepBytes) == hipSuccess);
         if (kept) {
             sums.ptr = ctx->shake_ws.ptr;
