@@ -134,8 +134,13 @@ static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, ui
         // search of a short stack); this call holds it until the stream has drained below.  With a
         // memory budget it does not: memory held between calls would be missing from a later
         // allocation that fits the budget.
-        kept = ctx->budget == 0 && sums_al + offs_bytes <= kShakeKeepBytes &&
-               (ctx->shake_ws.ptr || hipMalloc(&ctx->shake_ws.ptr, kShakeKeepBytes) == hipSuccess);
+        if (ctx->budget == 0 && sums_al + offs_bytes <= kShakeKeepBytes) {
+            kept = ctx->shake_ws.ptr || hipMalloc(&ctx->shake_ws.ptr, kShakeKeepBytes) == hipSuccess;
+            if (!kept) {
+                ctx->shake_ws.ptr = nullptr;
+                (void)hipGetLastError();  // not the call's error: its own table may still fit
+            }
+        }
         if (kept) {
             sums.ptr = ctx->shake_ws.ptr;
             if (!dev_out) offs.ptr = (uint8_t*)ctx->shake_ws.ptr + sums_al;

@@ -1,5 +1,9 @@
-"""The workspace cp_shake keeps with its context: not on a context with a device-memory budget."""
+"""The workspace cp_shake keeps with its context: not on a context with a device-memory budget, and not
+needed where there is no room for it."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -8,6 +12,8 @@ import chrono_photo_amd as cpa
 from chrono_photo_amd import hip as H
 
 pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _free_bytes():
@@ -34,3 +40,45 @@ def test_a_budgeted_context_keeps_no_device_memory(ctx):
     small.close()
     assert np.array_equal(off, ref)
     assert kept == 0, kept
+
+
+# Fails the workspace's allocation (its size alone) with the runtime's own out-of-memory error.
+NO_WORKSPACE = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+typedef int (*malloc_fn)(void**, size_t);
+extern "C" int hipMalloc(void** p, size_t n) {
+    void* h = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
+    malloc_fn real = (malloc_fn)dlsym(h, "hipMalloc");
+    return real(p, n == (size_t)4 << 20 ? (size_t)1 << 50 : n);
+}
+"""
+
+SEARCH = r'''
+import ctypes, sys
+ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)
+sys.path[:0] = [sys.argv[1]]
+import numpy as np
+import chrono_photo_amd as cpa
+print("case: shake search whose workspace cannot be allocated", flush=True)
+x = np.random.default_rng(5).integers(0, 256, (4, 32, 40, 3), np.uint8)
+ctx = cpa.Context(0)
+st = cpa.Stack.from_array(ctx, x)
+off = cpa.ShakeAnalyzer().analyze(st, [(20, 16)], 4, 3)
+print("OFFSETS", off.reshape(-1).tolist(), flush=True)
+'''
+
+
+def test_search_without_room_for_the_workspace(ctx, tmp_path):
+    """The smaller allocations of the call itself still succeed, and so does the call."""
+    (tmp_path / "no_ws.cpp").write_text(NO_WORKSPACE)
+    lib = str(tmp_path / "no_ws.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-o", lib, str(tmp_path / "no_ws.cpp"), "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-c", SEARCH, os.path.join(ROOT, "chrono-photo_amd"), lib],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    x = np.random.default_rng(5).integers(0, 256, (4, 32, 40, 3), np.uint8)
+    st = cpa.Stack.from_array(ctx, x)
+    ref = cpa.ShakeAnalyzer().analyze(st, [(20, 16)], 4, 3)
+    st.close()
+    assert f"OFFSETS {ref.reshape(-1).tolist()}" in r.stdout
