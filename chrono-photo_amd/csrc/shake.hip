@@ -159,6 +159,7 @@ static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, ui
     hipLaunchKernelGGL(zero_u64_kernel, dim3((uint32_t)std::min<uint64_t>(1024, (n_sums + 255) / 256)), dim3(256), 0,
                        hs, k.sums, n_sums);
     hipError_t e = hipGetLastError();
+    if (e != hipSuccess) rc = fail(CP_ERR_HIP, "shake kernels: %s", hipGetErrorString(e));
     // Launch plan: candidate blocks of up to 32 x 32, about kRows window rows per workgroup in
     // even chunks; where that does not fit LDS, the larger of the row counts shrinks, then the
     // candidate columns.

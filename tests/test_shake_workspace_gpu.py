@@ -82,3 +82,19 @@ def test_search_without_room_for_the_workspace(ctx, tmp_path):
     ref = cpa.ShakeAnalyzer().analyze(st, [(20, 16)], 4, 3)
     st.close()
     assert f"OFFSETS {ref.reshape(-1).tolist()}" in r.stdout
+
+
+def test_an_error_before_the_search_is_reported(ctx):
+    """An error that an earlier runtime call left unread ends the call, as it ends a composite, and is
+    gone with it; it never stands for offsets that were not written."""
+    x = np.random.default_rng(6).integers(0, 256, (4, 32, 40, 3), np.uint8)
+    st = cpa.Stack.from_array(ctx, x)
+    ref = cpa.ShakeAnalyzer().analyze(st, [(20, 16)], 4, 3)
+    assert ref.any()
+    p = C.c_void_p()
+    assert H.hip().hipMalloc(C.byref(p), 1 << 50) != 0
+    with pytest.raises(cpa.ChronoError) as e:
+        cpa.ShakeAnalyzer().analyze(st, [(20, 16)], 4, 3)
+    assert e.value.code == cpa.CP_ERR_HIP
+    assert np.array_equal(cpa.ShakeAnalyzer().analyze(st, [(20, 16)], 4, 3), ref)
+    st.close()
