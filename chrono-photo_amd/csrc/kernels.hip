@@ -29,8 +29,8 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
     // subset, up to 128 sample frames) or the tuned choice between the two kernels; 16-bit ones
     // the 16-bit kernel up to 1024 frames (and up to 128 sample frames); the one-lane-per-pixel
     // generic kernel takes the rest.  A packed-byte choice whose wide loads would read past a
-    // borrowed stack's end falls back to the bucket's 16-bit-halves shape, or to the generic
-    // kernel where the bucket has none.
+    // borrowed stack's end falls back to another candidate of its bucket, or to the generic kernel
+    // where none stays inside the stack.
     OutlierPlan p;
     const bool sums = k.background == 2 || k.outlier == 3;
     if (flags & CP_FLAG_FORCE_GENERIC) return p;
@@ -54,13 +54,15 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
     if (choice < 0) choice = untuned_shape(st->bps, k.n);
     if (choice >= kU8Base) {
         if (u8_fits(choice - kU8Base)) return {kPlanU8, choice - kU8Base};
-        // a borrowed stack the wide loads would overrun: the bucket's 16-bit-halves shape
+        // a borrowed stack the wide loads would overrun: the first of the bucket's candidates that
+        // stay inside it
         const int b = bucket_for(k.n);
         choice = -1;
-        for (int c = kMaxCand - 1; b >= 0 && c >= 0; --c) {
+        for (int c = 0; b >= 0 && choice < 0 && c < kMaxCand; ++c) {
             const int cand = kBucketCand[st->bps - 1][st->channels >= 3][b][c];
-            if (cand >= 0 && cand < kU8Base) choice = cand;  // the first of them
+            if (cand >= 0 && (cand < kU8Base || u8_fits(cand - kU8Base))) choice = cand;
         }
+        if (choice >= kU8Base) return {kPlanU8, choice - kU8Base};
     }
     if (choice >= 0) {
         if (kShapes[choice].X > 1 && !pair_tile_fits(st->dev, st->alloc_bytes, st->bps, st->channels, k, max_pos))
