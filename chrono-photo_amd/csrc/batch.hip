@@ -515,8 +515,10 @@ extern "C" CP_API int cp_autotune(cp_ctx* ctx, uint32_t bps, uint32_t channels, 
                     const float range = bps == 1 ? 255.0f : 65535.0f;
                     k.th = kind == 0 ? ThresholdK{1, 0.05f * range, 0.2f * range, 1.0f / (0.15f * range)}
                                      : ThresholdK{0, 2.0f, 4.0f, 0.5f};
-                    k.background = kind == 1 && bps == 1 ? 2 : 0;  // 16-bit average sums need N <= 256
-                    k.outlier = kind == 1 && bps == 1 ? 3 : 2;
+                    // absolute thresholds are timed in the extreme mode, relative ones in the average
+                    // mode; the choice then serves every mode
+                    k.background = kind == 1 ? 2 : 0;
+                    k.outlier = kind == 1 ? 3 : 2;
                     for (int i = 0; i < 4; ++i) k.w[i] = 1.0f;
                     k.fade.is_none = 1;
                     k.out_px = d_out;

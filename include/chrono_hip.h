@@ -270,7 +270,9 @@ CP_API int cp_batch_run(cp_ctx* ctx, const cp_job* jobs, uint32_t n_jobs, uint32
 /* Autotuner: for each threshold kind (absolute, relative) and frame-count bucket of the
  * register-resident outlier kernels (<= 16, 32, 64, 128, 256, 512, 768, 1024, 1280 frames:
  * CP_TILE_BUCKETS buckets) time the candidate kernel choices on a synthetic stack of this
- * sample width and channel count (1-4) and keep the fastest for the context.  A choice is a
+ * sample width and channel count (1-4) and keep the fastest for the context (absolute
+ * thresholds in the extreme mode, relative ones in the average mode; each choice then serves
+ * every mode, where an untuned context's defaults tell the average modes apart).  A choice is a
  * tile shape of the 16-bit-halves kernel or of the 8-bit packed-byte kernel, whose
  * one-lane-per-pixel shapes rank either by searches or by a sorting network; shapes (nullable,
  * 2 * CP_TILE_BUCKETS entries: absolute thresholds' buckets, then relative thresholds')
