@@ -199,8 +199,10 @@ __device__ __forceinline__ void load_block_exchange(const uint8_t* __restrict__ 
     // Forty frames of three channels leave no room for the loads' addresses at three waves per
     // SIMD; the last quad's loads then wait until the first quad has left its registers.  All at
     // once spilled 7 dwords per lane: 1200 x 1080p RGB8 wrote 412 MB instead of 13 and took 2228
-    // us, 2070 us so.
-    constexpr int HELD = FB >= 40 && C == 3 ? 4 : 0;
+    // us, 2070 us so.  Two channels are as tight from 24 frames on (their tiles run more waves):
+    // with nothing held back and the 160-frame tile at four waves, which spilled 36 dwords, 1280 x
+    // 1280x720 took 998 us, 688 us so; 768 frames 468 and 439 us.
+    constexpr int HELD = C == 3 ? (FB >= 40 ? 4 : 0) : (C == 2 ? (FB >= 40 ? 8 : FB >= 24 ? 4 : 0) : 0);
     vec raw[FB];
     auto load = [&](int t) { raw[t] = *(const __attribute__((address_space(1))) vec*)((base + o[t]) & ~(uintptr_t)3); };
 #pragma unroll
@@ -845,6 +847,10 @@ constexpr int waves_hint_u8(int C, int F, int X, int FS, bool ABS, bool sort, bo
         // a block of sample frames comes after the block of all frames and needs no registers when
         // that one's loads peak: 1200 x 1080p RGB8 with 64 sample frames 2490 us at 2 waves, 2034
         // us at 3
+        // the 160-frame tile of two channels fits three waves (1100 x 1280x720 abs/0.05/0.2 1000 us at
+        // the four that spill, 745 us; rel/2.0/4.0 1648 and 1615 us), except that relative thresholds
+        // over a sample block gain more from the fourth (1280 frames 2303 and 2164 us)
+        if (C == 2 && F == 160) return FS > 0 && !ABS ? 4 : 3;
         const int v = 512 / (C * F / 4 + 48 + planes);
         return v < 2 ? 2 : (v > 6 ? 6 : v);
     }

@@ -2,6 +2,7 @@
 the streaming darker/lighter kernels keep everything in registers (private memory in their frame loop
 costs them 3 to 6 %)."""
 import os
+import re
 import struct
 
 import msgpack
@@ -49,4 +50,16 @@ def test_simple_kernels_use_no_private_memory():
     found = {k[".name"]: k[".private_segment_fixed_size"] for e in _code_objects(blob) for k in _kernels(e)
              if "simple" in k[".name"]}
     assert len(found) >= 16, sorted(found)  # sample widths x channel counts x steps, at least
+    assert not {n: b for n, b in found.items() if b}
+
+
+def test_exchange_tiles_use_no_private_memory():
+    """8-bit tiles that exchange their loads (X = 1, no sample block, the last flag set), plain and
+    grouped: what spills there is written to HBM by every lane."""
+    with open(os.path.join(cpa.LIB_DIR, "libchrono_hip.so"), "rb") as f:
+        blob = f.read()
+    pat = re.compile(r"outlier_u8_(group_)?kernelILi\dELi\d+ELi\d+ELi1ELi0ELb[01]ELb0ELb1EE")
+    found = {k[".name"]: k[".private_segment_fixed_size"] for e in _code_objects(blob) for k in _kernels(e)
+             if pat.search(k[".name"])}
+    assert len(found) >= 96, len(found)  # 4 channel counts x 7 tiles x 2 threshold kinds, plain and grouped
     assert not {n: b for n, b in found.items() if b}
