@@ -44,7 +44,7 @@ OutlierPlan plan_outlier(cp_ctx* ctx, const cp_stack* st, const OutlierK& k, uin
             if (sh >= 0 && u8_fits(sh)) p = {kPlanU8, sh};
         }
         if (st->bps == 2 && k.n <= kFastMaxFrames && k.n_sample <= kFastMaxSample && k.samp_off) {
-            const int sh = fast_sample_shape(k.n, k.n_sample);
+            const int sh = fast_sample_shape(k.n, k.n_sample, k.th.absolute != 0);
             if (sh >= 0 && pair_tile_fits(st->dev, st->alloc_bytes, st->bps, st->channels, k, max_pos))
                 p = {kPlanFast, sh};
         }
