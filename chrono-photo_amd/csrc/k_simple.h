@@ -183,13 +183,17 @@ __device__ __forceinline__ void simple_pixels(const SimpleK& k) {
             uint32_t d[UF][ND + 1], sh[UF];
             auto load = [&](int u, uint64_t off) {
                 // whole dwords from the one that holds the first byte to the one that holds the
-                // last; the lanes of a wave share the shift.  One load for a shifted segment too
-                // (700 x 1280x721 RGB16 with crops 708 us with a second load for its last dword,
-                // 680 us so)
+                // last; the lanes of a wave share the shift.  The last dword of a shifted segment
+                // comes with the others in the crops of 8-bit stacks (200 x 1926x1086 RGB8 333 us
+                // with a load of its own, 303 us so), and by itself elsewhere: whole images seldom
+                // shift, and the wider loads are slower even where they do not run (64 x 1280x721
+                // mono 19.7 us with them, 16.2 us without), crops of 16 bits 200 x 1926x1086 mono
+                // 192 and 163 us.
+                constexpr bool TOGETHER = B == 1 && TABLE && ND < 4;
                 const uintptr_t a = base + off * B;
                 sh[u] = (base_sh + (uint32_t)off * B) & 3u;
                 const uintptr_t w = a & ~(uintptr_t)3;
-                if (ND < 4 && sh[u] != 0u) {
+                if (TOGETHER && sh[u] != 0u) {
                     const words1 v = *(const __attribute__((address_space(1))) words1*)w;
 #pragma unroll
                     for (int i = 0; i <= ND; ++i) d[u][i] = v[i];
@@ -199,7 +203,7 @@ __device__ __forceinline__ void simple_pixels(const SimpleK& k) {
 #pragma unroll
                 for (int i = 0; i < ND; ++i) d[u][i] = v[i];
                 d[u][ND] = 0u;
-                if (ND >= 4 && sh[u] != 0u) d[u][ND] = *(const __attribute__((address_space(1))) uint32_t*)(w + NB);
+                if (!TOGETHER && sh[u] != 0u) d[u][ND] = *(const __attribute__((address_space(1))) uint32_t*)(w + NB);
             };
             int32_t t = 0;
             for (; t + UF <= N; t += UF) {

@@ -106,34 +106,18 @@ static void launch_simple_b(const cp_stack* st, const SimpleK& k, bool plain, hi
 }
 
 // Whether a darker/lighter composite with unit weights and no fade takes the whole-number step
-// (k_simple.h); one_row: its frames run as one row.  It is the faster one nearly everywhere (us, general
-// and whole-number step: 64 x 1280x721 RGB8 48 and 29, 300 x 1281x721 RGB8 263 and 148, 300 x 1280x721
-// RGBA16 with crops 414 and 398), except that
-//  - the crops of four 8-bit channels that come from HBM (256 MB and more) suit the general step's five
-//    waves per SIMD better than eight, unless eight save a round of workgroups: 300 x 992x712 (712
-//    groups, one round of either) 182 and 214, 300 x 2592x712 (two of either) 432 and 497, but
-//    300 x 1272x712 (two and one) 316 and 249;
-//  - tall 16-bit mono stacks are read faster by the general step's waves, which do not keep step with
-//    one another, once they are many or the stack is very tall: 300 x 1440x960 176 and 202, 300 x 4K
-//    895 and 988, 700 x 1024x768 228 and 268, but 300 x 1280x721 128 and 124;
-//  - a grid a little over what the device holds at once pays for a whole second round of waves that
-//    keep step: 200 x 1400x800 RGB16 247 and 266, 400 x 2048x1080 RGB8 510 and 532.
-// Where segments start inside a dword the last two are the other way round (300 x 1921x1081 mono 16
-// bits 335 and 243).
+// (k_simple.h); one_row: its frames run as one row.  It is the faster one (us, general and whole-number
+// step: 64 x 1280x721 RGB8 48 and 28, 300 x 1281x721 RGB8 263 and 148, 200 x 1080p 16-bit mono 166 and
+// 148), except that the crops of four 8-bit channels that come from HBM (256 MB and more) suit the
+// general step's five waves per SIMD better than eight, unless eight save a round of workgroups: 300 x
+// 992x712 (712 groups, one round of either) 182 and 214, 300 x 2592x712 (two of either) 432 and 497,
+// but 300 x 1272x712 (two and one) 316 and 249.
 static bool whole_numbers(const cp_ctx* ctx, const cp_stack* st, const SimpleK& k, bool one_row) {
-    const uint32_t px = 4u / st->bps, n = k.n;
-    const uint64_t blocks = (uint64_t)((k.out_w + px * 256u - 1u) / (px * 256u)) * k.out_h;
-    const uint64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256, fill = 8u * cus;  // a wave per SIMD is a group per CU
-    if (st->bps == 1 && st->channels == 4 && !one_row) {
-        const uint64_t rounds8 = (blocks + fill - 1) / fill, rounds5 = (blocks + 5u * cus - 1) / (5u * cus);
-        return rounds8 < rounds5 || (uint64_t)k.out_w * k.out_h * 4u * n < (256ull << 20);
-    }
-    const bool little_over = blocks > fill && blocks <= fill + fill / 4;
-    const bool whole_dwords = one_row && st->width * st->channels * st->bps % 4u == 0 && ((uintptr_t)k.stack & 3u) == 0;
-    if (!whole_dwords) return true;
-    if (st->bps == 1) return !(st->channels == 3 && little_over && n > 256);
-    if (st->channels == 1) return n <= (blocks > fill ? 128u : 512u);
-    return !(st->channels == 3 && little_over && n > 128);
+    if (st->bps != 1 || st->channels != 4 || one_row) return true;
+    const uint64_t blocks = (uint64_t)((k.out_w + 1023u) / 1024u) * k.out_h;
+    const uint64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;  // a wave per SIMD is a group per CU
+    const uint64_t rounds8 = (blocks + 8u * cus - 1) / (8u * cus), rounds5 = (blocks + 5u * cus - 1) / (5u * cus);
+    return rounds8 < rounds5 || (uint64_t)k.out_w * k.out_h * 4u * k.n < (256ull << 20);
 }
 
 int launch_simple(cp_ctx* ctx, const cp_stack* st, const SimpleK& k_in, hipStream_t s) {
