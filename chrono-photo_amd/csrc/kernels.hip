@@ -135,6 +135,13 @@ int launch_simple(cp_ctx* ctx, const cp_stack* st, const SimpleK& k_in, hipStrea
         k.out_h = 1;
     }
     plain = plain && whole_numbers(ctx, st, k, one_row);
+    // Waves in step (k_simple.h) where one round of them fills three quarters of the device, or half of it
+    // on four channels.  us, eight loads in flight and one: RGB8 64 x 1080p (2025 groups for 2048 places)
+    // 71.2 and 67.0, 200 x 2592x712 (1802) 198 and 177, but 200 x 1366x768 (1024) 110 and 121 and, in two
+    // rounds, 64 x 2048x1080 (2160) 74 and 96; RGBA8 200 x 1366x768 143 and 136, 200 x 1000x667 (651) 95
+    // and 115.
+    const uint32_t cus = ctx->cu_count > 0 ? (uint32_t)ctx->cu_count : 256u, groups = k.out_w / 1024u;
+    k.in_step = one_row && groups >= (st->channels == 4 ? 4u : 6u) * cus && groups < 8u * cus;
     const bool table = k.pos_off.table != nullptr;
     if (st->bps == 1) table ? launch_simple_b<1, 4, true>(st, k, plain, s) : launch_simple_b<1, 4, false>(st, k, plain, s);
     else table ? launch_simple_b<2, 2, true>(st, k, plain, s) : launch_simple_b<2, 2, false>(st, k, plain, s);

@@ -85,6 +85,7 @@ struct SimpleK {
     uint32_t out_w, out_h;
     int32_t frame_offset;
     int32_t darker;
+    uint32_t in_step;  // whole-number step: one load at a time per wave (set by the launch)
     float w[4];
     FadeK fade;
     void* out_px;

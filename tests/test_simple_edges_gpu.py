@@ -52,3 +52,17 @@ def test_cropped_rows(ctx, bits, c, w):
     vertical = np.stack([np.zeros(n, np.int32), rng.integers(0, 3, n).astype(np.int32)], 1)
     _check(x, st, (bits, c, w, "vertical"), crop=(vertical, w + 3, h - 2))
     st.close()
+
+
+@pytest.mark.parametrize("c", [3, 4])
+@pytest.mark.parametrize("w,h", [(1600, 655), (1439, 729), (1600, 983), (1921, 819), (1601, 1309), (2048, 1024)])
+def test_large_whole_frames(ctx, c, w, h):
+    """8-bit images of about half, three quarters and all of what the device holds at once, one frame
+    more than the loads in flight."""
+    n = 9
+    x = np.random.default_rng(w + h + c).integers(0, 256, (n, h, w, c), dtype=np.uint8)
+    st = cpa.Stack.from_array(ctx, x)
+    for darker in (True, False):
+        img = cpa.SimpleProcessor((1, 1, 1, 1), cpa.Fade.none(), darker).process(st)
+        assert np.array_equal(img, O.simple(x, (1, 1, 1, 1), O.Fade.none(), darker)), (c, w, h, darker)
+    st.close()
