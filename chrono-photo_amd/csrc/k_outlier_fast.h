@@ -612,7 +612,7 @@ __device__ __forceinline__ void rank_pairs(const uint32_t (&raw)[C][NW], uint32_
     } else if constexpr (WINDOW) {
         // few lanes estimate the median more coarsely: a window of 256 values (one step more) up
         // to 128 frames saves most of the second searches (100 x 1937x1091 mono: 219 us with 128
-        // values, 192 us so)
+        // values, 192 us so, both before bit planes counted)
         constexpr int WB = G <= 4 ? 8 : 7;
         constexpr uint32_t TOP = (1u << WB) - 1u, LO_MAX = 65535u - TOP;
         const uint32_t nv = offering_lanes<G, 2 * NW>(count);
@@ -932,8 +932,8 @@ __device__ __forceinline__ void finish_pixel(const OutlierK& k, uint32_t bx, uin
     constexpr uint32_t MAXV = B == 1 ? 255u : 65535u;
     constexpr uint32_t NONE = 0xFFFFFFFFu;
     // outliers whose samples the finish re-reads together: eight for the two-pixel tiles
-    // (same registers as four, 0.4% faster on the 4K stack), one for the four-pixel-per-lane
-    // tiles (a batch pushes their kernels into private memory)
+    // (same registers as four, 0.4% faster on the 4K stack), one for the four-pixel tiles (those of
+    // 16-bit mono stacks up to 256 frames)
     constexpr int KB = X >= 4 ? 1 : (X == 2 ? 8 : 4);
     const uint32_t N = k.n;
     const uint32_t x = bx * P + p;
@@ -1910,7 +1910,9 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t nb) {
 // 4-channel tiles one fewer; two 3- or 4-channel pixels per lane double the frame registers
 // (three waves, two for 4 channels or relative thresholds), two or four pixels of two or one
 // channels take two thirds of that (three waves, four for two channels and absolute thresholds); the 64-frame
-// tiles get the whole register file.
+// tiles get the whole register file.  The three-channel tile of 128 frames with a sample block spills 6
+// registers at three waves and is faster with them than at two (128 x 1280x720, 60 sample frames 225
+// and 253 us).
 constexpr int waves_hint(int F, int C, bool absolute, int X = 1) {
     return F > 32   ? 1
            : X == 1 ? (absolute ? 5 : 4) - (C > 3 ? 1 : 0)

@@ -16,9 +16,9 @@
 // With unit weights and no fade (the defaults) a pixel's value is the sum of its samples, a whole
 // number that f32 holds exactly, and a new extreme replaces the pixel: PlainPixels keeps the
 // pixels packed as they lie in memory and takes one or two dot products, a compare and two
-// selects per pixel and frame.  Bound by HBM.  The general step (about 28 VALU instructions per
-// pixel and frame) was bound by VALU issue: 64 x 1080p RGB8, per call, 93 us with it and 67.5 us
-// (6.0 TB/s) without.
+// selects per pixel and frame (simple_plain_kernel).  Bound by HBM.  The general step, about 28 VALU
+// instructions per pixel and frame (simple_kernel), is bound by VALU issue: 64 x 1080p RGB8, per call,
+// 89.6 us with it and 67.7 us (6.0 TB/s) with whole numbers.
 #pragma once
 #include "device_common.h"
 

@@ -1,9 +1,10 @@
 // kernels_fast.h -- tile shapes of the register-resident outlier kernel and their launch.
 //
-// A shape (G, F) puts G lanes on each pixel and F frames in each lane (G * F >= N); a
-// 256-lane workgroup then covers 256 / G pixels.  Frame counts fall into buckets; each bucket
-// has up to two candidate shapes and the autotuner (cp_autotune) measures both on the device
-// and records the faster one per (sample width, channels, bucket) in the context.
+// A shape (G, F, X) puts G lanes on each group of X pixels and F frames in each lane (G * F >= N);
+// a 256-lane workgroup then covers X * 256 / G pixels.  Frame counts fall into buckets; each bucket
+// has up to kMaxCand candidate shapes, of this kernel and of the packed-byte one, and the autotuner
+// (cp_autotune) measures them on the device and records the fastest per (sample width, channels,
+// bucket, threshold kind) in the context.
 #pragma once
 #include "k_outlier_fast.h"
 #include "runtime.h"
@@ -16,12 +17,13 @@ struct TileShape {
 
 // Shapes from 10 on put several pixels in each lane (16-bit stacks): one 8- to 16-byte load per
 // frame instead of one per pixel, which is what lets a wave's loads reach HBM speed; narrow_shape
-// gives the one-pixel shape with the same blocks (3 and 4 channels up to 256 frames).  X is 2
+// gives the one-pixel shape with the same blocks (3 and 4 channels; for 512 frames one of
+// longer blocks).  X is 2
 // there, and 4 for one channel (wide_px).  Shapes from 17 on carry an FS-frame block of the
 // `--sample` positions.  Before the shapes for 1 and 2 channels, above 512 frames and with a
 // sample block, those stacks took the one-lane-per-pixel kernel, which reads every frame from
-// L2 once per value bit: 100 x 1937x1091 mono took 4.19 ms and takes 0.222 ms, 300 x 960x541 RGB
-// with 48 sample frames 4.42 and 0.440 ms.
+// L2 once per value bit: 100 x 1937x1091 mono took 4.19 ms and takes 0.176 ms, 300 x 960x541 RGB
+// with 48 sample frames 4.41 and 0.380 ms.
 constexpr int kNumShapes = 21;
 constexpr TileShape kShapes[kNumShapes] = {
     {1, 16, 1, 0}, {1, 32, 1, 0},  {2, 16, 1, 0},  {2, 32, 1, 0},  {4, 16, 1, 0},  {4, 32, 1, 0},  {8, 16, 1, 0},
@@ -50,8 +52,8 @@ inline int fast_sample_shape(uint32_t n, uint32_t s, bool absolute) {
 }
 // Frame-count buckets of the tuned kernel choice.  A choice is a shape of this kernel
 // (kShapes index) or, from kU8Base on, a shape of the 8-bit packed-byte kernel (kU8Shapes
-// index + kU8Base, kernels_u8.h); each bucket has up to kMaxCand candidates, the first being
-// the default, and cp_autotune keeps the fastest per (sample width, channels, bucket).
+// index + kU8Base, kernels_u8.h); each bucket has up to kMaxCand candidates.  kDefault says
+// which of them a context takes that was not tuned.
 constexpr int kNumBuckets = 9;
 constexpr uint32_t kBucketMax[kNumBuckets] = {16, 32, 64, 128, 256, 512, 768, 1024, 1280};
 constexpr int kU8Base = 64;

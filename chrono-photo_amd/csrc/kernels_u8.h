@@ -14,8 +14,8 @@ struct U8Shape {
     constexpr int load_px() const { return L ? L : X; }
 };
 
-// One pixel per lane for short stacks; four pixels per lane (one 16-byte load per frame)
-// for tall ones; `--sample` shapes carry an FS-frame block of the sample positions; shapes
+// One pixel per lane for short stacks; four pixels per lane (one 16-byte load per frame) as
+// the autotuner's candidates for tall ones; `--sample` shapes carry an FS-frame block of the sample positions; shapes
 // 14-16 rank one lane's whole pixel with a sorting network; shape 17 holds a 64-frame pixel
 // in one lane.  Shapes 12, 13 and from 18 on are exchange tiles, 12, 13 and 24 with a block of
 // up to 128 sample frames.

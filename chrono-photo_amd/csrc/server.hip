@@ -74,8 +74,8 @@ void* mapped_host(void* p) {
     return (uint8_t*)a.devicePointer + ((uint8_t*)p - (uint8_t*)a.hostPointer);
 }
 
-// Result download: through the DMA path, or, while uploads are in flight (a download
-// queued behind a multi-megabyte upload in a DMA engine would hold its slot), by a copy
+// Result download: by the runtime's copy, or, while uploads are in flight (a download the
+// runtime gives to a DMA engine behind a multi-megabyte upload would hold its slot), by a copy
 // kernel on the slot's own queue when the host buffer is pinned.
 int download(void* host, const void* dev, uint64_t bytes, hipStream_t s, bool by_kernel, uint32_t* kernel_count) {
     void* d = by_kernel ? mapped_host(host) : nullptr;

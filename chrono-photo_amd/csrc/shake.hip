@@ -160,7 +160,7 @@ static int shake_run(cp_ctx* ctx, const cp_stack* st, const uint32_t* frames, ui
                        hs, k.sums, n_sums);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) rc = fail(CP_ERR_HIP, "shake kernels: %s", hipGetErrorString(e));
-    // Launch plan: candidate blocks of up to 32 x 32, about kRows window rows per workgroup in
+    // Launch plan: candidate blocks of up to 32 x 32, about kShakeRows window rows per workgroup in
     // even chunks; where that does not fit LDS, the larger of the row counts shrinks, then the
     // candidate columns.
     const int32_t size = (int32_t)(2 * r + 1), C = (int32_t)st->channels, planes = (int32_t)st->bps;

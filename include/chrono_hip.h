@@ -313,7 +313,7 @@ typedef struct {
     uint64_t peak_bytes;      /* highest admitted HBM use */
     uint32_t peak_inflight;
     uint32_t kernel_downloads; /* results written to pinned host memory by a copy kernel
-                                  (while uploads were in flight) instead of the DMA path */
+                                  (while uploads were in flight) instead of the runtime's copy */
 } cp_server_stats;
 
 CP_API int cp_server_create(cp_ctx* ctx, uint64_t hbm_budget_bytes, uint32_t max_inflight,
